@@ -11,8 +11,8 @@
 //   memory    read-out backward, the scan's backward (ava_mem_scan_bwd), the inputs' preparation backward
 //             (unit norms, gates, value residual), the projections and the rank-32 gate read-outs
 //   spiking   dS = dx Wout^T, the LIF scan's backward (ava_lif_scan_bwd), the (1 - beta) scale, dWin
-// The plain products (x W, dY W^T, X^T dY) are library GEMMs (rocBLAS, f32); the rest is the library's
-// own kernels. theta is detached (as in the reference's LIF backward) and the gate offsets are constants,
+// The plain products (x W, dY W^T, X^T dY) run on the f16 matrix cores in split form (hgemm.hip), small
+// ones as library GEMMs (rocBLAS, f32); the rest is the library's own kernels. theta is detached (as in the reference's LIF backward) and the gate offsets are constants,
 // so their gradients are zero.
 #include <math.h>
 #include <string.h>
@@ -20,9 +20,11 @@
 #include <rocblas/rocblas.h>
 
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
+#include "hgemm.h"
 #include "train.h"
 
 namespace {
@@ -84,6 +86,11 @@ struct ava_trainer {
     size_t lws_floats = 0;
     float *att_part = nullptr;
     size_t att_part_floats = 0;
+    // the products' split operands (a stack: see Arena) and scratch
+    char *hplanes = nullptr;
+    size_t hplanes_bytes = 0, hplanes_used = 0;
+    float *hpart = nullptr;
+    size_t hpart_floats = 0;
 
     ~ava_trainer() { release(); }
     void release() {
@@ -124,14 +131,74 @@ size_t block_count(const ava_config &c, int i, const std::string &nm) {
     return d;  // the norms' gains, beta_p, theta, arho, again, off
 }
 
-// row-major C [M][N] (ldc) = alpha op(A) op(B) + beta C, op(A) [M][K] (A stored [M][K], or [K][M] when tA)
-int gemm(rocblas_handle h, bool tA, bool tB, int M, int N, int K, float alpha, const float *A, int lda, const float *B,
-         int ldb, float beta, float *C, int ldc) {
+// A product operand: x [rows][cols] in f32 and, once a product on the matrix cores has asked for them, its
+// split forms over k = cols (n) and over k = rows (t), which live in the trainer's stack of planes until the
+// Arena around the operand ends.
+struct Op {
+    const float *x;
+    int rows, cols, ld;
+    ava::HgemmOp n{nullptr, nullptr}, t{nullptr, nullptr};
+};
+struct Arena {
+    ava_trainer *tr;
+    size_t used;
+    explicit Arena(ava_trainer *t) : tr(t), used(t->hplanes_used) {}
+    ~Arena() { tr->hplanes_used = used; }
+};
+
+// Splits x over k = rows (tr) or cols, if it is not yet and the stack has room.
+int split(ava_trainer *t, Op &x, bool tr, hipStream_t st) {
+    ava::HgemmOp &o = tr ? x.t : x.n;
+    if (o.planes) return AVA_OK;
+    const int rows = tr ? x.cols : x.rows, k = tr ? x.rows : x.cols;
+    const size_t pb = (ava::hgemm_plane_bytes(rows, k) + 255) & ~(size_t)255, eb = ((size_t)rows * 4 + 255) & ~(size_t)255;
+    const size_t need = pb + eb + (tr ? ((ava::hgemm_part_floats(x.rows, x.cols) * 4 + 255) & ~(size_t)255) : 0);
+    if (t->hplanes_used + need > t->hplanes_bytes) return AVA_OK;
+    char *p = t->hplanes + t->hplanes_used;
+    t->hplanes_used += need;
+    if (tr) {
+        if (int r = ava::hgemm_split_cols(x.x, x.rows, x.cols, x.ld, p, (int *)(p + pb), (float *)(p + pb + eb), st)) return r;
+    } else {
+        if (int r = ava::hgemm_split_rows(x.x, x.rows, x.cols, x.ld, p, (int *)(p + pb), st)) return r;
+    }
+    o = {p, (const int *)(p + pb)};
+    return AVA_OK;
+}
+
+// Products of at least this many multiply-adds go to the f16 matrix cores: 8192 x 1024 x 1024 (8.6e9) takes
+// 49 us there and 12 + 8 us to split both operands, 148 us in rocBLAS; 2048 x 1024 x 1024 (2.1e9) 29 + 4 + 8
+// against 36; below, rocBLAS. Thin ones (at most 64 rows or columns: the gates, the rank-r read-outs, the
+// single-head engram) go there from HGEMM_THIN when the large operand is already split for another product:
+// 8192 x 64 x 1024 18 us against 29, 1024 x 64 x 8192 24 against 58.
+constexpr double HGEMM_MACS = 2e9, HGEMM_THIN = 1e8;
+
+// row-major C [M][N] (ldc) = op(A) op(B) (+ C with add), op(A) [M][K] (A stored [M][K], or [K][M] when tA)
+// keepA, keepB: the operand is used again, its planes stay when the call ends (they are split first, below the
+// others in the stack).
+// f32: in rocBLAS whatever its size.
+int gemm(ava_trainer *t, bool tA, bool tB, Op &A, Op &B, bool keepA, bool keepB, bool add, float *C, int ldc,
+         hipStream_t st, bool f32 = false) {
+    const int M = tA ? A.cols : A.rows, K = tA ? A.rows : A.cols, N = tB ? B.rows : B.cols;
     if (M == 0 || N == 0) return AVA_OK;
+    const double macs = (double)M * N * K;
+    const ava::HgemmOp &pa = tA ? A.t : A.n, &pb = tB ? B.n : B.t;
+    const bool thin = std::min(M, N) <= 64 && macs >= HGEMM_THIN && (M >= N ? pa : pb).planes;
+    const int parts = ava::hgemm_splits(M, N, K);
+    if (!f32 && (macs >= HGEMM_MACS || thin) && (parts == 1 || (size_t)parts * M * N <= t->hpart_floats)) {
+        if (keepA)
+            if (int r = split(t, A, tA, st)) return r;
+        if (keepB)
+            if (int r = split(t, B, !tB, st)) return r;
+        Arena call(t);
+        if (int r = split(t, A, tA, st)) return r;
+        if (int r = split(t, B, !tB, st)) return r;
+        if (pa.planes && pb.planes) return ava::hgemm(pa, pb, M, N, K, C, ldc, add, t->hpart, t->hpart_floats, st);
+    }
+    const float one = 1.0f, beta = add ? 1.0f : 0.0f;
     const rocblas_status s =
-        rocblas_sgemm(h, tB ? rocblas_operation_transpose : rocblas_operation_none,
-                      tA ? rocblas_operation_transpose : rocblas_operation_none, N, M, K, &alpha, B, ldb, A, lda, &beta,
-                      C, ldc);
+        rocblas_sgemm(t->blas, tB ? rocblas_operation_transpose : rocblas_operation_none,
+                      tA ? rocblas_operation_transpose : rocblas_operation_none, N, M, K, &one, B.x, B.ld, A.x, A.ld,
+                      &beta, C, ldc);
     AVA_REQUIRE(s == rocblas_status_success, AVA_ERR_HIP, "train: rocblas_sgemm failed (%d) M=%d N=%d K=%d", (int)s, M,
                 N, K);
     return AVA_OK;
@@ -209,6 +276,21 @@ int ensure(ava_trainer *t, int B, int T) {
         AF(t->lws, t->lws_floats);
         for (size_t i = 0; i < L; i++) AF(t->acts[i].lpark, ava::lif_park_floats(B, T, (int)d));
     }
+    // the split operands: the largest set alive at once (the head's products, the MLP's, the memory's with the
+    // normed rows kept); none when no product of this batch is large enough. A product that finds no room
+    // runs in rocBLAS.
+    t->hplanes_bytes = t->hpart_floats = 0;
+    if ((double)N * d * std::max<size_t>(H, V) >= HGEMM_MACS) {
+        auto pl = [](size_t rows, size_t k) {
+            return ava::hgemm_plane_bytes(rows, (int)k) + 4 * (rows + ava::hgemm_part_floats((int)k, (int)rows)) + 4096;
+        };
+        t->hplanes_bytes = std::max({pl(N, d) + pl(V, d), pl(V, N) + pl(d, N), pl(N, V) + pl(d, V),
+                                     pl(H, N) + pl(d, N), pl(N, d) + pl(H, d), pl(N, H) + pl(d, H),
+                                     pl(d, N) * 2 + pl(N, d) + pl(d, d)}) + pl(d, N);
+        TR(alloc(t, (void **)&t->hplanes, t->hplanes_bytes));
+        t->hpart_floats = ava::hgemm_part_max();
+        AF(t->hpart, t->hpart_floats);
+    }
     t->N = (int)N;
     t->B = B;
     t->T = T;
@@ -233,13 +315,18 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
     const int L = c.layers, d = c.d, H = c.hidden, hs = c.head_size, nh = d / hs, r = c.gate_rank, V = c.vocab;
     const int N = B * T, de = c.eng_dim, enh = eng_nh(c);
     const size_t Nd = (size_t)N * d;
-    rocblas_handle hb = t->blas;
-    AVA_REQUIRE(rocblas_set_stream(hb, st) == rocblas_status_success, AVA_ERR_HIP, "train: rocblas_set_stream");
+    AVA_REQUIRE(rocblas_set_stream(t->blas, st) == rocblas_status_success, AVA_ERR_HIP, "train: rocblas_set_stream");
     float *pb = const_cast<float *>(prm);
     const float *E = pb + t->find("tok_emb", -1)->off;
     const float *fnorm = pb + t->find("final_norm", -1)->off;
     const float *wdense = pb + t->dense_off;
     AVA_HIP(hipMemsetAsync(grads, 0, t->nparams * sizeof(float), st));
+    t->hplanes_used = 0;
+    // a named operand keeps its planes to the end of its Arena
+    auto mm = [&](bool tA, bool tB, auto &&A, auto &&B, bool add, float *C, int ldc) {
+        return gemm(t, tA, tB, A, B, std::is_lvalue_reference<decltype(A)>::value,
+                    std::is_lvalue_reference<decltype(B)>::value, add, C, ldc, st);
+    };
 
     // ------------------------------------------------------------ forward
     float *x0 = t->streams;  // stream 0: the embedding
@@ -251,7 +338,11 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
         const float *xin = i == 0 ? x0 : (c.dense ? t->xmix + (size_t)(i - 1) * Nd : t->streams + (size_t)i * Nd);
         // spiking layer: z = rms(x) Win, cur = z (1 - beta), the scan, x1 = x + s Wout
         TR(ava::train::rms_fwd(xin, N, d, w("lif_norm"), a.h1, a.inv1, st));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.h1, d, w("win"), d, 0.0f, a.z, d));
+        Arena fwd(t);  // this block's split operands
+        // (the currents stay in rocBLAS: their last bits decide spikes, and a step's spikes are those of a step
+        // before the split products; 148 us against 69 with the splits at 8192 rows)
+        Op h1{a.h1, N, d, d}, win{w("win"), d, d, d};
+        TR(gemm(t, false, false, h1, win, false, false, false, a.z, d, st, true));
         TR(ava::train::lif_params(w("beta_p"), w("theta"), w("arho"), w("again"), d, c.alif, a.ps, a.omb, st));
         if (c.lif_scale)
             TR(ava::train::scale_cols(a.z, a.omb, N, d, a.cur, st));
@@ -264,20 +355,21 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
                          t->lif_seg ? a.lpark : nullptr));
         TR(ava::train::i8_to_f32(a.spk, Nd, a.S, st));
         AVA_HIP(hipMemcpyAsync(a.x1, xin, Nd * 4, hipMemcpyDeviceToDevice, st));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.S, d, w("wout"), d, 1.0f, a.x1, d));
+        TR(mm(false, false, Op{a.S, N, d, d}, Op{w("wout"), d, d, d}, true, a.x1, d));
         // memory
         TR(ava::train::rms_fwd(a.x1, N, d, w("mem_norm"), a.h2, a.inv2, st));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.h2, d, w("wq"), d, 0.0f, a.q, d));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.h2, d, w("wk"), d, 0.0f, a.k, d));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.h2, d, w("wv"), d, 0.0f, a.v, d));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.h2, d, w("we"), d, 0.0f, a.we, d));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.h2, d, w("wg"), d, 0.0f, a.g, d));
-        TR(gemm(hb, false, false, N, nh, d, 1.0f, a.h2, d, w("wa"), nh, 0.0f, a.zab, 2 * nh));
-        TR(gemm(hb, false, false, N, nh, d, 1.0f, a.h2, d, w("wb"), nh, 0.0f, a.zab + nh, 2 * nh));
-        TR(gemm(hb, false, false, N, r, d, 1.0f, a.h2, d, w("wa1"), r, 0.0f, a.z1, 2 * r));
-        TR(gemm(hb, false, false, N, r, d, 1.0f, a.h2, d, w("wb1"), r, 0.0f, a.z1 + r, 2 * r));
-        TR(gemm(hb, false, false, N, d, r, 1.0f, a.z1, 2 * r, w("wa2"), d, 0.0f, a.lra, d));
-        TR(gemm(hb, false, false, N, d, r, 1.0f, a.z1 + r, 2 * r, w("wb2"), d, 0.0f, a.lrb, d));
+        Op h2{a.h2, N, d, d};
+        TR(mm(false, false, h2, Op{w("wq"), d, d, d}, false, a.q, d));
+        TR(mm(false, false, h2, Op{w("wk"), d, d, d}, false, a.k, d));
+        TR(mm(false, false, h2, Op{w("wv"), d, d, d}, false, a.v, d));
+        TR(mm(false, false, h2, Op{w("we"), d, d, d}, false, a.we, d));
+        TR(mm(false, false, h2, Op{w("wg"), d, d, d}, false, a.g, d));
+        TR(mm(false, false, h2, Op{w("wa"), d, nh, nh}, false, a.zab, 2 * nh));
+        TR(mm(false, false, h2, Op{w("wb"), d, nh, nh}, false, a.zab + nh, 2 * nh));
+        TR(mm(false, false, h2, Op{w("wa1"), d, r, r}, false, a.z1, 2 * r));
+        TR(mm(false, false, h2, Op{w("wb1"), d, r, r}, false, a.z1 + r, 2 * r));
+        TR(mm(false, false, Op{a.z1, N, r, 2 * r}, Op{w("wa2"), r, d, d}, false, a.lra, d));
+        TR(mm(false, false, Op{a.z1 + r, N, r, 2 * r}, Op{w("wb2"), r, d, d}, false, a.lrb, d));
         if (i == 0) vfirst = a.v;
         TrainPrep pp{a.q, a.k, a.v, a.we, a.zab, a.lra, a.lrb, w("ba"), w("bb"), w("off"),
                      (c.value_residual && i > 0) ? vfirst : nullptr, w("vres"),
@@ -289,26 +381,28 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
                         a.y, st));
         TR(ava::train::readout_fwd(a.y, a.g, B, T, nh, a.o, st));
         AVA_HIP(hipMemcpyAsync(a.x2, a.x1, Nd * 4, hipMemcpyDeviceToDevice, st));
-        TR(gemm(hb, false, false, N, d, d, 1.0f, a.o, d, w("wo"), d, 1.0f, a.x2, d));
+        TR(mm(false, false, Op{a.o, N, d, d}, Op{w("wo"), d, d, d}, true, a.x2, d));
         const float *x3 = a.x2;
         if (i == c.eng_block) {
             TR(ava::train::rms_fwd(a.x2, N, d, w("eng_norm"), a.h3, a.inv3, st));
-            TR(gemm(hb, false, false, N, de, d, 1.0f, a.h3, d, w("ewq"), de, 0.0f, a.eq, de));
-            TR(gemm(hb, false, false, N, de, d, 1.0f, a.h3, d, w("ewk"), de, 0.0f, a.ek, de));
-            TR(gemm(hb, false, false, N, de, d, 1.0f, a.h3, d, w("ewv"), de, 0.0f, a.ev, de));
+            Op h3{a.h3, N, d, d};
+            TR(split(t, h3, false, st));  // one split for three thin products
+            TR(mm(false, false, h3, Op{w("ewq"), d, de, de}, false, a.eq, de));
+            TR(mm(false, false, h3, Op{w("ewk"), d, de, de}, false, a.ek, de));
+            TR(mm(false, false, h3, Op{w("ewv"), d, de, de}, false, a.ev, de));
             TR(ava_attend_heads(a.eq, de, a.ek, a.ev, 0, T, 0, B, T, de, enh, a.att, t->att_part, t->att_part_floats,
                                 st));
             AVA_HIP(hipMemcpyAsync(a.x3, a.x2, Nd * 4, hipMemcpyDeviceToDevice, st));
-            TR(gemm(hb, false, false, N, d, de, 1.0f, a.att, de, w("ewo"), d, 1.0f, a.x3, d));
+            TR(mm(false, false, Op{a.att, N, de, de}, Op{w("ewo"), de, d, d}, true, a.x3, d));
             x3 = a.x3;
         }
         // sparse MLP; the block's raw output is stream i + 1
         float *raw = t->streams + (size_t)(i + 1) * Nd;
         TR(ava::train::rms_fwd(x3, N, d, w("mlp_norm"), a.h4, a.inv4, st));
-        TR(gemm(hb, false, false, N, H, d, 1.0f, a.h4, d, w("w1"), H, 0.0f, a.u, H));
+        TR(mm(false, false, Op{a.h4, N, d, d}, Op{w("w1"), d, H, H}, false, a.u, H));
         TR(ava_kwta(a.u, N, H, c.kwta_k, 1, a.a, a.kth, st));
         AVA_HIP(hipMemcpyAsync(raw, x3, Nd * 4, hipMemcpyDeviceToDevice, st));
-        TR(gemm(hb, false, false, N, d, H, 1.0f, a.a, H, w("w2"), d, 1.0f, raw, d));
+        TR(mm(false, false, Op{a.a, N, H, H}, Op{w("w2"), H, d, d}, true, raw, d));
         if (c.dense) {
             std::vector<const float *> ss(i + 2);
             for (int j = 0; j <= i + 1; j++) ss[j] = t->streams + (size_t)j * Nd;
@@ -317,13 +411,13 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
     }
     const float *xL = c.dense ? t->xmix + (size_t)(L - 1) * Nd : t->streams + (size_t)L * Nd;
     TR(ava::train::rms_fwd(xL, N, d, fnorm, t->hf, t->invf, st));
-    TR(gemm(hb, false, true, N, V, d, 1.0f, t->hf, d, E, d, 0.0f, t->logits, V));
+    TR(mm(false, true, Op{t->hf, N, d, d}, Op{E, V, d, d}, false, t->logits, V));
     TR(ava::train::cross_entropy(t->logits, tgt, N, V, t->lse, t->lrow, t->valid, loss, t->scal, st));
 
     // ------------------------------------------------------------ backward
     float *dE = grads + t->find("tok_emb", -1)->off;
-    TR(gemm(hb, true, false, V, d, N, 1.0f, t->logits, V, t->hf, d, 0.0f, dE, d));   // dE = dlogits^T h
-    TR(gemm(hb, false, false, N, d, V, 1.0f, t->logits, V, E, d, 0.0f, t->dA, d));   // dh = dlogits E
+    TR(mm(true, false, Op{t->logits, N, V, V}, Op{t->hf, N, d, d}, false, dE, d));   // dE = dlogits^T h
+    TR(mm(false, false, Op{t->logits, N, V, V}, Op{E, V, d, d}, false, t->dA, d));   // dh = dlogits E
     float *GL = t->G + (size_t)(L - 1) * Nd;
     AVA_HIP(hipMemsetAsync(GL, 0, Nd * 4, st));
     TR(ava::train::rms_bwd(xL, t->invf, fnorm, t->dA, N, d, GL, grads + t->find("final_norm", -1)->off, t->part, st));
@@ -342,30 +436,33 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
             AVA_HIP(hipMemcpyAsync(t->dx, Gi, Nd * 4, hipMemcpyDeviceToDevice, st));
         // MLP
         const float *x3 = i == c.eng_block ? a.x3 : a.x2;
-        TR(gemm(hb, true, false, H, d, N, 1.0f, a.a, H, t->dx, d, 0.0f, gw("w2"), d));
-        TR(gemm(hb, false, true, N, H, d, 1.0f, t->dx, d, w("w2"), d, 0.0f, t->dH, H));
+        TR(mm(true, false, Op{a.a, N, H, H}, Op{t->dx, N, d, d}, false, gw("w2"), d));
+        TR(mm(false, true, Op{t->dx, N, d, d}, Op{w("w2"), H, d, d}, false, t->dH, H));
         TR(ava_kwta_relu2_bwd(a.u, a.kth, N, H, t->dH, t->dH2, st));
-        TR(gemm(hb, true, false, d, H, N, 1.0f, a.h4, d, t->dH2, H, 0.0f, gw("w1"), H));
-        TR(gemm(hb, false, true, N, d, H, 1.0f, t->dH2, H, w("w1"), H, 0.0f, t->dA, d));
+        TR(mm(true, false, Op{a.h4, N, d, d}, Op{t->dH2, N, H, H}, false, gw("w1"), H));
+        TR(mm(false, true, Op{t->dH2, N, H, H}, Op{w("w1"), d, H, H}, false, t->dA, d));
         TR(ava::train::rms_bwd(x3, a.inv4, w("mlp_norm"), t->dA, N, d, t->dx, gw("mlp_norm"), t->part, st));
         // engram
         if (i == c.eng_block) {
-            TR(gemm(hb, true, false, de, d, N, 1.0f, a.att, de, t->dx, d, 0.0f, gw("ewo"), d));
-            TR(gemm(hb, false, true, N, de, d, 1.0f, t->dx, d, w("ewo"), d, 0.0f, t->datt, de));
+            TR(mm(true, false, Op{a.att, N, de, de}, Op{t->dx, N, d, d}, false, gw("ewo"), d));
+            TR(mm(false, true, Op{t->dx, N, d, d}, Op{w("ewo"), de, d, d}, false, t->datt, de));
             TrainAttn at{a.eq, a.ek, a.ev, a.att, t->datt, t->deq, t->dek, t->dev, t->alse, t->adsum,
                          B, T, de, enh, de / enh, (float)(1.0 / sqrt((double)(de / enh)))};
             TR(ava::train::attn_bwd(at, st));
-            TR(gemm(hb, true, false, d, de, N, 1.0f, a.h3, d, t->deq, de, 0.0f, gw("ewq"), de));
-            TR(gemm(hb, true, false, d, de, N, 1.0f, a.h3, d, t->dek, de, 0.0f, gw("ewk"), de));
-            TR(gemm(hb, true, false, d, de, N, 1.0f, a.h3, d, t->dev, de, 0.0f, gw("ewv"), de));
-            TR(gemm(hb, false, true, N, d, de, 1.0f, t->deq, de, w("ewq"), de, 0.0f, t->dA, d));
-            TR(gemm(hb, false, true, N, d, de, 1.0f, t->dek, de, w("ewk"), de, 1.0f, t->dA, d));
-            TR(gemm(hb, false, true, N, d, de, 1.0f, t->dev, de, w("ewv"), de, 1.0f, t->dA, d));
+            Op h3{a.h3, N, d, d};
+            Arena eng(t);
+            TR(split(t, h3, true, st));  // one split for three thin products
+            TR(mm(true, false, h3, Op{t->deq, N, de, de}, false, gw("ewq"), de));
+            TR(mm(true, false, h3, Op{t->dek, N, de, de}, false, gw("ewk"), de));
+            TR(mm(true, false, h3, Op{t->dev, N, de, de}, false, gw("ewv"), de));
+            TR(mm(false, true, Op{t->deq, N, de, de}, Op{w("ewq"), d, de, de}, false, t->dA, d));
+            TR(mm(false, true, Op{t->dek, N, de, de}, Op{w("ewk"), d, de, de}, true, t->dA, d));
+            TR(mm(false, true, Op{t->dev, N, de, de}, Op{w("ewv"), d, de, de}, true, t->dA, d));
             TR(ava::train::rms_bwd(a.x2, a.inv3, w("eng_norm"), t->dA, N, d, t->dx, gw("eng_norm"), t->part, st));
         }
         // memory: read-out, scan, input preparation, projections
-        TR(gemm(hb, true, false, d, d, N, 1.0f, a.o, d, t->dx, d, 0.0f, gw("wo"), d));
-        TR(gemm(hb, false, true, N, d, d, 1.0f, t->dx, d, w("wo"), d, 0.0f, t->dA, d));
+        TR(mm(true, false, Op{a.o, N, d, d}, Op{t->dx, N, d, d}, false, gw("wo"), d));
+        TR(mm(false, true, Op{t->dx, N, d, d}, Op{w("wo"), d, d, d}, false, t->dA, d));
         TR(ava::train::readout_bwd(a.y, a.g, t->dA, B, T, nh, t->dB, t->dg, st));
         TR(ava_mem_scan_bwd(a.hq, a.hk, a.he, a.hv, a.hla, a.hb, B * nh, T, 64, 64, c.momentum, c.cap, nullptr,
                             nullptr, t->dB, nullptr, nullptr, t->dq, t->dk, t->de, t->dv, t->dla, t->db, nullptr,
@@ -378,32 +475,34 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
         TR(ava::train::prep_bwd(pp, pg, st));
         if (res) TR(ava::train::colsum(t->vres_part, N * nh, 2, 2, gw("vres"), 0, t->part, st));
         if (i == 0 && c.value_residual) TR(ava::train::axpy(t->dv_raw, t->dvfirst, 1.0f, Nd, st));
+        Arena mem(t);
+        Op h2{a.h2, N, d, d};
         const float *dps[5] = {t->dq_raw, t->dk_raw, t->dv_raw, t->dwe, t->dg};
         const char *wn[5] = {"wq", "wk", "wv", "we", "wg"};
         for (int p = 0; p < 5; p++) {
-            TR(gemm(hb, true, false, d, d, N, 1.0f, a.h2, d, dps[p], d, 0.0f, gw(wn[p]), d));
-            TR(gemm(hb, false, true, N, d, d, 1.0f, dps[p], d, w(wn[p]), d, p == 0 ? 0.0f : 1.0f, t->dA, d));
+            TR(mm(true, false, h2, Op{dps[p], N, d, d}, false, gw(wn[p]), d));
+            TR(mm(false, true, Op{dps[p], N, d, d}, Op{w(wn[p]), d, d, d}, p > 0, t->dA, d));
         }
         // the head gates and their biases
-        TR(gemm(hb, true, false, d, nh, N, 1.0f, a.h2, d, t->dzab, 2 * nh, 0.0f, gw("wa"), nh));
-        TR(gemm(hb, true, false, d, nh, N, 1.0f, a.h2, d, t->dzab + nh, 2 * nh, 0.0f, gw("wb"), nh));
-        TR(gemm(hb, false, true, N, d, nh, 1.0f, t->dzab, 2 * nh, w("wa"), nh, 1.0f, t->dA, d));
-        TR(gemm(hb, false, true, N, d, nh, 1.0f, t->dzab + nh, 2 * nh, w("wb"), nh, 1.0f, t->dA, d));
+        TR(mm(true, false, h2, Op{t->dzab, N, nh, 2 * nh}, false, gw("wa"), nh));
+        TR(mm(true, false, h2, Op{t->dzab + nh, N, nh, 2 * nh}, false, gw("wb"), nh));
+        TR(mm(false, true, Op{t->dzab, N, nh, 2 * nh}, Op{w("wa"), d, nh, nh}, true, t->dA, d));
+        TR(mm(false, true, Op{t->dzab + nh, N, nh, 2 * nh}, Op{w("wb"), d, nh, nh}, true, t->dA, d));
         TR(ava::train::colsum(t->dzab, N, nh, 2 * nh, gw("ba"), 0, t->part, st));
         TR(ava::train::colsum(t->dzab + nh, N, nh, 2 * nh, gw("bb"), 0, t->part, st));
         // the rank-r read-outs: lr = (h Wx1) Wx2
         const float *dlr[2] = {t->dza, t->dzb};
         const char *w1n[2] = {"wa1", "wb1"}, *w2n[2] = {"wa2", "wb2"};
         for (int p = 0; p < 2; p++) {
-            TR(gemm(hb, true, false, r, d, N, 1.0f, a.z1 + p * r, 2 * r, dlr[p], d, 0.0f, gw(w2n[p]), d));
-            TR(gemm(hb, false, true, N, r, d, 1.0f, dlr[p], d, w(w2n[p]), d, 0.0f, t->dz1 + p * r, 2 * r));
-            TR(gemm(hb, true, false, d, r, N, 1.0f, a.h2, d, t->dz1 + p * r, 2 * r, 0.0f, gw(w1n[p]), r));
-            TR(gemm(hb, false, true, N, d, r, 1.0f, t->dz1 + p * r, 2 * r, w(w1n[p]), r, 1.0f, t->dA, d));
+            TR(mm(true, false, Op{a.z1 + p * r, N, r, 2 * r}, Op{dlr[p], N, d, d}, false, gw(w2n[p]), d));
+            TR(mm(false, true, Op{dlr[p], N, d, d}, Op{w(w2n[p]), r, d, d}, false, t->dz1 + p * r, 2 * r));
+            TR(mm(true, false, h2, Op{t->dz1 + p * r, N, r, 2 * r}, false, gw(w1n[p]), r));
+            TR(mm(false, true, Op{t->dz1 + p * r, N, r, 2 * r}, Op{w(w1n[p]), d, r, r}, true, t->dA, d));
         }
         TR(ava::train::rms_bwd(a.x1, a.inv2, w("mem_norm"), t->dA, N, d, t->dx, gw("mem_norm"), t->part, st));
         // spiking layer
-        TR(gemm(hb, true, false, d, d, N, 1.0f, a.S, d, t->dx, d, 0.0f, gw("wout"), d));
-        TR(gemm(hb, false, true, N, d, d, 1.0f, t->dx, d, w("wout"), d, 0.0f, t->dA, d));  // dL/dspikes
+        TR(mm(true, false, Op{a.S, N, d, d}, Op{t->dx, N, d, d}, false, gw("wout"), d));
+        TR(mm(false, true, Op{t->dx, N, d, d}, Op{w("wout"), d, d, d}, false, t->dA, d));  // dL/dspikes
         AVA_HIP(hipMemsetAsync(t->lv, 0, (size_t)B * d * 4, st));
         if (t->lif_seg)
             TR(ava::lif_scan_bwd_seg(a.cur, B, T, d, a.ps, t->lv, t->lv, t->lv, c.levels, 1, c.alif, t->slope,
@@ -431,8 +530,8 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
             TR(ava::train::sigmoid_chain(w("arho"), t->dvec, d, gw("arho"), st));
             TR(ava::train::colsum(t->dgsh, B, d, d, gw("again"), 0, t->part, st));
         }
-        TR(gemm(hb, true, false, d, d, N, 1.0f, a.h1, d, dz, d, 0.0f, gw("win"), d));
-        TR(gemm(hb, false, true, N, d, d, 1.0f, dz, d, w("win"), d, 0.0f, t->dA, d));
+        TR(mm(true, false, Op{a.h1, N, d, d}, Op{dz, N, d, d}, false, gw("win"), d));
+        TR(mm(false, true, Op{dz, N, d, d}, Op{w("win"), d, d, d}, false, t->dA, d));
         TR(ava::train::rms_bwd(xin, a.inv1, w("lif_norm"), t->dA, N, d, t->dx, gw("lif_norm"), t->part, st));
         // dx is now dL/d(the block's input) = G_{i-1}
         if (i > 0) AVA_HIP(hipMemcpyAsync(t->G + (size_t)(i - 1) * Nd, t->dx, Nd * 4, hipMemcpyDeviceToDevice, st));

@@ -22,8 +22,22 @@ def rel(a, b):
 @pytest.mark.parametrize("name,B,T", [("tiny", 2, 16), ("tiny_heads", 2, 12), ("small", 1, 24), ("tiny", 1, 45),
                                       ("tiny_heads", 1, 70), ("tiny", 2, 200)])
 def test_train_step_matches_autograd(name, B, T):
-    from ava_amd.train import Trainer
+    check_step(name, synth.config(name), B, T)
+
+
+# Batches whose head, wide-layer and square products go to the f16 matrix cores: rows that fill neither a
+# 128-row tile nor a 64-value K block (1029, 501), K cut into parts and not, a vocabulary that is no
+# multiple of 4 (the 4-byte split passes, a ragged last tile), thin products on shared operands.
+@pytest.mark.parametrize("name,B,T,over", [("ava04_d512", 1, 501, {}), ("ava04_d512", 1, 1029, {"vocab": 5003}),
+                                           ("ava04_d1024", 3, 704, {"vocab": 300})])
+def test_train_step_on_the_matrix_cores_matches_autograd(name, B, T, over):
     cfg = synth.config(name)
+    cfg.update(layers=1, eng_block=0, **over)
+    check_step(name, cfg, B, T)
+
+
+def check_step(name, cfg, B, T):
+    from ava_amd.train import Trainer
     prm = synth.params(cfg, seed=81)
     rng = np.random.default_rng(82)
     ids = rng.integers(0, cfg["vocab"], (B, T)).astype(np.int32)
