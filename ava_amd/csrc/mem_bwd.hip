@@ -11,25 +11,29 @@
 //   db_i = k_i sv_i - a_i e_i sr_i;  dalpha_i -= b_i e_i sr_i;  de_i = -a_i b_i sr_i + sum_j dr_j F_ij;
 //   dF <- a_i gP_ij + e_i dr_j;  dla = dalpha a (summed over the head's rows for per-head gates).
 //
-// Columns of F never mix in the forward, nor in the carried gradients; only the row sums above
-// (over all 64 columns) couple them. So wave w owns columns 16w..16w+15 outright, and lane l of it
-// a 4 x 4 block: rows 4 (l & 15).., columns 16w + 4 (l >> 4)... A column sum (r, dr, dv) is 4 FMAs
-// in the lane and 4 DPP adds over the 16 lanes of a DPP row; a row sum is 4 in the lane and two
-// lane swaps over the wave's column groups, then the four waves' partials add up in LDS once per
-// CK steps.
-//
-// States for the backward come from recomputation: pass 1 replays the forward and parks (F, S)
-// every CK steps in the caller's workspace; pass 2 walks the checkpoints from the last, replays CK
-// steps from each with every state F_t kept in registers (CK + 1 of them, and r_t), and walks those
-// steps back. The inputs of CK steps are staged in LDS; the next group's are loaded meanwhile.
-// Workspace: BH x ceil(T / CK) x (1 or 2 with momentum) x 16 KB.
-#include <stdlib.h>
+// Columns of F never mix in the forward, nor in the carried gradients; only the row sums above (over all 64
+// columns) couple them, and nothing carried depends on those. So the serial part is two walks of the T
+// steps, each its own recurrence and no more, and everything else is parallel over the chunks of CK steps:
+//   1. mem_bwd_walk_kernel: the forward from (F0, S0), parking (F, S) at every chunk's start and r_j of
+//      every step; and, in other workgroups of the same launch, the reverse walk of (dF, dS) as if no
+//      element reached the bound, parking (dF, dS) at every chunk's end and dr_j of every step, and writing dv.
+//      The forward marks the workgroups in which an element did reach it.
+//   2. mem_bwd_bound_kernel: the reverse walk again, with the bound's mask, in the marked workgroups' columns
+//      (the others return at once).
+//   3. mem_bwd_rows_kernel: per (head, chunk) the steps replayed from the parked states and walked back from
+//      the parked gradients. r_j and dr_j are known, so no column sum is left: lane = row, each wave 8
+//      columns, the row sums in the lane, the per-column values in scalar registers.
+// Measured, per-channel gates and momentum: 64 heads x 2048 steps 783 us (walks 478 us under the profiler, rows 445), 16 heads 343
+// us, 256 heads 2.64 ms, 1024 heads x 512 steps 2.59 ms; one kernel that parked every 4th state and walked three times
+// in series, the last walk forming the row sums too: 2.41, 1.87, 5.14 and 3.49 ms.
+// Workspace per (head, chunk): (F, S, dF, dS) of 16 KB (F and dF without momentum), and r and dr per step.
+#include <algorithm>
 
 #include "common.h"
 
 namespace {
 
-constexpr int HS = 64, CK = 4;
+constexpr int HS = 64, CK = 16;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -45,390 +49,635 @@ __device__ __forceinline__ float sum16(float v) {
     v += dppf<0x141>(v);
     return v + dppf<0x140>(v);
 }
-// v[l] + v[l ^ 16] + v[l ^ 32] + v[l ^ 48] in every lane (the gfx950 lane swaps).
-__device__ __forceinline__ float sum_cols(float v) {
-    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
-    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
-}
 
-// v[0..19] summed over the four 16-lane groups of the wave; lane group g gets the sums of
-// v[5 g .. 5 g + 4] in w. Each lane swap exchanges a pair of values between groups, so a stage adds
-// two values per swap: v_permlane32_swap pairs v[q] with v[q + 10] across the wave's halves, then
-// v_permlane16_swap pairs u[q] with u[q + 5] across the 16-lane groups of each half.
-__device__ __forceinline__ void rs_rows(const float (&v)[20], float (&w)[5]) {
-    float u[10];
-#pragma unroll
-    for (int q = 0; q < 10; q++) {
-        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[q]), __float_as_uint(v[q + 10]), false, false);
-        u[q] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+// A column's 64 rows over 64 / R lanes (R = 4: a DPP row, R = 2: two), lane l its rows R l .. R l + R - 1: the sum
+// over those lanes, in every one of them.
+template <int R>
+__device__ __forceinline__ float col_sum(float v) {
+    v = sum16(v);
+    if (R == 2) {
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
     }
-#pragma unroll
-    for (int q = 0; q < 5; q++) {
-        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(u[q]), __float_as_uint(u[q + 5]), false, false);
-        w[q] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
-    }
+    return v;
 }
 
 struct MemBwdArgs {
     const float *q, *k, *e, *v, *la, *b, *F0, *S0, *dy, *dFT, *dST;
-    float *dq, *dk, *de, *dv, *dla, *db, *dF0, *dS0, *ck, *part;
-    int T;
+    float *dq, *dk, *de, *dv, *dla, *db, *dF0, *dS0;
+    float *ck;       // [BH][chunk][state][64 columns][64 rows]: F, dF (and S, dS with momentum)
+    float *r, *dr;   // [BH][T][64]
+    int *hit;        // [BH][groups]: an element of the forward workgroup's columns reached the bound
+    int groups, BH, T;
     float m, cap;
 };
 
+// Whether an element of the head reached the bound, by the forward walk's workgroups.
+__device__ __forceinline__ bool head_hit(const MemBwdArgs &p, int bh) {
+    int any = 0;
+    for (int g = 0; g < p.groups; g++) any |= p.hit[bh * p.groups + g];
+    return any != 0;
+}
+
+// The parked state `which` of (head, chunk): 0 F, 1 dF, 2 S, 3 dS
+template <bool MOM>
+__device__ __forceinline__ float *parked(const MemBwdArgs &p, int bh, int c, int which) {
+    const int nck = (p.T + CK - 1) / CK;
+    return p.ck + (((size_t)bh * nck + c) * (MOM ? 4 : 2) + which) * (HS * HS);
+}
+
+// One chunk's inputs of a head in LDS: [step][row] each. The walks stage the next chunk while they scan this one.
 struct Stage {
-    float q[CK][HS], k[CK][HS], e[CK][HS], v[CK][HS], a[CK][HS], b[CK][HS], bk[CK][HS], abe[CK][HS], dy[CK][HS];
+    float q[CK][HS], e[CK][HS], a[CK][HS], bk[CK][HS], abe[CK][HS], c[CK][HS];  // c: v (forward), dy (reverse)
 };
 
-// One forward step on the lane's 4 x CPL block (rows i0.., columns j0..): r (the block's CPL columns of
-// e^T F, summed over all rows) is returned for the backward.
-template <bool MOM, int CPL>
-__device__ __forceinline__ void fwd_step(float (&F)[4 * CPL], float (&S)[4 * CPL], const Stage &sg, int s, int i0,
-                                         int j0, float M, float cap, float (&r)[CPL]) {
-    const f32x4 e4 = *reinterpret_cast<const f32x4 *>(&sg.e[s][i0]);
+// A thread's share of a chunk's inputs (step st, rows si .. si + 3), loaded one chunk ahead of its staging.
+template <bool G1, bool FWD>
+struct Loader {
+    f32x4 q, k, e, c, la, b;
+    __device__ __forceinline__ void load(const MemBwdArgs &p, int bh, int t0, int tid) {
+        const int t = t0 + (tid >> 4), si = (tid & 15) * 4;
+        const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+        q = k = e = c = la = b = z;
+        if (t0 < 0 || t >= p.T) return;
+        const size_t o = ((size_t)bh * p.T + t) * HS + si;
+        auto at = [&](const float *x) { return *reinterpret_cast<const f32x4 *>(x + o); };
+        k = at(p.k);
+        e = at(p.e);
+        c = at(FWD ? p.v : p.dy);
+        if (!FWD) q = at(p.q);
+        if (G1) {
+            const float l = p.la[(size_t)bh * p.T + t], g = p.b[(size_t)bh * p.T + t];
+            la = f32x4{l, l, l, l};
+            b = f32x4{g, g, g, g};
+        } else {
+            la = at(p.la);
+            b = at(p.b);
+        }
+    }
+    __device__ __forceinline__ void stage(Stage &s, int tid) const {
+        const int st = tid >> 4, si = (tid & 15) * 4;
+        f32x4 a, bk, abe;
+#pragma unroll
+        for (int z = 0; z < 4; z++) {
+            a[z] = expf(la[z]);
+            bk[z] = b[z] * k[z];
+            abe[z] = (a[z] * b[z]) * e[z];
+        }
+        auto put = [&](float (&d)[CK][HS], const f32x4 &x) { *reinterpret_cast<f32x4 *>(&d[st][si]) = x; };
+        if (!FWD) put(s.q, q);
+        put(s.e, e);
+        put(s.a, a);
+        put(s.bk, bk);
+        put(s.abe, abe);
+        put(s.c, c);
+    }
+};
+
+// The lane's operands of one step: its R rows' and its CPL columns'.
+template <int R, int CPL, bool FWD>
+struct StepIn {
+    typedef float vec __attribute__((ext_vector_type(R)));
+    vec q, e, a, k, x;
+    float c[CPL];
+    __device__ __forceinline__ void read(const Stage &s, int t, int i0, int j0) {
+        auto at = [&](const float (&d)[CK][HS]) { return *reinterpret_cast<const vec *>(&d[t][i0]); };
+        e = at(s.e);
+        x = at(s.abe);
+        k = at(s.bk);
+        a = at(s.a);
+        if (!FWD) q = at(s.q);
+#pragma unroll
+        for (int z = 0; z < CPL; z++) c[z] = s.c[t][j0 + z];
+    }
+};
+
+// One forward step on the lane's R x CPL block (element CPL ri + c): r gets the columns' e^T F.
+template <bool MOM, int R, int CPL>
+__device__ __forceinline__ void fwd_step(float (&F)[R * CPL], float (&S)[R * CPL], const StepIn<R, CPL, true> &in,
+                                         float M, float cap, float (&r)[CPL]) {
 #pragma unroll
     for (int c = 0; c < CPL; c++) {
-        float x = e4[0] * F[c];
-        x = fmaf(e4[1], F[CPL + c], x);
-        x = fmaf(e4[2], F[2 * CPL + c], x);
-        x = fmaf(e4[3], F[3 * CPL + c], x);
-        r[c] = sum16(x);
+        r[c] = in.e[0] * F[c];
+#pragma unroll
+        for (int ri = 1; ri < R; ri++) r[c] = fmaf(in.e[ri], F[CPL * ri + c], r[c]);
     }
-    float v4[CPL];
 #pragma unroll
-    for (int c = 0; c < CPL; c++) v4[c] = sg.v[s][j0 + c];
-    const f32x4 a4 = *reinterpret_cast<const f32x4 *>(&sg.a[s][i0]);
-    const f32x4 k4 = *reinterpret_cast<const f32x4 *>(&sg.bk[s][i0]);
-    const f32x4 x4 = *reinterpret_cast<const f32x4 *>(&sg.abe[s][i0]);
+    for (int c = 0; c < CPL; c++) r[c] = col_sum<R>(r[c]);
 #pragma unroll
-    for (int ri = 0; ri < 4; ri++)
+    for (int ri = 0; ri < R; ri++)
 #pragma unroll
         for (int c = 0; c < CPL; c++) {
             const int m = CPL * ri + c;
-            const float u = fmaf(-x4[ri], r[c], k4[ri] * v4[c]);
+            const float u = fmaf(-in.x[ri], r[c], in.k[ri] * in.c[c]);
             float f;
             if (MOM) {
                 S[m] = fmaf(M, S[m], u);
-                f = fmaf(a4[ri], F[m], S[m]);
+                f = fmaf(in.a[ri], F[m], S[m]);
             } else {
-                f = fmaf(a4[ri], F[m], u);
+                f = fmaf(in.a[ri], F[m], u);
             }
             F[m] = __builtin_amdgcn_fmed3f(f, -cap, cap);
         }
 }
 
-// NCG workgroups per head, each owning 64 / NCG of its value columns: NCG = 1, wave w owns columns
-// 16w.. and lane group g = lane / 16 four of them (CPL = 4); NCG = 4 (few heads: four times the
-// workgroups), workgroup cg owns columns 16cg.., wave w four of them and lane group g one (CPL = 1).
-// The rows' sums over the workgroup's columns then go to `part` [BH][NCG][T][5][64] and mem_bwd_rows
-// adds the column groups in order.
-template <bool G1, bool MOM, int NCG>
-__global__ __launch_bounds__(256, 2) void mem_bwd_kernel(MemBwdArgs p) {
-    constexpr int CPL = 4 / NCG, NE = 4 * CPL;
-    __shared__ __attribute__((aligned(16))) Stage sg;
-    __shared__ float red[CK][4][5][HS];  // per step, wave and row: dq, sum gP F, sv, sr, sum dr F
+// One reverse step: (dF, dS) before it from those after it. Fb: F after the step, where the bound's mask is wanted
+// (NULL: it passes every gradient). dr, dv: the columns' sums.
+template <bool MOM, int R, int CPL>
+__device__ __forceinline__ void rev_step(float (&dF)[R * CPL], float (&dS)[R * CPL], const StepIn<R, CPL, false> &in,
+                                         float M, const float *Fb, float cap, float (&dr)[CPL], float (&dv)[CPL]) {
+#pragma unroll
+    for (int c = 0; c < CPL; c++) dr[c] = dv[c] = 0.0f;
+#pragma unroll
+    for (int ri = 0; ri < R; ri++)
+#pragma unroll
+        for (int c = 0; c < CPL; c++) {
+            const int m = CPL * ri + c;
+            float gP = fmaf(in.q[ri], in.c[c], dF[m]);
+            if (Fb) gP = fabsf(Fb[m]) < cap ? gP : 0.0f;
+            float du = gP;
+            if (MOM) {
+                du = gP + dS[m];
+                dS[m] = M * du;
+            }
+            dr[c] = fmaf(-du, in.x[ri], dr[c]);
+            dv[c] = fmaf(du, in.k[ri], dv[c]);
+            dF[m] = in.a[ri] * gP;
+        }
+#pragma unroll
+    for (int c = 0; c < CPL; c++) {
+        dr[c] = col_sum<R>(dr[c]);
+        dv[c] = col_sum<R>(dv[c]);
+    }
+#pragma unroll
+    for (int ri = 0; ri < R; ri++)
+#pragma unroll
+        for (int c = 0; c < CPL; c++) dF[CPL * ri + c] = fmaf(in.e[ri], dr[c], dF[CPL * ri + c]);
+}
 
-    const int wg = blockIdx.x, bh = wg / NCG, cg = wg - bh * NCG;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int i0 = 4 * (lane & 15);
-    const int j0 = (NCG == 1 ? 16 * wave : 16 * cg + 4 * wave) + CPL * (lane >> 4);
+template <int R, int CPL>
+__device__ __forceinline__ void park(float *dst, const float (&X)[R * CPL], int i0, int j0) {
+    typedef float vec __attribute__((ext_vector_type(R)));
+#pragma unroll
+    for (int c = 0; c < CPL; c++) {
+        vec v;
+#pragma unroll
+        for (int ri = 0; ri < R; ri++) v[ri] = X[CPL * ri + c];
+        *reinterpret_cast<vec *>(dst + (j0 + c) * HS + i0) = v;
+    }
+}
+
+// 1. The walks. 4 / CPL workgroups per head and direction, each 16 CPL columns: lane l of wave w holds rows 4 (l &
+// 15).. + 3 of the CPL columns from j0, so a column sum is 4 FMAs and 4 DPP adds. A step's time is the dependent
+// chain through that sum and back (about 15 operations) against its issue and its LDS reads (5 16-byte vectors a
+// wave, 8 cycles of the CU's LDS each): step t + 1's operands are read during step t, and one barrier per chunk
+// covers the staging of the next. A wave alone on its SIMD issues one VALU operation per 8 cycles, two waves share
+// them: so few heads are split into more, smaller workgroups (2 rows a lane up to 32 heads; 4 rows of 1, 2 and 4
+// columns up to 64, 128 and beyond, where the operations per element fall: 9, 8 and 7 forward). 64 heads: 478 us with 1
+// column a lane (two waves per SIMD), 468 with 2 (one wave). The columns' r (dr, dv) of step s stay in lane s of the 16, so a chunk's go out in
+// one store. Workgroups: the forward walks first, then the reverse.
+template <bool G1, bool MOM, int R, int CPL>
+__global__ __launch_bounds__(256) void mem_bwd_walk_kernel(MemBwdArgs p) {
+    constexpr int LPC = HS / R, WC = CPL * R, NG = HS / (4 * WC), NE = R * CPL;  // lanes a column, columns a wave
+    __shared__ __attribute__((aligned(16))) Stage sg[2];
+    const bool rev = (int)blockIdx.x >= p.BH * NG;
+    const int wg = blockIdx.x - (rev ? p.BH * NG : 0), bh = wg / NG, cg = wg - bh * NG;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lc = lane & (LPC - 1);
+    const int i0 = R * lc, j0 = 4 * WC * cg + WC * wave + CPL * (lane / LPC);
     const int T = p.T, nck = (T + CK - 1) / CK;
-    constexpr int NS = MOM ? 2 : 1;
-    const size_t hb = (size_t)bh * T * HS;
-    const size_t gb = G1 ? (size_t)bh * T : hb;
-    // a workgroup's checkpoints: 256 lanes x NE floats per state
-    float *ckh = p.ck + (size_t)wg * nck * NS * (256 * NE) + (size_t)tid * NE;
+    const size_t hb = (size_t)bh * T * HS, fb = (size_t)bh * HS * HS;
     const float M = p.m, cap = p.cap;
 
-    float F[NE], S[NE];
-    {
-        const size_t o0 = (size_t)bh * HS * HS;
+    if (!rev) {
+        float F[NE], S[NE], top = 0.0f;
 #pragma unroll
         for (int m = 0; m < NE; m++) {
-            const size_t o = o0 + (size_t)(i0 + m / CPL) * HS + j0 + m % CPL;
+            const size_t o = fb + (size_t)(i0 + m / CPL) * HS + j0 + m % CPL;
             F[m] = p.F0 ? p.F0[o] : 0.0f;
             S[m] = (MOM && p.S0) ? p.S0[o] : 0.0f;
         }
+        Loader<G1, true> in;
+        in.load(p, bh, 0, tid);
+        in.stage(sg[0], tid);
+        in.load(p, bh, CK, tid);
+        for (int c = 0; c < nck; c++) {
+            __syncthreads();  // chunk c is staged; everyone is done with the other buffer
+            if (c + 1 < nck) in.stage(sg[(c + 1) & 1], tid);
+            in.load(p, bh, (c + 2) * CK, tid);
+            const Stage &st = sg[c & 1];
+            park<R, CPL>(parked<MOM>(p, bh, c, 0), F, i0, j0);
+            if (MOM) park<R, CPL>(parked<MOM>(p, bh, c, 2), S, i0, j0);
+            const int n = min(CK, T - c * CK);
+            float kept[CPL];
+            auto step = [&](const StepIn<R, CPL, true> &x, int s) {
+                float r[CPL];
+                fwd_step<MOM, R, CPL>(F, S, x, M, cap, r);
+#pragma unroll
+                for (int z = 0; z < CPL; z++) kept[z] = lc == s ? r[z] : kept[z];
+#pragma unroll
+                for (int m = 0; m < NE; m++) top = fmaxf(top, fabsf(F[m]));
+            };
+#pragma unroll
+            for (int z = 0; z < CPL; z++) kept[z] = 0.0f;
+            StepIn<R, CPL, true> cur, nxt;
+            cur.read(st, 0, i0, j0);
+            if (n == CK) {
+#pragma unroll
+                for (int s = 0; s < CK; s++) {
+                    if (s + 1 < CK) nxt.read(st, s + 1, i0, j0);
+                    step(cur, s);
+                    cur = nxt;
+                }
+            } else {
+                for (int s = 0; s < n; s++) {
+                    nxt.read(st, min(s + 1, CK - 1), i0, j0);
+                    step(cur, s);
+                    cur = nxt;
+                }
+            }
+            if (lc < n)
+#pragma unroll
+                for (int z = 0; z < CPL; z++) p.r[hb + (size_t)(c * CK + lc) * HS + j0 + z] = kept[z];
+        }
+        // (a bounded element holds +-cap, a NaN became -cap)
+        const int any = __syncthreads_or(!(top < cap));
+        if (tid == 0) p.hit[bh * NG + cg] = any;
+        return;
     }
 
-    // staging: thread -> (step st of the group, channel cc); the loads of a group are issued one
-    // group ahead
-    const int st = tid >> 6, cc = tid & 63;
-    float lq = 0, lk = 0, le = 0, lv = 0, ll = 0, lb = 0, ld = 0;
-    auto load = [&](int t0, bool bwd) {
-        const int t = t0 + st;
-        if (t < T && t0 >= 0) {
-            const size_t o = hb + (size_t)t * HS + cc;
-            lk = p.k[o];
-            le = p.e[o];
-            lv = p.v[o];
-            const size_t og = G1 ? gb + t : o;
-            ll = p.la[og];
-            lb = p.b[og];
-            if (bwd) {
-                lq = p.q[o];
-                ld = p.dy[o];
+    float dF[NE], dS[NE];
+#pragma unroll
+    for (int m = 0; m < NE; m++) {
+        const size_t o = fb + (size_t)(i0 + m / CPL) * HS + j0 + m % CPL;
+        dF[m] = p.dFT ? p.dFT[o] : 0.0f;
+        dS[m] = (MOM && p.dST) ? p.dST[o] : 0.0f;
+    }
+    Loader<G1, false> in;
+    in.load(p, bh, (nck - 1) * CK, tid);
+    in.stage(sg[(nck - 1) & 1], tid);
+    in.load(p, bh, (nck - 2) * CK, tid);
+    for (int c = nck - 1; c >= 0; c--) {
+        __syncthreads();
+        if (c > 0) in.stage(sg[(c - 1) & 1], tid);
+        in.load(p, bh, (c - 2) * CK, tid);
+        const Stage &st = sg[c & 1];
+        park<R, CPL>(parked<MOM>(p, bh, c, 1), dF, i0, j0);
+        if (MOM) park<R, CPL>(parked<MOM>(p, bh, c, 3), dS, i0, j0);
+        const int n = min(CK, T - c * CK);
+        float keptr[CPL], keptv[CPL];
+        auto step = [&](const StepIn<R, CPL, false> &x, int s) {
+            float dr[CPL], dv[CPL];
+            rev_step<MOM, R, CPL>(dF, dS, x, M, nullptr, cap, dr, dv);
+#pragma unroll
+            for (int z = 0; z < CPL; z++) {
+                keptr[z] = lc == s ? dr[z] : keptr[z];
+                keptv[z] = lc == s ? dv[z] : keptv[z];
+            }
+        };
+#pragma unroll
+        for (int z = 0; z < CPL; z++) keptr[z] = keptv[z] = 0.0f;
+        StepIn<R, CPL, false> cur, nxt;
+        cur.read(st, n - 1, i0, j0);
+        if (n == CK) {
+#pragma unroll
+            for (int s = CK - 1; s >= 0; s--) {
+                if (s > 0) nxt.read(st, s - 1, i0, j0);
+                step(cur, s);
+                cur = nxt;
             }
         } else {
-            lq = lk = le = lv = ll = lb = ld = 0.0f;
+            for (int s = n - 1; s >= 0; s--) {
+                nxt.read(st, max(s - 1, 0), i0, j0);
+                step(cur, s);
+                cur = nxt;
+            }
         }
-    };
-    auto stage = [&]() {
-        const float a = expf(ll);
-        sg.q[st][cc] = lq;
-        sg.k[st][cc] = lk;
-        sg.e[st][cc] = le;
-        sg.v[st][cc] = lv;
-        sg.a[st][cc] = a;
-        sg.b[st][cc] = lb;
-        sg.bk[st][cc] = lb * lk;
-        sg.abe[st][cc] = (a * lb) * le;
-        sg.dy[st][cc] = ld;
-    };
-    auto park = [&](int c, const float (&X)[NE], int which) {
-        float *dst = ckh + ((size_t)c * NS + which) * (256 * NE);
+        if (lc < n) {
 #pragma unroll
-        for (int z = 0; z < NE / 4; z++)
-            *reinterpret_cast<f32x4 *>(dst + 4 * z) = f32x4{X[4 * z], X[4 * z + 1], X[4 * z + 2], X[4 * z + 3]};
-    };
-    auto unpark = [&](int c, float (&X)[NE], int which) {
-        const float *src = ckh + ((size_t)c * NS + which) * (256 * NE);
-#pragma unroll
-        for (int z = 0; z < NE / 4; z++) {
-            const f32x4 x = *reinterpret_cast<const f32x4 *>(src + 4 * z);
-            X[4 * z] = x[0];
-            X[4 * z + 1] = x[1];
-            X[4 * z + 2] = x[2];
-            X[4 * z + 3] = x[3];
-        }
-    };
-
-    // 1. the forward, parking the state at the start of every group of CK steps
-    load(0, false);
-    for (int c = 0; c < nck; c++) {
-        __syncthreads();
-        stage();
-        __syncthreads();
-        load((c + 1) * CK, false);
-        park(c, F, 0);
-        if (MOM) park(c, S, 1);
-        const int n = min(CK, T - c * CK);
-#pragma unroll
-        for (int s = 0; s < CK; s++) {
-            if (s < n) {
-                float r[CPL];
-                fwd_step<MOM, CPL>(F, S, sg, s, i0, j0, M, cap, r);
+            for (int z = 0; z < CPL; z++) {
+                const size_t o = hb + (size_t)(c * CK + lc) * HS + j0 + z;
+                p.dr[o] = keptr[z];
+                p.dv[o] = keptv[z];
             }
         }
     }
-
-    // 2. backwards, group by group
-    float dF[NE], dS[NE];
-    {
-        const size_t o0 = (size_t)bh * HS * HS;
 #pragma unroll
-        for (int m = 0; m < NE; m++) {
-            const size_t o = o0 + (size_t)(i0 + m / CPL) * HS + j0 + m % CPL;
-            dF[m] = p.dFT ? p.dFT[o] : 0.0f;
-            dS[m] = (MOM && p.dST) ? p.dST[o] : 0.0f;
-        }
+    for (int m = 0; m < NE; m++) {
+        const size_t o = fb + (size_t)(i0 + m / CPL) * HS + j0 + m % CPL;
+        if (p.dF0) p.dF0[o] = dF[m];
+        if (MOM && p.dS0) p.dS0[o] = dS[m];
     }
-    load((nck - 1) * CK, true);
+}
+
+// 2. The reverse walk with the bound's mask, for the heads in which an element reached it: every
+// chunk's states are replayed from its parked ones (r is known) and kept, then the chunk is walked back.
+template <bool G1, bool MOM>
+__global__ __launch_bounds__(256) void mem_bwd_bound_kernel(MemBwdArgs p) {
+    const int bh = blockIdx.x >> 2, cg = blockIdx.x & 3;
+    if (!head_hit(p, bh)) return;
+    __shared__ __attribute__((aligned(16))) Stage sg;
+    __shared__ float sv[CK][HS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15;
+    const int i0 = 4 * l16, j = 16 * cg + 4 * wave + (lane >> 4);
+    const int T = p.T, nck = (T + CK - 1) / CK;
+    const size_t hb = (size_t)bh * T * HS, fb = (size_t)bh * HS * HS;
+    const float M = p.m, cap = p.cap;
+    float dF[4], dS[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const size_t o = fb + (size_t)(i0 + m) * HS + j;
+        dF[m] = p.dFT ? p.dFT[o] : 0.0f;
+        dS[m] = (MOM && p.dST) ? p.dST[o] : 0.0f;
+    }
     for (int c = nck - 1; c >= 0; c--) {
-        const int t0 = c * CK, n = min(CK, T - t0);
-        __syncthreads();  // the previous group's combine is done with the staging and red
-        stage();
+        const int n = min(CK, T - c * CK);
         __syncthreads();
-        load(t0 - CK, true);  // nothing past the first group (t0 - CK < 0)
-        float Ft[CK + 1][NE], rt[CK][CPL];
-        unpark(c, Ft[0], 0);
-        if (MOM) unpark(c, S, 1);
+        Loader<G1, false> in;
+        in.load(p, bh, c * CK, tid);
+        in.stage(sg, tid);
+        for (int z = tid; z < n * HS; z += 256) sv[z / HS][z % HS] = p.v[hb + (size_t)c * CK * HS + z];
+        __syncthreads();
+        park<4, 1>(parked<MOM>(p, bh, c, 1), dF, i0, j);
+        if (MOM) park<4, 1>(parked<MOM>(p, bh, c, 3), dS, i0, j);
+        float Ft[CK + 1][4], S[4];
+        const f32x4 f0 = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, c, 0) + j * HS + i0);
+        f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (MOM) s0 = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, c, 2) + j * HS + i0);
 #pragma unroll
-        for (int s = 0; s < CK; s++) {
-            if (s < n) {
-#pragma unroll
-                for (int m = 0; m < NE; m++) Ft[s + 1][m] = Ft[s][m];
-                fwd_step<MOM, CPL>(Ft[s + 1], S, sg, s, i0, j0, M, cap, rt[s]);
-            }
+        for (int m = 0; m < 4; m++) {
+            Ft[0][m] = f0[m];
+            S[m] = s0[m];
         }
 #pragma unroll
-        for (int s = CK - 1; s >= 0; s--) {
+        for (int s = 0; s < CK; s++)
             if (s < n) {
-                const float(&Fa)[NE] = Ft[s];      // F before the step
-                const float(&Fb)[NE] = Ft[s + 1];  // after it
-                const f32x4 q4 = *reinterpret_cast<const f32x4 *>(&sg.q[s][i0]);
-                const f32x4 e4 = *reinterpret_cast<const f32x4 *>(&sg.e[s][i0]);
-                const f32x4 a4 = *reinterpret_cast<const f32x4 *>(&sg.a[s][i0]);
-                const f32x4 k4 = *reinterpret_cast<const f32x4 *>(&sg.bk[s][i0]);
-                const f32x4 x4 = *reinterpret_cast<const f32x4 *>(&sg.abe[s][i0]);
-                float v4[CPL], y4[CPL];
+                const float r = p.r[hb + (size_t)(c * CK + s) * HS + j], vj = sv[s][j];
 #pragma unroll
-                for (int cj = 0; cj < CPL; cj++) {
-                    v4[cj] = sg.v[s][j0 + cj];
-                    y4[cj] = sg.dy[s][j0 + cj];
+                for (int m = 0; m < 4; m++) {
+                    const float u = fmaf(-sg.abe[s][i0 + m], r, sg.bk[s][i0 + m] * vj);
+                    if (MOM) S[m] = fmaf(M, S[m], u);
+                    const float f = fmaf(sg.a[s][i0 + m], Ft[s][m], MOM ? S[m] : u);
+                    Ft[s + 1][m] = __builtin_amdgcn_fmed3f(f, -cap, cap);
                 }
-                float pdq[4], pal[4], psv[4], psr[4], pde[4], cdr[CPL], cdv[CPL];
+            }
 #pragma unroll
-                for (int z = 0; z < 4; z++) pdq[z] = pal[z] = psv[z] = psr[z] = pde[z] = 0.0f;
+        for (int s = CK - 1; s >= 0; s--)
+            if (s < n) {
+                StepIn<4, 1, false> x;
+                x.read(sg, s, i0, j);
+                float dr[1], dv[1];
+                rev_step<MOM, 4, 1>(dF, dS, x, M, Ft[s + 1], cap, dr, dv);
+                if (l16 == 0) {
+                    const size_t o = hb + (size_t)(c * CK + s) * HS + j;
+                    p.dr[o] = dr[0];
+                    p.dv[o] = dv[0];
+                }
+            }
+    }
 #pragma unroll
-                for (int z = 0; z < CPL; z++) cdr[z] = cdv[z] = 0.0f;
+    for (int m = 0; m < 4; m++) {
+        const size_t o = fb + (size_t)(i0 + m) * HS + j;
+        if (p.dF0) p.dF0[o] = dF[m];
+        if (MOM && p.dS0) p.dS0[o] = dS[m];
+    }
+}
+
+// 3. The rows' gradients of one (head, chunk): lane = row, wave w columns 8w .. 8w + 7. The steps are replayed from
+// the parked (F, S), every F of half a chunk kept (the first half is replayed twice: 72 registers instead of 136
+// leave room for two workgroups on a CU, whose loads and barriers then hide behind each other), and walked back
+// from the parked (dF, dS); a step's five row sums over the wave's columns go to LDS, and once per two steps (two
+// buffers, one barrier) the eight waves' are added in order. 17 VALU operations per element and step (21 with the
+// bound's mask) and no exchange between lanes. 64 heads x 2048 steps: 445 us, of which the VALU 170 and the 1.05 GB
+// 210; keeping all 16 F (one workgroup per CU) 580, without the operands' read-ahead 487.
+constexpr int RW = 8, RG = 2, HC = CK / 2;  // waves (8 columns each), steps per combine, steps whose F are kept
+
+typedef const __attribute__((address_space(4))) float *ScalarPtr;  // uniform, not written by the kernel
+
+struct RowsLds {
+    float q[CK][HS], e[CK][HS], a[CK][HS], bk[CK][HS], abe[CK][HS];
+    float red[2][RW][RG][5][HS];  // per buffer, wave and step: dq, sum gP F, sv, sr, sum dr F
+};
+
+template <bool G1, bool MOM, bool FULL, bool BOUND>
+__device__ __forceinline__ void rows_chunk(const MemBwdArgs &p, RowsLds &L, int bh, int c, int n, int lane, int wave) {
+    constexpr int NC = HS / RW;
+    const float M = p.m, cap = p.cap;
+    const size_t hb = (size_t)bh * p.T * HS, o0 = hb + (size_t)c * CK * HS;
+    ScalarPtr v = (ScalarPtr)(p.v + o0 + NC * wave), rr = (ScalarPtr)(p.r + o0 + NC * wave);
+    const ScalarPtr dy = (ScalarPtr)(p.dy + o0 + NC * wave), drr = (ScalarPtr)(p.dr + o0 + NC * wave);
+    // the two pointers made new to the compiler: each pass over the steps loads its v and r again, where keeping a
+    // pass's for the next would spill the scalar registers
+    auto renew = [&]() {
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("" : "+s"(v), "+s"(rr));
+#endif
+    };
+    float Ft[HC + 1][NC], S[NC], dF[NC], dS[NC];
+    auto get = [&](float (&X)[NC], int which) {
+        const float *src = parked<MOM>(p, bh, c, which) + NC * wave * HS + lane;
 #pragma unroll
-                for (int ri = 0; ri < 4; ri++)
+        for (int z = 0; z < NC; z++) X[z] = src[z * HS];
+    };
+    // A step's operands are read while the step before it is computed, and not earlier (sched_barrier ends each
+    // step: the scalar registers hold two steps').
+    struct FwdIn {
+        float v[NC], r[NC], a, k, x;
+    };
+    struct RevIn {
+        float v[NC], r[NC], y[NC], d[NC], q, e, a;
+    };
+    auto read_fwd = [&](FwdIn &in, int s) {
 #pragma unroll
-                    for (int cj = 0; cj < CPL; cj++) {
-                        const int m = CPL * ri + cj;
-                        pdq[ri] = fmaf(y4[cj], Fb[m], pdq[ri]);
-                        float gP = fmaf(q4[ri], y4[cj], dF[m]);
-                        gP = fabsf(Fb[m]) < cap ? gP : 0.0f;
-                        pal[ri] = fmaf(gP, Fa[m], pal[ri]);
+        for (int z = 0; z < NC; z++) {
+            in.v[z] = v[s * HS + z];
+            in.r[z] = rr[s * HS + z];
+        }
+        in.a = L.a[s][lane];
+        in.k = L.bk[s][lane];
+        in.x = L.abe[s][lane];
+    };
+    auto read_rev = [&](RevIn &in, int s) {
+#pragma unroll
+        for (int z = 0; z < NC; z++) {
+            in.v[z] = v[s * HS + z];
+            in.r[z] = rr[s * HS + z];
+            in.y[z] = dy[s * HS + z];
+            in.d[z] = drr[s * HS + z];
+        }
+        in.q = L.q[s][lane];
+        in.e = L.e[s][lane];
+        in.a = L.a[s][lane];
+    };
+    // F after a step from F before it (S in place)
+    auto replay = [&](const FwdIn &in, const float (&Fa)[NC], float (&Fb)[NC]) {
+#pragma unroll
+        for (int z = 0; z < NC; z++) {
+            const float u = fmaf(-in.x, in.r[z], in.k * in.v[z]);
+            if (MOM) S[z] = fmaf(M, S[z], u);
+            const float f = fmaf(in.a, Fa[z], MOM ? S[z] : u);
+            Fb[z] = BOUND ? __builtin_amdgcn_fmed3f(f, -cap, cap) : f;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    get(dF, 1);
+    if (MOM) get(dS, 3);
+#pragma unroll
+    for (int h = 1; h >= 0; h--) {
+        const int s0 = h * HC;
+        if (!FULL && s0 >= n) continue;
+        get(Ft[0], 0);
+        if (MOM) get(S, 2);
+        // (an operand past the chunk's last step, read ahead, is the last step's again: in bounds, unused)
+        auto at = [&](int s) { return FULL ? s : min(s, n - 1); };
+        FwdIn fin[2];
+        read_fwd(fin[0], 0);
+        if (h) {
+#pragma unroll
+            for (int s = 0; s < HC; s++) {
+                read_fwd(fin[(s + 1) & 1], at(s + 1));
+                replay(fin[s & 1], Ft[0], Ft[0]);
+            }
+        }
+        renew();
+#pragma unroll
+        for (int s = 0; s < HC; s++)
+            if (FULL || s0 + s < n) {
+                if (s + 1 < HC) read_fwd(fin[(s + 1) & 1], at(s0 + s + 1));
+                replay(fin[s & 1], Ft[s], Ft[s + 1]);
+            }
+        renew();
+        RevIn rin[2];
+        const int top = FULL ? s0 + HC - 1 : min(s0 + HC, n) - 1;  // the half's last step
+        read_rev(rin[(HC - 1) & 1], top);
+        if (!FULL) rin[0] = rin[1];
+#pragma unroll
+        for (int g = HC / RG - 1; g >= 0; g--) {
+            const int g0 = s0 + g * RG;
+            if (!FULL && g0 >= n) continue;
+#pragma unroll
+            for (int w = RG - 1; w >= 0; w--) {
+                const int s = g0 + w;
+                if (FULL || s < n) {
+                    const float(&Fa)[NC] = Ft[g * RG + w];
+                    const float(&Fb)[NC] = Ft[g * RG + w + 1];
+                    const RevIn &in = rin[s & 1];
+                    if (g * RG + w > 0) read_rev(rin[(s - 1) & 1], s - 1);
+                    float sq = 0.0f, sa = 0.0f, sv = 0.0f, sr = 0.0f, sd = 0.0f;
+#pragma unroll
+                    for (int z = 0; z < NC; z++) {
+                        const float yz = in.y[z], dz = in.d[z];
+                        sq = fmaf(yz, Fb[z], sq);
+                        float gP = fmaf(in.q, yz, dF[z]);
+                        if (BOUND) gP = fabsf(Fb[z]) < cap ? gP : 0.0f;
+                        sa = fmaf(gP, Fa[z], sa);
                         float du = gP;
                         if (MOM) {
-                            du = gP + dS[m];
-                            dS[m] = M * du;
+                            du = gP + dS[z];
+                            dS[z] = M * du;
                         }
-                        psv[ri] = fmaf(du, v4[cj], psv[ri]);
-                        psr[ri] = fmaf(du, rt[s][cj], psr[ri]);
-                        cdr[cj] = fmaf(-du, x4[ri], cdr[cj]);
-                        cdv[cj] = fmaf(du, k4[ri], cdv[cj]);
-                        dF[m] = a4[ri] * gP;
+                        sv = fmaf(du, in.v[z], sv);
+                        sr = fmaf(du, in.r[z], sr);
+                        sd = fmaf(dz, Fa[z], sd);
+                        dF[z] = fmaf(in.e, dz, in.a * gP);
                     }
-#pragma unroll
-                for (int cj = 0; cj < CPL; cj++) {
-                    cdr[cj] = sum16(cdr[cj]);
-                    cdv[cj] = sum16(cdv[cj]);
-                }
-#pragma unroll
-                for (int ri = 0; ri < 4; ri++)
-#pragma unroll
-                    for (int cj = 0; cj < CPL; cj++) {
-                        const int m = CPL * ri + cj;
-                        pde[ri] = fmaf(cdr[cj], Fa[m], pde[ri]);
-                        dF[m] = fmaf(e4[ri], cdr[cj], dF[m]);
-                    }
-                {
-                    // the 20 row partials (quantity z, row ri: index 4 z + ri) summed over the wave's four
-                    // lane groups by a reduce-scatter: lane group g ends with the sums of 5 g .. 5 g + 4
-                    float v[20];
-#pragma unroll
-                    for (int ri = 0; ri < 4; ri++) {
-                        v[ri] = pdq[ri];
-                        v[4 + ri] = pal[ri];
-                        v[8 + ri] = psv[ri];
-                        v[12 + ri] = psr[ri];
-                        v[16 + ri] = pde[ri];
-                    }
-                    float w[5];
-                    rs_rows(v, w);
-                    const int g = lane >> 4;
-#pragma unroll
-                    for (int z = 0; z < 5; z++) {
-                        const int k = 5 * g + z;
-                        red[s][wave][k >> 2][i0 + (k & 3)] = w[z];
-                    }
-                }
-                if ((lane & 15) == 0) {
-                    float *dvp = p.dv + hb + (size_t)(t0 + s) * HS + j0;
-                    if (CPL == 4) *reinterpret_cast<f32x4 *>(dvp) = f32x4{cdv[0], cdv[CPL > 1 ? 1 : 0], cdv[CPL > 2 ? 2 : 0], cdv[CPL > 3 ? 3 : 0]};
-                    else dvp[0] = cdv[0];
+                    float(&o)[5][HS] = L.red[g & 1][wave][w];
+                    o[0][lane] = sq;
+                    o[1][lane] = sa;
+                    o[2][lane] = sv;
+                    o[3][lane] = sr;
+                    o[4][lane] = sd;
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-        }
-        __syncthreads();
-        // the rows' gradients: thread -> (step st, row cc), the four waves' partials added
-        if (st < n) {
-            const int t = t0 + st;
-            float x[5];
+            __syncthreads();  // the group's sums are in; this buffer's last ones were combined before this barrier
+            // wave 2 i (waves 0 and 2) finishes dq and dla of step i of the group, wave 2 i + 1 its dk, de and db
+            const int i = wave >> 1, s = g0 + i, t = c * CK + s;
+            if (i < RG && (FULL || s < n)) {
+                auto sum = [&](int z) {
+                    float x = L.red[g & 1][0][i][z][lane];
 #pragma unroll
-            for (int z = 0; z < 5; z++) x[z] = ((red[st][0][z][cc] + red[st][1][z][cc]) + red[st][2][z][cc]) + red[st][3][z][cc];
-            if (NCG > 1) {
-                // this workgroup's columns only: mem_bwd_rows adds the groups
-                float *pp = p.part + (((size_t)bh * NCG + cg) * T + t) * (5 * HS) + cc;
-#pragma unroll
-                for (int z = 0; z < 5; z++) pp[z * HS] = x[z];
-            } else {
-                const float a = sg.a[st][cc], b = sg.b[st][cc], k = sg.k[st][cc], e = sg.e[st][cc];
-                const size_t o = hb + (size_t)t * HS + cc;
-                p.dq[o] = x[0];
-                p.dk[o] = b * x[2];
-                p.de[o] = fmaf(-(a * b), x[3], x[4]);
-                const float dal = fmaf(-(b * e), x[3], x[1]);
-                const float dbr = fmaf(-(a * e), x[3], k * x[2]);
-                if (G1) {
-                    const float sa = ava::wave_sum(dal * a), sb = ava::wave_sum(dbr);
-                    if (cc == 0) {
-                        p.dla[gb + t] = sa;
-                        p.db[gb + t] = sb;
+                    for (int w = 1; w < RW; w++) x += L.red[g & 1][w][i][z][lane];
+                    return x;
+                };
+                const size_t o = hb + (size_t)t * HS + lane, og = G1 ? (size_t)bh * p.T + t : o;
+                const float a = L.a[s][lane], b = p.b[og], e = L.e[s][lane], sr = sum(3);
+                if ((wave & 1) == 0) {
+                    p.dq[o] = sum(0);
+                    const float da = fmaf(-(b * e), sr, sum(1)) * a;
+                    if (G1) {
+                        const float x = ava::wave_sum(da);
+                        if (lane == 0) p.dla[og] = x;
+                    } else {
+                        p.dla[o] = da;
                     }
                 } else {
-                    p.dla[o] = dal * a;
-                    p.db[o] = dbr;
+                    const float sv = sum(2);
+                    p.dk[o] = b * sv;
+                    p.de[o] = fmaf(-(a * b), sr, sum(4));
+                    const float db = fmaf(-(a * e), sr, p.k[o] * sv);
+                    if (G1) {
+                        const float x = ava::wave_sum(db);
+                        if (lane == 0) p.db[og] = x;
+                    } else {
+                        p.db[o] = db;
+                    }
                 }
             }
         }
     }
+}
+
+template <bool G1, bool MOM>
+__global__ __launch_bounds__(64 * RW, 4) void mem_bwd_rows_kernel(MemBwdArgs p) {
+    __shared__ __attribute__((aligned(16))) RowsLds L;
+    const int nck = (p.T + CK - 1) / CK, bh = blockIdx.x / nck, c = blockIdx.x - bh * nck, n = min(CK, p.T - c * CK);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+    for (int h = 0; h < CK / RW; h++) {
+        const int s = wave + RW * h;
+        if (s < n) {
+            const size_t o = ((size_t)bh * p.T + c * CK + s) * HS + lane, og = G1 ? (size_t)bh * p.T + c * CK + s : o;
+            const float a = expf(p.la[og]), b = p.b[og], e = p.e[o];
+            L.q[s][lane] = p.q[o];
+            L.e[s][lane] = e;
+            L.a[s][lane] = a;
+            L.bk[s][lane] = b * p.k[o];
+            L.abe[s][lane] = (a * b) * e;
+        }
+    }
+    // the chunk's v, dy, r and dr rows come into L2 together here; the scalar loads of a step then miss no further
+    float warm = 0.0f;
     {
-        const size_t o0 = (size_t)bh * HS * HS;
-#pragma unroll
-        for (int m = 0; m < NE; m++) {
-            const size_t o = o0 + (size_t)(i0 + m / CPL) * HS + j0 + m % CPL;
-            if (p.dF0) p.dF0[o] = dF[m];
-            if (MOM && p.dS0) p.dS0[o] = dS[m];
+        const size_t o = ((size_t)bh * p.T + c * CK) * HS + min(2 * tid, n * HS - 2);
+        for (const float *x : {p.v, p.dy, (const float *)p.r, (const float *)p.dr}) {
+            const float2 w = *reinterpret_cast<const float2 *>(x + o);
+            warm += w.x + w.y;
         }
     }
+    const bool bound = head_hit(p, bh);
+    asm volatile("" ::"v"(warm));
+    __syncthreads();
+    if (bound)
+        rows_chunk<G1, MOM, false, true>(p, L, bh, c, n, lane, wave);
+    else if (n == CK)
+        rows_chunk<G1, MOM, true, false>(p, L, bh, c, n, lane, wave);
+    else
+        rows_chunk<G1, MOM, false, false>(p, L, bh, c, n, lane, wave);
 }
 
-// The rows' gradients from the column groups' partial sums (NCG > 1): thread -> (step, row), the groups
-// added in order, then the combine of mem_bwd_kernel.
-template <bool G1, int NCG>
-__global__ __launch_bounds__(256) void mem_bwd_rows(MemBwdArgs p) {
-    const int T = p.T, tid = threadIdx.x, cc = tid & 63;
-    const int t = blockIdx.x * 4 + (tid >> 6), bh = blockIdx.y;
-    if (t >= T) return;  // whole waves (4 steps per workgroup, one wave each)
-    float x[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int g = 0; g < NCG; g++) {
-        const float *pp = p.part + (((size_t)bh * NCG + g) * T + t) * (5 * HS) + cc;
-#pragma unroll
-        for (int z = 0; z < 5; z++) x[z] = g ? x[z] + pp[z * HS] : pp[z * HS];
-    }
-    const size_t hb = (size_t)bh * T * HS, gb = G1 ? (size_t)bh * T : hb;
-    const size_t o = hb + (size_t)t * HS + cc, og = G1 ? gb + t : o;
-    const float a = expf(p.la[og]), b = p.b[og], k = p.k[o], e = p.e[o];
-    p.dq[o] = x[0];
-    p.dk[o] = b * x[2];
-    p.de[o] = fmaf(-(a * b), x[3], x[4]);
-    const float dal = fmaf(-(b * e), x[3], x[1]);
-    const float dbr = fmaf(-(a * e), x[3], k * x[2]);
-    if (G1) {
-        const float sa = ava::wave_sum(dal * a), sb = ava::wave_sum(dbr);
-        if (cc == 0) {
-            p.dla[gb + t] = sa;
-            p.db[gb + t] = sb;
-        }
-    } else {
-        p.dla[o] = dal * a;
-        p.db[o] = dbr;
-    }
-}
-
-// Column groups per head: four when there are too few heads to fill the GPU with one workgroup each
-// (AVA_MEM_BWD_GROUPS=1 or 4 chooses).
-int mem_bwd_groups(int BH) {
-    static const int forced = getenv("AVA_MEM_BWD_GROUPS") ? atoi(getenv("AVA_MEM_BWD_GROUPS")) : 0;
-    if (forced == 1 || forced == 4) return forced;
-    return BH < 512 ? 4 : 1;
+struct Layout {
+    size_t ck, r, hit;  // floats
+    size_t bytes() const { return (ck + 2 * r + hit) * sizeof(float); }
+};
+Layout layout(int BH, int T, bool mom) {
+    return {(size_t)BH * ((T + CK - 1) / CK) * (mom ? 4 : 2) * HS * HS, (size_t)BH * T * HS, (size_t)BH * 8};
 }
 
 }  // namespace
 
 extern "C" size_t ava_mem_scan_bwd_workspace(int BH, int T, int momentum) {
     if (BH <= 0 || T <= 0) return 0;
-    const int ncg = mem_bwd_groups(BH);
-    const size_t ck = (size_t)BH * ((T + CK - 1) / CK) * (momentum ? 2 : 1) * HS * HS * sizeof(float);
-    const size_t part = ncg > 1 ? (size_t)BH * ncg * T * 5 * HS * sizeof(float) : 0;
-    return ck + part;
+    return layout(BH, T, momentum != 0).bytes();
 }
 
 // The backward of ava_mem_scan (same layout and gates), from the initial state F0, S0 (nullable:
@@ -447,21 +696,28 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
     const bool mom = m != 0.0f;
     const size_t need = ava_mem_scan_bwd_workspace(BH, T, mom);
     AVA_REQUIRE(work_bytes >= need, AVA_ERR_SHAPE, "mem_scan_bwd: workspace %zu < %zu bytes", work_bytes, need);
-    const int ncg = mem_bwd_groups(BH);
-    float *ck = (float *)work;
-    float *part = ncg > 1 ? ck + (size_t)BH * ((T + CK - 1) / CK) * (mom ? 2 : 1) * HS * HS : nullptr;
+    const Layout lo = layout(BH, T, mom);
+    float *w = (float *)work;
     MemBwdArgs p{q, k, e, v, la, b, F0, mom ? S0 : nullptr, dy, dF_T, mom ? dS_T : nullptr, dq, dk, de, dv, dla, db,
-                 dF0, mom ? dS0 : nullptr, ck, part, T, m, cap};
+                 dF0, mom ? dS0 : nullptr, w, w + lo.ck, w + lo.ck + lo.r, (int *)(w + lo.ck + 2 * lo.r), 0, BH, T, m, cap};
     const hipStream_t st = (hipStream_t)stream;
-#define AVA_MB(G1_, MOM_)                                                                           \
-    do {                                                                                             \
-        if (ncg > 1) {                                                                               \
-            mem_bwd_kernel<G1_, MOM_, 4><<<BH * 4, 256, 0, st>>>(p);                                 \
-            mem_bwd_rows<G1_, 4><<<dim3(ava::ceil_div(T, 4), BH), 256, 0, st>>>(p);                       \
-        } else {                                                                                     \
-            mem_bwd_kernel<G1_, MOM_, 1><<<BH, 256, 0, st>>>(p);                                     \
-        }                                                                                            \
-    } while (0)
+    const int rows = BH * ava::ceil_div(T, CK);
+    auto walk = [&](auto kern, int groups) {
+        p.groups = groups;
+        kern<<<BH * groups * 2, 256, 0, st>>>(p);
+    };
+    auto run = [&](auto w8, auto w4, auto w2, auto w1, auto bound, auto rows_k) {
+        if (BH <= 32) walk(w8, 8);
+        else if (BH <= 64) walk(w4, 4);
+        else if (BH <= 128) walk(w2, 2);
+        else walk(w1, 1);
+        bound<<<BH * 4, 256, 0, st>>>(p);
+        rows_k<<<rows, 64 * RW, 0, st>>>(p);
+    };
+#define AVA_MB(G1_, MOM_)                                                                                            \
+    run(mem_bwd_walk_kernel<G1_, MOM_, 2, 1>, mem_bwd_walk_kernel<G1_, MOM_, 4, 1>,                                 \
+        mem_bwd_walk_kernel<G1_, MOM_, 4, 2>, mem_bwd_walk_kernel<G1_, MOM_, 4, 4>, mem_bwd_bound_kernel<G1_, MOM_>, \
+        mem_bwd_rows_kernel<G1_, MOM_>)
     if (g == 1) {
         if (mom) AVA_MB(true, true);
         else AVA_MB(true, false);

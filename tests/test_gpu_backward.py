@@ -241,6 +241,40 @@ def test_mem_bwd_many_heads():
         assert e < 1e-5, (n, e)
 
 
+def clear_heads(x, m, cap):
+    """The heads none of whose float64 states comes within 3e-7 of the bound before it is applied (a few
+    float32 roundings of a value of 0.6): there float32 decides the bound as float64 does."""
+    q, k, e, v, la, b, F, S = (z.astype(np.float64) for z in x[:8])
+    margin = np.full(q.shape[0], np.inf)
+    S = S if m else 0.0 * S
+    for t in range(q.shape[1]):
+        a, bt = np.exp(la[:, t]), b[:, t]
+        r = np.einsum("hi,hij->hj", e[:, t], F)
+        S = m * S + (bt * k[:, t])[:, :, None] * v[:, t][:, None] - (a * bt * e[:, t])[:, :, None] * r[:, None]
+        P = a[:, :, None] * F + S
+        margin = np.minimum(margin, np.abs(np.abs(P) - cap).min(axis=(1, 2)))
+        F = np.clip(P, -cap, cap)
+    return margin > 3e-7
+
+
+@pytest.mark.parametrize("BH,T", [(32, 16), (33, 33), (65, 17), (129, 47)])
+@pytest.mark.parametrize("g,m", [(64, 0.5), (1, 0.0)])
+@pytest.mark.parametrize("cap", [1e5, 0.6])
+def test_mem_bwd_walk_shapes(BH, T, g, m, cap):
+    """Each split of a head's columns over workgroups (up to 32, 64, 128 heads, more), chunks of 16 steps whole and
+    short, with the bound never and often reached (the reverse walk's second form and the masked rows)."""
+    x = mem_inputs(BH + T + g, BH, T, g)
+    print(f"mem_bwd BH={BH} T={T} g={g} m={m} cap={cap}", flush=True)
+    o = O.mem_rec_bwd(*x[:6], x[8], m=m, cap=cap, F0=x[6], S0=x[7] if m else None, dF_T=x[9],
+                      dS_T=x[10] if m else None)
+    gpu = run_mem(x, m, cap)
+    ok = clear_heads(x, m, cap)
+    assert np.mean(ok) > 0.5, np.mean(ok)
+    for n in MEM_OUT + (("dS0",) if m else ()):
+        e = rel(gpu[n][ok], o[n][ok])
+        assert e < 1e-5, (n, e)
+
+
 def test_wrappers_ignore_the_default_dtype():
     """The wrappers allocate float32 whatever torch's default dtype is (a float64 default once gave
     float64 output buffers that the kernels, writing float32, left mostly unwritten)."""
