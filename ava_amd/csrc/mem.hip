@@ -19,6 +19,8 @@
 // per (row, head) at column h of a [B T][ldg] matrix.
 #include <stdlib.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -217,131 +219,249 @@ __global__ __launch_bounds__(256) void mem_scan_kernel(MemArgs p) {
     }
 }
 
-// The same scan for few heads: each head's 64 value columns in four workgroups (the recurrence never
-// mixes columns), so B nh < 512 heads still fill the GPU. Workgroup (head, cg) owns columns 16 cg ..;
-// wave w four of them, lane l rows 4 (l & 15) .. + 3 of column 16 cg + 4 w + l / 16: a column sum is 4
-// FMAs and a sum over the 16 lanes of a DPP row. The staging is mem_scan_kernel's (every workgroup
-// stages all 64 rows of its head's inputs).
-__device__ __forceinline__ float sum16r(float v) {
-    v = sum8(v);
-    return v + dppf<0x140>(v);
+// The fused step's guard (gpu/model/fstep/arch.rs:780-783, 861-864): a non-finite gate, key, query or
+// value refuses the token before anything is committed. Here a head that stages one leaves its F and
+// S as they were (the scan keeps them in registers until the end) and marks its stream in bad.
+__device__ __forceinline__ bool finite6(float a, float b, float c, float d, float e, float f) {
+    return isfinite(a) && isfinite(b) && isfinite(c) && isfinite(d) && isfinite(e) && isfinite(f);
 }
 
-template <bool G1, bool MOM>
-__global__ __launch_bounds__(256) void mem_scan_cols_kernel(MemArgs p) {
-    __shared__ __attribute__((aligned(16))) float s_q[TS][HS], s_e[TS][HS], s_v[TS][HS];
-    __shared__ __attribute__((aligned(16))) float s_a[TS][HS], s_bk[TS][HS], s_abe[TS][HS];
-    __shared__ __attribute__((aligned(16))) float s_y[TS][16];
+// The same scan for few heads: each head's 64 value columns over several workgroups (the recurrence never mixes
+// columns), so B nh < 512 heads still fill the GPU. A lane holds R rows of CPL columns, 64 / R lanes a column; a
+// wave R CPL columns, a workgroup 4 R CPL, 16 / (R CPL) workgroups a head. A step's time is the dependent chain through a
+// column's sum and back against its issue: a wave alone on its SIMD issues one VALU operation per 8 cycles, two share
+// them, so few heads take few rows a lane. Step s + 1's operands are read from LDS during step s, the next chunk's
+// inputs are staged into the other buffer during this one's scan (one barrier a chunk), and a column's y of step s
+// stays in its lane s, so a chunk's read-outs leave in one store.
+// R = 8 (CPL = 1) sums a column in the order of scan_step's 8 x 2 blocks: the same bits as mem_scan_kernel's and
+// mem_fused_kernel's scan.
+// SRC: where the gates come from: la and b per head (SRC_HEAD) or channel (SRC_CHAN), or the block's prepared factors
+// (SRC_PREP: k holds b k, la alpha, b alpha b e; a head that stages a non-finite value leaves F and S and marks its
+// stream, as mem_fused_kernel).
+enum { SRC_HEAD = 0, SRC_CHAN = 1, SRC_PREP = 2 };
 
-    const int bh = blockIdx.x >> 2, cg = blockIdx.x & 3;
+template <int R>
+__device__ __forceinline__ float col_sum(float v) {
+    v = sum8(v);
+    if (R <= 4) v += dppf<0x140>(v);
+    if (R <= 2) v = xsum16(v);
+    return v;
+}
+
+// col_sum of N values y[s][c] per column c (N = 8 or 16 steps), lane s < N of the column's lanes with the sum of
+// y[s]: a stage adds lanes l and l ^ 1 (then of the pairs, quads, octets) and keeps half the values in each, 3 operations
+// per value kept, in col_sum's order of additions, so the sums have its bits; 45 operations for 16 steps against 16 col_sums.
+__device__ __forceinline__ float xor4_add(float a, float b, int lane) {
+    // lane l ^ 4 within 8 lanes: half_mirror (7 - l) then quad_perm [3,2,1,0] (l ^ 3 within 4)
+    const bool hi = lane & 4;
+    const float mine = hi ? b : a, other = hi ? a : b;
+    return mine + dppf<0x1B>(dppf<0x141>(other));
+}
+template <int CTRL, int BIT>
+__device__ __forceinline__ float scatter_add(float a, float b, int lane) {  // lanes with BIT set keep b's sum
+    const bool hi = lane & BIT;
+    return (hi ? b : a) + dppf<CTRL>(hi ? a : b);
+}
+template <int R, int N, int CPL>
+__device__ __forceinline__ void scatter_sum(const float (&y)[N][CPL], int lane, float (&z)[CPL]) {
+    // stage by stage, bit i of the lane picks bit i of the step. col_sum's mirrors within 8 and 16 lanes add the same
+    // quads and octets as the exchanges with lanes l ^ 4 and l ^ 8 here, where the lanes of a quad hold different steps.
+#pragma unroll
+    for (int c = 0; c < CPL; c++) {
+        float a[N / 2], b[N / 4], d[N / 8];
+#pragma unroll
+        for (int k = 0; k < N / 2; k++) a[k] = scatter_add<0xB1, 1>(y[2 * k][c], y[2 * k + 1][c], lane);
+#pragma unroll
+        for (int k = 0; k < N / 4; k++) b[k] = scatter_add<0x4E, 2>(a[2 * k], a[2 * k + 1], lane);
+#pragma unroll
+        for (int k = 0; k < N / 8; k++) d[k] = xor4_add(b[2 * k], b[2 * k + 1], lane);
+        if (N == 16) z[c] = scatter_add<0x128, 8>(d[0], d[N / 8 - 1], lane);  // row_ror:8 is xor 8 within 16 lanes
+        else z[c] = d[0];
+        if (R <= 2) z[c] = xsum16(z[c]);
+    }
+}
+
+struct ScanStage {
+    float q[TS][HS], e[TS][HS], a[TS][HS], bk[TS][HS], abe[TS][HS], v[TS][HS];
+};
+
+template <int SRC, bool MOM, int R, int CPL>
+__global__ __launch_bounds__(256) void mem_scan_split_kernel(MemArgs p, int heads, int *bad) {
+    constexpr int LPC = HS / R, WC = R * CPL, NG = HS / (4 * WC), NE = R * CPL;
+    typedef float vec __attribute__((ext_vector_type(R)));
+    __shared__ __attribute__((aligned(16))) ScanStage sg[2];
+
+    // a head's workgroups on one XCD (workgroups go round-robin over the 8): its L2 then holds the inputs once
+    int bh, cg;
+    if (heads % 8 == 0) {
+        bh = (int)blockIdx.x / (8 * NG) * 8 + (blockIdx.x & 7);
+        cg = (blockIdx.x >> 3) % NG;
+    } else {
+        bh = blockIdx.x / NG;
+        cg = blockIdx.x - bh * NG;
+    }
     const int bi = bh / p.nh, hh = bh - bi * p.nh;
     const size_t base = (size_t)bi * p.T * p.ld + (size_t)hh * HS;
-    const size_t gbase = G1 ? (size_t)bi * p.T * p.ldg + hh : (size_t)bi * p.T * p.ldg + (size_t)hh * HS;
-    const size_t ybase = (size_t)bi * p.T * p.ldy + (size_t)hh * HS + 16 * cg;
+    const size_t gbase = (size_t)bi * p.T * p.ldg + (SRC == SRC_HEAD ? hh : hh * HS);
+    const size_t ybase = (size_t)bi * p.T * p.ldy + (size_t)hh * HS;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int i0 = 4 * (lane & 15), jl = 4 * wave + (lane >> 4), j = 16 * cg + jl;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lc = lane & (LPC - 1);
+    const int i0 = R * lc, j0 = 4 * WC * cg + WC * wave + CPL * (lane / LPC);
 
-    float Fr[4], Sr[4];
+    float Fr[NE], Sr[NE];
     float *Fh = p.F + (size_t)bh * HS * HS, *Sh = MOM ? p.S + (size_t)bh * HS * HS : nullptr;
 #pragma unroll
-    for (int ri = 0; ri < 4; ri++) {
-        const int o = (i0 + ri) * HS + j;
-        Fr[ri] = Fh[o];
-        Sr[ri] = MOM ? Sh[o] : 0.0f;
+    for (int m = 0; m < NE; m++) {
+        const int o = (i0 + m / CPL) * HS + j0 + m % CPL;
+        Fr[m] = Fh[o];
+        Sr[m] = MOM ? Sh[o] : 0.0f;
     }
 
     const int st = tid >> 4, si = (tid & 15) * 4;
     f32x4 rq, rk, re, rv, rla, rb;
+    int nf = 0;
     auto load = [&](int t0) {
         const int t = t0 + st;
-        if (t < p.T) {
-            const size_t o = base + (size_t)t * p.ld + si;
-            rq = *reinterpret_cast<const f32x4 *>(p.q + o);
-            rk = *reinterpret_cast<const f32x4 *>(p.k + o);
-            re = *reinterpret_cast<const f32x4 *>(p.e + o);
-            rv = *reinterpret_cast<const f32x4 *>(p.v + o);
-            if (G1) {
-                const float l = p.la[gbase + (size_t)t * p.ldg], b = p.b[gbase + (size_t)t * p.ldg];
-                rla = f32x4{l, l, l, l};
-                rb = f32x4{b, b, b, b};
-            } else {
-                const size_t og = gbase + (size_t)t * p.ldg + si;
-                rla = *reinterpret_cast<const f32x4 *>(p.la + og);
-                rb = *reinterpret_cast<const f32x4 *>(p.b + og);
-            }
+        rq = rk = re = rv = rla = rb = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (t >= p.T) return;
+        const size_t o = base + (size_t)t * p.ld + si, og = gbase + (size_t)t * p.ldg;
+        rq = *reinterpret_cast<const f32x4 *>(p.q + o);
+        rk = *reinterpret_cast<const f32x4 *>(p.k + o);
+        re = *reinterpret_cast<const f32x4 *>(p.e + o);
+        rv = *reinterpret_cast<const f32x4 *>(p.v + o);
+        if constexpr (SRC == SRC_HEAD) {
+            const float l = p.la[og], b = p.b[og];
+            rla = f32x4{l, l, l, l};
+            rb = f32x4{b, b, b, b};
         } else {
-            rq = rk = re = rv = rla = rb = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            rla = *reinterpret_cast<const f32x4 *>(p.la + og + si);
+            rb = *reinterpret_cast<const f32x4 *>(p.b + og + si);
         }
     };
-    auto stage = [&]() {
-        f32x4 a, bk, abe;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            a[c] = expf(rla[c]);
-            bk[c] = rb[c] * rk[c];
-            abe[c] = (a[c] * rb[c]) * re[c];
+    auto stage = [&](ScanStage &s) {
+        f32x4 a = rla, bk = rk, abe = rb;
+        if constexpr (SRC == SRC_PREP) {
+            nf |= !(finite6(rq[0], re[0], rv[0], rla[0], rk[0], rb[0]) && finite6(rq[1], re[1], rv[1], rla[1], rk[1], rb[1]) &&
+                    finite6(rq[2], re[2], rv[2], rla[2], rk[2], rb[2]) && finite6(rq[3], re[3], rv[3], rla[3], rk[3], rb[3]));
+        } else {
+            a = f32x4{expf(rla[0]), expf(rla[1]), expf(rla[2]), expf(rla[3])};
+            bk = rb * rk;
+            abe = (a * rb) * re;
         }
-        *reinterpret_cast<f32x4 *>(&s_q[st][si]) = rq;
-        *reinterpret_cast<f32x4 *>(&s_e[st][si]) = re;
-        *reinterpret_cast<f32x4 *>(&s_v[st][si]) = rv;
-        *reinterpret_cast<f32x4 *>(&s_a[st][si]) = a;
-        *reinterpret_cast<f32x4 *>(&s_bk[st][si]) = bk;
-        *reinterpret_cast<f32x4 *>(&s_abe[st][si]) = abe;
+        auto put = [&](float (&d)[TS][HS], const f32x4 &x) { *reinterpret_cast<f32x4 *>(&d[st][si]) = x; };
+        put(s.q, rq);
+        put(s.e, re);
+        put(s.v, rv);
+        put(s.a, a);
+        put(s.bk, bk);
+        put(s.abe, abe);
+    };
+    struct In {
+        vec e, x, k, a, q;
+        float v[CPL];
+    };
+    auto read = [&](In &in, const ScanStage &s, int t) {
+        auto at = [&](const float (&d)[TS][HS]) { return *reinterpret_cast<const vec *>(&d[t][i0]); };
+        in.e = at(s.e);
+        in.x = at(s.abe);
+        in.k = at(s.bk);
+        in.a = at(s.a);
+        in.q = at(s.q);
+#pragma unroll
+        for (int c = 0; c < CPL; c++) in.v[c] = s.v[t][j0 + c];
     };
 
     const float M = p.m, cap = p.cap;
-    load(0);
-    for (int t0 = 0; t0 < p.T; t0 += TS) {
-        __syncthreads();
-        stage();
-        __syncthreads();
-        if (t0 + TS < p.T) load(t0 + TS);
-        const int n = min(TS, p.T - t0);
-        for (int s = 0; s < n; s++) {
-            const f32x4 e4 = *reinterpret_cast<const f32x4 *>(&s_e[s][i0]);
-            float r = e4[0] * Fr[0];
-            r = fmaf(e4[1], Fr[1], r);
-            r = fmaf(e4[2], Fr[2], r);
-            r = fmaf(e4[3], Fr[3], r);
-            r = sum16r(r);
-            const float vj = s_v[s][j];
-            const f32x4 q4 = *reinterpret_cast<const f32x4 *>(&s_q[s][i0]);
-            const f32x4 a4 = *reinterpret_cast<const f32x4 *>(&s_a[s][i0]);
-            const f32x4 k4 = *reinterpret_cast<const f32x4 *>(&s_bk[s][i0]);
-            const f32x4 x4 = *reinterpret_cast<const f32x4 *>(&s_abe[s][i0]);
-            float ya = 0.0f;
+    // y: the lane's rows' share of the columns' q^T F after the step
+    auto step = [&](const In &in, float (&y)[CPL]) {
+        float r[CPL];
 #pragma unroll
-            for (int ri = 0; ri < 4; ri++) {
-                const float u = fmaf(-x4[ri], r, k4[ri] * vj);
+        for (int c = 0; c < CPL; c++) r[c] = y[c] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < R; i++)
+#pragma unroll
+            for (int c = 0; c < CPL; c++) r[c] = fmaf(in.e[i], Fr[CPL * i + c], r[c]);
+#pragma unroll
+        for (int c = 0; c < CPL; c++) r[c] = col_sum<R>(r[c]);
+#pragma unroll
+        for (int i = 0; i < R; i++)
+#pragma unroll
+            for (int c = 0; c < CPL; c++) {
+                const int m = CPL * i + c;
+                const float u = fmaf(-in.x[i], r[c], in.k[i] * in.v[c]);
                 float f;
                 if (MOM) {
-                    Sr[ri] = fmaf(M, Sr[ri], u);
-                    f = fmaf(a4[ri], Fr[ri], Sr[ri]);
+                    Sr[m] = fmaf(M, Sr[m], u);
+                    f = fmaf(in.a[i], Fr[m], Sr[m]);
                 } else {
-                    f = fmaf(a4[ri], Fr[ri], u);
+                    f = fmaf(in.a[i], Fr[m], u);
                 }
                 f = __builtin_amdgcn_fmed3f(f, -cap, cap);
-                Fr[ri] = f;
-                ya = fmaf(q4[ri], f, ya);
+                Fr[m] = f;
+                y[c] = fmaf(in.q[i], f, y[c]);
             }
-            ya = sum16r(ya);
-            if ((lane & 15) == 0) s_y[s][jl] = ya;
+    };
+    load(0);
+    stage(sg[0]);
+    load(TS);
+    for (int t0 = 0, buf = 0; t0 < p.T; t0 += TS, buf ^= 1) {
+        __syncthreads();  // the chunk is staged; everyone is done with the other buffer
+        if (t0 + TS < p.T) {
+            stage(sg[buf ^ 1]);
+            load(t0 + 2 * TS);
         }
-        __syncthreads();
-        // the chunk's read-outs of the workgroup's 16 columns: thread -> (step, 4 columns)
-        if (tid < 4 * n) {
-            const int sy = tid >> 2, c4 = (tid & 3) * 4;
-            *reinterpret_cast<f32x4 *>(p.y + ybase + (size_t)(t0 + sy) * p.ldy + c4) =
-                *reinterpret_cast<const f32x4 *>(&s_y[sy][c4]);
+        const ScanStage &sc = sg[buf];
+        const int n = min(TS, p.T - t0);
+        In in[2];
+        read(in[0], sc, 0);
+        float *yp = p.y + ybase + (size_t)t0 * p.ldy + j0;
+        if (n == TS) {
+            // KEEP steps' shares are summed together (scatter_sum): lane s of a column ends with step s's
+            constexpr int KEEP = LPC < TS ? LPC : TS;
+            float y[KEEP][CPL];
+#pragma unroll
+            for (int s = 0; s < TS; s++) {
+                if (s + 1 < TS) read(in[(s + 1) & 1], sc, s + 1);
+                step(in[s & 1], y[s % KEEP]);
+                if ((s + 1) % KEEP == 0) {
+                    float z[CPL];
+                    scatter_sum<R, KEEP, CPL>(y, lane, z);
+                    if (lc < KEEP)
+#pragma unroll
+                        for (int c = 0; c < CPL; c++) yp[(size_t)(s + 1 - KEEP + lc) * p.ldy + c] = z[c];
+                }
+            }
+        } else {
+            for (int s = 0; s < n; s++) {
+                read(in[1], sc, min(s + 1, TS - 1));
+                float y[CPL];
+                step(in[0], y);
+#pragma unroll
+                for (int c = 0; c < CPL; c++) {
+                    y[c] = col_sum<R>(y[c]);
+                    if (lc == 0) yp[(size_t)s * p.ldy + c] = y[c];
+                }
+                in[0] = in[1];
+            }
+        }
+    }
+    if (SRC == SRC_PREP) {
+        if (__syncthreads_or(nf)) {
+            if (tid == 0 && cg == 0 && bad) bad[bi] = 1;
+            return;  // nothing committed
         }
     }
 #pragma unroll
-    for (int ri = 0; ri < 4; ri++) {
-        const int o = (i0 + ri) * HS + j;
-        Fh[o] = Fr[ri];
-        if (MOM) Sh[o] = Sr[ri];
+    for (int m = 0; m < NE; m++) {
+        const int o = (i0 + m / CPL) * HS + j0 + m % CPL;
+        Fh[o] = Fr[m];
+        if (MOM) Sh[o] = Sr[m];
     }
+}
+
+template <int SRC, bool MOM, int R, int CPL>
+void launch_scan_split(const MemArgs &a, int heads, int *bad, hipStream_t st) {
+    mem_scan_split_kernel<SRC, MOM, R, CPL><<<heads * (16 / (R * CPL)), 256, 0, st>>>(a, heads, bad);
 }
 
 // ------------------------------------------------------------------ the block's memory, prep fused
@@ -364,13 +484,6 @@ struct FusedArgs {
     float *F, *S, *y;  // F, S [B nh][64][64]; y [B T][d]
     int *bad;          // [B] or NULL: streams that met a non-finite memory input
 };
-
-// The fused step's guard (gpu/model/fstep/arch.rs:780-783, 861-864): a non-finite gate, key, query or
-// value refuses the token before anything is committed. Here a head that stages one leaves its F and
-// S as they were (the scan keeps them in registers until the end) and marks its stream in bad.
-__device__ __forceinline__ bool finite6(float a, float b, float c, float d, float e, float f) {
-    return isfinite(a) && isfinite(b) && isfinite(c) && isfinite(d) && isfinite(e) && isfinite(f);
-}
 
 // The gates as the reference forms them, with the correctly rounded-to-an-ulp expf/logf and an IEEE
 // divide: a bias of a few ulp in alpha would move the fast weights by that bias over (1 - alpha), ~256x
@@ -1533,18 +1646,27 @@ int mem_scan_strided(const float *q, const float *k, const float *e, const float
     if (B == 0 || T == 0) return AVA_OK;
     MemArgs a{q, k, e, v, la, b, T, nh, ld, ldg, ldy, m, cap, F, S, y};
     dim3 block(256);
-    // fewer than 512 heads: four workgroups per head (AVA_MEM_SCAN_GROUPS=1 or 4 chooses)
+    // up to 512 heads: each over 8 to 1 workgroups, as many as the 256 CUs hold at once (three each, by LDS);
+    // T = 2048, us, mem_scan_split_kernel's choice / the next one: 64 heads 324 (2 x 1 a lane) / 367 (4 x 1), 128 425
+    // (4 x 1), 384 930 (4 x 2) / 1120 (4 x 4), 512 1140 (4 x 4) / 1190 (mem_scan_kernel); more heads: 1024 2170 / 2000.
+    // AVA_MEM_SCAN_GROUPS=1 takes mem_scan_kernel for any.
     static const int forced = getenv("AVA_MEM_SCAN_GROUPS") ? atoi(getenv("AVA_MEM_SCAN_GROUPS")) : 0;
-    const bool cols = forced == 4 || (forced != 1 && B * nh < 512);
-    if (cols) {
-        dim3 grid(B * nh * 4);
-        if (g == 1) {
-            if (m != 0.0f) mem_scan_cols_kernel<true, true><<<grid, block, 0, st>>>(a);
-            else mem_scan_cols_kernel<true, false><<<grid, block, 0, st>>>(a);
-        } else {
-            if (m != 0.0f) mem_scan_cols_kernel<false, true><<<grid, block, 0, st>>>(a);
-            else mem_scan_cols_kernel<false, false><<<grid, block, 0, st>>>(a);
-        }
+    const int heads = B * nh;
+    if (forced != 1 && heads <= 512) {
+        auto go = [&](auto src, auto mom) {
+            constexpr int S_ = decltype(src)::value;
+            constexpr bool M_ = decltype(mom)::value;
+            if (heads <= 64) launch_scan_split<S_, M_, 2, 1>(a, heads, nullptr, st);
+            else if (heads <= 128) launch_scan_split<S_, M_, 4, 1>(a, heads, nullptr, st);
+            else if (heads <= 384) launch_scan_split<S_, M_, 4, 2>(a, heads, nullptr, st);
+            else launch_scan_split<S_, M_, 4, 4>(a, heads, nullptr, st);
+        };
+        auto go2 = [&](auto src) {
+            if (m != 0.0f) go(src, std::integral_constant<bool, true>{});
+            else go(src, std::integral_constant<bool, false>{});
+        };
+        if (g == 1) go2(std::integral_constant<int, SRC_HEAD>{});
+        else go2(std::integral_constant<int, SRC_CHAN>{});
     } else {
         dim3 grid(B * nh);
         if (g == 1) {

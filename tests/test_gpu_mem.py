@@ -59,6 +59,22 @@ def test_mem_scan_matches_recurrence(g, m, T, BH):
         assert np.array_equal(S, S0)  # untouched without momentum
 
 
+# each split of a head's columns over workgroups (up to 64, 128, 384, 512 heads, more), head counts that are and are
+# not multiples of the XCDs, whole chunks of 16 steps with a short one behind them
+@pytest.mark.parametrize("BH", [64, 65, 129, 136, 385, 392, 513])
+@pytest.mark.parametrize("g,m,T", [(64, 0.5, 33), (1, 0.0, 16)])
+def test_mem_scan_splits_match_recurrence(BH, g, m, T):
+    print(f"mem_scan BH={BH} g={g} m={m} T={T}", flush=True)
+    q, k, e, v, la, b = inputs(BH, T, g, BH + T)
+    from ava_amd import ops
+    y, F, S = ops.mem_gen(cuda(q), cuda(k), cuda(e), cuda(v), cuda(la), cuda(b), m=m)
+    y64, F64, S64 = O.mem_rec_f64(q, k, e, v, la, b, m=m)
+    # 33 steps of sums of 64 products in float32: some tens of roundings of 6e-8
+    assert rel(host(y), y64) < 1e-5 and rel(host(F), F64) < 1e-5
+    if m:
+        assert rel(host(S), S64) < 1e-5
+
+
 def test_mem_scan_cap_bounds_state():
     """gpu/mem_gen.rs:683: a tiny cap bounds every state entry (the clamp path)."""
     q, k, e, v, la, b = inputs(3, 40, 64, 11, unit=False)
