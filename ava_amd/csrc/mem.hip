@@ -497,6 +497,103 @@ __device__ __forceinline__ float gate_alpha(float z) {
 __device__ __forceinline__ float gate_sig(float z) { return 1.0f / (expf(-z) * 1.0f + 1.0f); }
 
 
+// The raw inputs of a wave's 4 steps t .. t + 3 of a head (lane = channel), rows row0 + t.. of the stream.
+struct PrepIn {
+    float q[4], k[4], v[4], w[4], v0[4], z[4], za[4], zb[4];
+};
+__device__ __forceinline__ void prep_load(const FusedArgs &p, PrepIn &in, size_t row0, int t1, int hh, int lane) {
+    const int d = p.nh * HS, ldp = 5 * d, ldg = 2 * p.nh + 2 * p.r, c = hh * HS + lane;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const size_t rw = row0 + min(t1 + s, p.T - 1);  // past the end: the last step, never used
+        const float *Pr = p.P + rw * ldp, *Gr = p.G + rw * ldg;
+        in.q[s] = Pr[c];
+        in.k[s] = Pr[d + c];
+        in.v[s] = Pr[2 * d + c];
+        in.w[s] = Pr[3 * d + c];
+        in.v0[s] = p.v0 ? p.v0[rw * d + c] : 0.0f;
+        in.z[s] = (lane & 31) < p.r ? Gr[2 * p.nh + (lane < 32 ? lane : lane - 32 + p.r)] : 0.0f;
+        in.za[s] = Gr[hh];
+        in.zb[s] = Gr[p.nh + hh];
+    }
+}
+// The memory's inputs of those steps: raw_v(s, v) with the raw value, then put(s, q, e, v, alpha, b k, alpha b e).
+// The rank-r gate read-outs of the 4 steps run on the matrix cores (v_mfma_f32_4x4x1, 16 blocks): lane l gives A =
+// z(step l & 3, jj) and B = w2(jj, channel l), and register s of the accumulator then holds sum_jj z(s, jj) w2(jj,
+// l). zs: 4 LDS rows of this wave for the z rows (free again when it returns).
+template <class RawV, class Put>
+__device__ __forceinline__ void prep_steps(const FusedArgs &p, const PrepIn &in, float *zs, const float (&s_wa2)[32][HS],
+                                           const float (&s_wb2)[32][HS], int lane, float bah, float bbh, float offc,
+                                           float p0, float p1, RawV raw_v, Put put) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) zs[s * HS + lane] = in.z[s];
+    f32x4 lra = {0.0f, 0.0f, 0.0f, 0.0f}, lrb = {0.0f, 0.0f, 0.0f, 0.0f};
+    const float *za = zs + (lane & 3) * HS;
+    for (int jj = 0; jj < p.r; jj++) {
+        lra = __builtin_amdgcn_mfma_f32_4x4x1f32(za[jj], s_wa2[jj][lane], lra, 0, 0, 0);
+        lrb = __builtin_amdgcn_mfma_f32_4x4x1f32(za[32 + jj], s_wb2[jj][lane], lrb, 0, 0, 0);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const float ek = in.k[s] + in.w[s];
+        const float sq = wsum(in.q[s] * in.q[s]), sk = wsum(in.k[s] * in.k[s]), se = wsum(ek * ek);
+        const float qn = in.q[s] * rsqrtf(sq + 1e-6f);
+        const float kn = in.k[s] * rsqrtf(sk + 1e-6f);
+        const float en = ek * rsqrtf(se + 1e-6f);
+        float v = in.v[s];
+        raw_v(s, v);
+        if (p.v0) v = v * p0 + in.v0[s] * p1;
+        const float a = gate_alpha(((in.za[s] + bah) + offc) + lra[s]);
+        const float bw = gate_sig((in.zb[s] + bbh) + lrb[s]) * 2.0f;
+        put(s, qn, en, v, a, bw * kn, (a * bw) * en);
+    }
+}
+
+// For few heads the preparation alone, into q, e, v, alpha, b k, alpha b e [B T][d] each (mem_scan_split_kernel's
+// SRC_PREP): a workgroup takes PREP_T steps of a head, its waves 4 at a time.
+constexpr int PREP_T = 64;
+struct PrepOut {
+    float *q, *e, *v, *a, *bk, *abe;
+};
+__global__ __launch_bounds__(256) void mem_prep_kernel(FusedArgs p, PrepOut o) {
+    __shared__ float s_wa2[32][HS], s_wb2[32][HS], s_z[4][4 * HS];
+    const int parts = (p.T + PREP_T - 1) / PREP_T, bh = blockIdx.x / parts, t0 = (blockIdx.x - bh * parts) * PREP_T;
+    const int d = p.nh * HS, bi = bh / p.nh, hh = bh - bi * p.nh, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = hh * HS + lane;
+    const size_t row0 = (size_t)bi * p.T;
+    for (int x = tid; x < p.r * HS; x += 256) {
+        const int rr = x >> 6, cc = x & 63;
+        s_wa2[rr][cc] = p.wa2[(size_t)rr * d + hh * HS + cc];
+        s_wb2[rr][cc] = p.wb2[(size_t)rr * d + hh * HS + cc];
+    }
+    const float offc = p.off[c], bah = p.ba[hh], bbh = p.bb[hh];
+    const float p0 = p.vres ? p.vres[0] * 1.0f + 1.0f : 0.0f, p1 = p.vres ? p.vres[1] : 0.0f;
+    PrepIn in[2];
+    prep_load(p, in[0], row0, t0 + wave * 4, hh, lane);
+    __syncthreads();
+    const int t1 = min(p.T, t0 + PREP_T);
+#pragma unroll
+    for (int k = 0; k < PREP_T / 16; k++) {
+        const int t = t0 + 16 * k + wave * 4;
+        if (t >= t1) break;
+        if (k + 1 < PREP_T / 16) prep_load(p, in[(k + 1) & 1], row0, t + 16, hh, lane);
+        prep_steps(p, in[k & 1], s_z[wave], s_wa2, s_wb2, lane, bah, bbh, offc, p0, p1,
+                   [&](int s, float v) {
+                       if (p.v0_out && t + s < t1) p.v0_out[(row0 + t + s) * d + c] = v;
+                   },
+                   [&](int s, float qn, float en, float v, float a, float bk, float abe) {
+                       if (t + s >= t1) return;
+                       const size_t x = (row0 + t + s) * d + c;
+                       o.q[x] = qn;
+                       o.e[x] = en;
+                       o.v[x] = v;
+                       o.a[x] = a;
+                       o.bk[x] = bk;
+                       o.abe[x] = abe;
+                   });
+    }
+}
+
 template <bool MOM, bool PF>
 __global__ __launch_bounds__(256, 4) void mem_fused_kernel(FusedArgs p) {
     // 40 KB of LDS and at most 128 VGPRs, so all four heads' blocks of a CU are resident at once
@@ -536,61 +633,26 @@ __global__ __launch_bounds__(256, 4) void mem_fused_kernel(FusedArgs p) {
         Sr[m] = MOM ? Sh[o] : 0.0f;
     }
 
-    // the raw inputs of this wave's 4 steps of a chunk, prefetched one chunk ahead
-    float rq[4], rk[4], rv[4], rw[4], rv0[4], rz[4], rza[4], rzb[4];
+    PrepIn raw;  // the raw inputs of this wave's 4 steps of a chunk, prefetched one chunk ahead
     int nf = 0;  // this lane staged a non-finite value
-    auto load = [&](int t0) {
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int t = min(t0 + wave * 4 + s, p.T - 1);  // past the end: the last step, never used
-            const size_t rw_ = row0 + t;
-            const float *Pr = p.P + rw_ * ldp, *Gr = p.G + rw_ * ldg;
-            rq[s] = Pr[c];
-            rk[s] = Pr[d + c];
-            rv[s] = Pr[2 * d + c];
-            rw[s] = Pr[3 * d + c];
-            rv0[s] = p.v0 ? p.v0[rw_ * d + c] : 0.0f;
-            rz[s] = (lane & 31) < p.r ? Gr[2 * p.nh + (lane < 32 ? lane : lane - 32 + p.r)] : 0.0f;
-            rza[s] = Gr[hh];
-            rzb[s] = Gr[p.nh + hh];
-        }
-    };
+    auto load = [&](int t0) { prep_load(p, raw, row0, t0 + wave * 4, hh, lane); };
     auto stage = [&](int t0) {
-        // the rank-r gate read-outs of the wave's 4 steps on the matrix cores (v_mfma_f32_4x4x1, 16
-        // blocks): lane l gives A = z(step l & 3, jj) and B = w2(jj, channel l), and register s of the
-        // accumulator then holds sum_jj z(s, jj) w2(jj, l). The z rows pass through LDS rows of s_abe
-        // that only this wave uses and rewrites below.
-        float *zs = &s_abe[wave * 4][0];
-#pragma unroll
-        for (int s = 0; s < 4; s++) zs[s * HS + lane] = rz[s];
-        f32x4 lra = {0.0f, 0.0f, 0.0f, 0.0f}, lrb = {0.0f, 0.0f, 0.0f, 0.0f};
-        const float *za = zs + (lane & 3) * HS;
-        for (int jj = 0; jj < p.r; jj++) {
-            lra = __builtin_amdgcn_mfma_f32_4x4x1f32(za[jj], s_wa2[jj][lane], lra, 0, 0, 0);
-            lrb = __builtin_amdgcn_mfma_f32_4x4x1f32(za[32 + jj], s_wb2[jj][lane], lrb, 0, 0, 0);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int st = wave * 4 + s, t = t0 + st;
-            const float ek = rk[s] + rw[s];
-            const float sq = wsum(rq[s] * rq[s]), sk = wsum(rk[s] * rk[s]), se = wsum(ek * ek);
-            const float qn = rq[s] * rsqrtf(sq + 1e-6f);
-            const float kn = rk[s] * rsqrtf(sk + 1e-6f);
-            const float en = ek * rsqrtf(se + 1e-6f);
-            float v = rv[s];
-            if (p.v0_out && t < p.T) p.v0_out[(row0 + t) * d + c] = v;
-            if (p.v0) v = v * p0 + rv0[s] * p1;
-            const float a = gate_alpha(((rza[s] + bah) + offc) + lra[s]);
-            const float bw = gate_sig((rzb[s] + bbh) + lrb[s]) * 2.0f;
-            const float bk = bw * kn, abe = (a * bw) * en;
-            if (t < p.T && !finite6(qn, en, v, a, bk, abe)) nf = 1;
-            s_q[st][lane] = qn;
-            s_e[st][lane] = en;
-            s_v[st][lane] = v;
-            s_a[st][lane] = a;
-            s_bk[st][lane] = bk;
-            s_abe[st][lane] = abe;
-        }
+        // the z rows pass through LDS rows of s_abe that only this wave uses and rewrites below
+        prep_steps(p, raw, &s_abe[wave * 4][0], s_wa2, s_wb2, lane, bah, bbh, offc, p0, p1,
+                   [&](int s, float v) {
+                       const int t = t0 + wave * 4 + s;
+                       if (p.v0_out && t < p.T) p.v0_out[(row0 + t) * d + c] = v;
+                   },
+                   [&](int s, float qn, float en, float v, float a, float bk, float abe) {
+                       const int st = wave * 4 + s;
+                       if (t0 + st < p.T && !finite6(qn, en, v, a, bk, abe)) nf = 1;
+                       s_q[st][lane] = qn;
+                       s_e[st][lane] = en;
+                       s_v[st][lane] = v;
+                       s_a[st][lane] = a;
+                       s_bk[st][lane] = bk;
+                       s_abe[st][lane] = abe;
+                   });
     };
 
     const float M = p.m, cap = p.cap;
@@ -1681,10 +1743,12 @@ int mem_scan_strided(const float *q, const float *k, const float *e, const float
     return AVA_OK;
 }
 
-// The block's memory from the raw projections P and gate projections G (see mem_fused_kernel).
+// The block's memory from the raw projections P and gate projections G (see mem_fused_kernel). prep (nullable): six
+// buffers of B T nh 64 floats for the few-heads form.
+constexpr int MEM_PREP_HEADS = 384, MEM_PREP_MIN_T = 32;
 int mem_block(const float *P, const float *G, int B, int T, int nh, int r, const float *ba, const float *bb,
               const float *off, const float *wa2, const float *wb2, const float *vres, const float *v0, float *v0_out,
-              float m, float cap, float *F, float *S, float *y, int *bad, hipStream_t st) {
+              float m, float cap, float *F, float *S, float *y, int *bad, float *const *prep, hipStream_t st) {
     AVA_REQUIRE(P && G && ba && bb && off && wa2 && wb2 && F && y, AVA_ERR_ARG, "mem_block: NULL buffer");
     AVA_REQUIRE(m == 0.0f || S, AVA_ERR_ARG, "mem_block: momentum needs S");
     AVA_REQUIRE(B > 0 && T > 0 && nh > 0 && r > 0 && r <= 32, AVA_ERR_SHAPE, "mem_block: B=%d T=%d nh=%d r=%d", B, T,
@@ -1694,6 +1758,21 @@ int mem_block(const float *P, const float *G, int B, int T, int nh, int r, const
         if (m != 0.0f) mem_step_kernel<true><<<B * nh, 256, 0, st>>>(a);
         else mem_step_kernel<false><<<B * nh, 256, 0, st>>>(a);
         AVA_LAUNCHED("mem_step");
+        return AVA_OK;
+    }
+    // few heads (three workgroups a CU, the LDS's limit, hold them): the preparation over all steps at once, then the
+    // scan with each head's columns over two workgroups, the same bits as the one kernel below, which runs a head's
+    // whole chain in one workgroup. T = 2048: 16 heads 1283 us there, 400 so; 256 heads 1372 / 640.
+    // Below two chunks of steps the second launch costs what the shorter chain saves (17 steps: 123 / 125 us a forward).
+    if (prep && B * nh <= MEM_PREP_HEADS && T >= MEM_PREP_MIN_T) {
+        const PrepOut o{prep[0], prep[1], prep[2], prep[3], prep[4], prep[5]};
+        mem_prep_kernel<<<B * nh * ceil_div(T, PREP_T), 256, 0, st>>>(a, o);
+        AVA_LAUNCHED("mem_prep");
+        const int d = nh * HS;
+        const MemArgs sa{o.q, o.bk, o.e, o.v, o.a, o.abe, T, nh, d, d, d, m, cap, F, S, y};
+        if (m != 0.0f) launch_scan_split<SRC_PREP, true, 8, 1>(sa, B * nh, bad, st);
+        else launch_scan_split<SRC_PREP, false, 8, 1>(sa, B * nh, bad, st);
+        AVA_LAUNCHED("mem_scan");
         return AVA_OK;
     }
     // the token loop (the chunk's inputs are staged by the scan's own waves); the chunked form

@@ -481,10 +481,13 @@ int forward(ava_model *m, ava_state *s, const int32_t *ids, int B, int T, float 
         }
         const bool vr = c.value_residual != 0;
         const size_t sm = (size_t)i * B * nh * 64 * 64;
+        // the wide layer's input, the currents and the normed rows are free here: scratch for few heads
+        float *const prep[6] = {m->u, m->u + (size_t)N * d, m->u + 2 * (size_t)N * d, m->u + 3 * (size_t)N * d, m->cur, m->h};
         AVA_RUN("mem_scan", ava::mem_block(m->P, m->G, B, T, nh, r, b.ba, b.bb, b.off, b.wa2, b.wb2,
                                            vr && i > 0 ? b.vres : nullptr, vr && i > 0 ? m->v0 : nullptr,
                                            vr && i == 0 ? m->v0 : nullptr, c.momentum, c.cap, s->mem_f + sm,
-                                           c.momentum != 0.0f ? s->mem_s + sm : nullptr, m->y, m->bad, st));
+                                           c.momentum != 0.0f ? s->mem_s + sm : nullptr, m->y, m->bad, H >= 4 * d ? prep : nullptr,
+                                           st));
         AVA_RUN("mem_post", ava::mem_post(m->y, N, d, m->P + 4 * d, 5 * d, P, m->xq, m->xexp, ldd, st));
         AVA_RUN("q8_gemm", ava::q8_gemm(m->xq, m->xexp, P, N, &b.wo.w, ava::Q8_ADD, m->x, d, nullptr, st));
         // the engram read

@@ -133,6 +133,44 @@ def test_config3_rows_split_across_forwards_give_the_same_bits(dev):
         assert torch.equal(getattr(st, name), torch.cat([getattr(x, name) for x in sts], dim=0)), name
 
 
+@pytest.mark.parametrize("T", [31, 32, 45])
+def test_memory_forms_give_the_same_bits(dev, T):
+    """400 heads (25 streams of 16: one kernel per block's memory) equal the same streams as 13 and 12 (208
+    and 192 heads: the preparation over all steps, then the scan over two workgroups per head) bit for bit, two blocks
+    (the second with the value residual), whole and short chunks of steps, one stream with a non-finite token:
+    it is marked and its fast weights stay in both."""
+    from ava_amd.model import Model
+    cfg = synth.config("ava04_d1024")
+    cfg.update(layers=2, eng_block=1)
+    prm = synth.params(cfg, seed=51)
+    bad = cfg["vocab"] - 1
+    prm["tok_emb"] = np.array(prm["tok_emb"], np.float32, copy=True)
+    prm["tok_emb"][bad] = np.nan
+    m = Model(cfg, prm)
+    B, cut = 25, 13
+    ids = np.random.default_rng(52).integers(0, bad, (B, T)).astype(np.int32)
+    ids[14, T // 2] = bad
+    ids = torch.from_numpy(ids).cuda()
+    print(f"memory forms B={B} T={T}", flush=True)
+    st = m.state(B, eng_cap=T)
+    whole = m.forward_with_state(ids, st)
+    assert m.nonfinite() == [14]
+    parts, sts = [], []
+    for lo, hi, want in ((0, cut, []), (cut, B, [14 - cut])):
+        sh = m.state(hi - lo, eng_cap=T)
+        parts.append(m.forward_with_state(ids[lo:hi].contiguous(), sh))
+        assert m.nonfinite() == want
+        sts.append(sh)
+    torch.cuda.synchronize()
+    clean = [r for r in range(B) if r != 14]
+    both = torch.cat(parts, dim=0).view(B, T, -1)
+    assert torch.equal(whole.view(B, T, -1)[clean], both[clean])
+    for name in ("lif_v", "lif_s", "lif_a", "mem_f", "mem_s"):
+        full, got = getattr(st, name), torch.cat([getattr(x, name) for x in sts], dim=1)
+        assert torch.equal(full[:, clean], got[:, clean]), name
+    assert not torch.any(st.mem_f[:, 14]) and not torch.any(sts[1].mem_f[:, 14 - cut])
+
+
 def test_config0_greedy_512_prompt_128_steps(dev):
     """config[0]: the d=512 model, one stream, a 512-token prompt and 128 greedy steps (argmax, the
     lowest id on ties) as Model.generate runs them (one forward per token with carried state). The
