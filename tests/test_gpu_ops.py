@@ -95,6 +95,39 @@ def test_lif_config1_shape_bit_exact(B, T, D, dev):
     assert np.mean(np.abs(spk_o) == 2) > 0  # both levels occur
 
 
+def test_lif_thresholds_outside_the_counted_form(dev):
+    """Waves (64 channels) whose thresholds may leave the finite range take the difference form: infinite and
+    huge thetas, a trace that grows (rho > 1), a carried spike of infinity, against currents that reach infinity; the
+    third wave is ordinary. Spikes, membranes and traces as the oracle's, NaN for NaN."""
+    B, T, D = 2, 70, 192
+    rng = np.random.default_rng(17)
+    cur = (rng.standard_normal((B, T, D)) * 1.5).astype(np.float32)
+    cur[0, 5, :8] = np.inf
+    cur[1, 9, 2:12] = -np.inf
+    cur[0, 30, 70:75] = np.inf
+    beta = sig(rng.uniform(1.5, 4.5, D).astype(np.float32))
+    theta = np.ones(D, np.float32)
+    theta[:4] = np.inf
+    theta[4:6] = -np.inf
+    theta[6:9] = 3e38
+    theta[130:140] = -0.3  # both signs' edges can hold at once: the counted form still
+    rho = np.full(D, 0.95, np.float32)
+    rho[64:72] = 1.5
+    gain = np.full(D, 0.05, np.float32)
+    s0 = np.zeros((B, D), np.float32)
+    s0[1, 80] = np.inf
+    z = np.zeros((B, D), np.float32)
+    ps = np.concatenate([beta, theta, rho, gain]).astype(np.float32)
+    with np.errstate(all="ignore"):
+        spk_o, v_o, s_o, a_o = O.lif_scan(cur, ps, z, s0, z, 2, True, True)
+    from ava_amd import ops
+    spk, st = ops.lif_gen(cuda(cur), cuda(beta), cuda(theta), (cuda(rho), cuda(gain)), levels=2, signed=True,
+                          init=ops.LifState(cuda(z), cuda(s0), cuda(z)))
+    assert np.array_equal(host(spk), spk_o)
+    for got, want in ((st.v, v_o), (st.s, s_o), (st.a, a_o)):
+        assert np.array_equal(host(got), want, equal_nan=True)
+
+
 # ----------------------------------------------------------------------------- kWTA
 
 
