@@ -176,6 +176,22 @@ __device__ __forceinline__ float lif_spike(float v, float th, int levels, int is
     return h;
 }
 
+// The spike for finite thresholds, as a whole number: with v - k th rounded, its sign is that of the exact
+// difference, so v - k th >= 0 is v >= k th (they part only where both are infinite). A compare and an add with
+// carry per level and side where the differences take four operations.
+template <int LEVELS, bool SIGNED>
+__device__ __forceinline__ int lif_count(float v, float th) {
+    if (!SIGNED) return v >= th ? 1 : 0;
+    int h = 0;
+#pragma unroll
+    for (int k = 1; k <= LEVELS; k++) {
+        const float kth = th * (float)k;
+        h += v >= kth ? 1 : 0;
+        h -= -v >= kth ? 1 : 0;
+    }
+    return h;
+}
+
 // lif.hip / kwta.hip / mem.hip
 // park (nullable): the state (v, s, a) at the start of every LIF_SEG_STEPS-step segment, as
 // park [segment][3][B D] (lif_park_floats), for lif_scan_bwd_seg.

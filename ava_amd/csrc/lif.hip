@@ -156,21 +156,6 @@ __global__ __launch_bounds__(256) void lif_scan_kernel(const float *__restrict__
     }
 }
 
-// The spike for finite thresholds, as a whole number: with v - k th rounded, its sign is that of the exact
-// difference, so v - k th >= 0 is v >= k th (they part only where both are infinite). A compare and an add with
-// carry per level and side where the differences take four operations.
-template <int LEVELS, bool SIGNED>
-__device__ __forceinline__ int spike_count(float v, float th) {
-    if (!SIGNED) return v >= th ? 1 : 0;
-    int h = 0;
-#pragma unroll
-    for (int k = 1; k <= LEVELS; k++) {
-        const float kth = th * (float)k;
-        h += v >= kth ? 1 : 0;
-        h -= -v >= kth ? 1 : 0;
-    }
-    return h;
-}
 // Whether every threshold theta + a gain of a chain stays far from infinity: rho in [0, 1] keeps the trace a within
 // its start, the carried spike and the spikes' largest (2).
 __device__ __forceinline__ bool finite_thresholds(float th0, float rho, float gain, float a0, float s0) {
@@ -185,7 +170,7 @@ __device__ __forceinline__ bool finite_thresholds(float th0, float rho, float ga
 // blocks of PF steps run without per-step bound checks, and a segment's parked state is written at the
 // end of its block (PF = LIF_SEG_STEPS). The same arithmetic as lif_scan_kernel, so the same bits. With up to one
 // wave per SIMD (65,536 chains) a step's time is its VALU operations at 8 cycles each, so waves whose thresholds
-// stay finite count spikes by spike_count: 20 operations a step instead of 27, 64 x 2048 x 1024 158 us instead of 202,
+// stay finite count spikes by lif_count: 20 operations a step instead of 27, 64 x 2048 x 1024 158 us instead of 202,
 // 4 x 2048 x 1024 146 instead of 176; 64 x 2048 x 2048 247 instead of 258, bound by HBM (5.4 TB/s).
 template <int PF, int LEVELS, bool SIGNED, bool ALIF>
 __global__ __launch_bounds__(256) void lif_scan_buf_kernel(const float *__restrict__ cur, int B, int T, int D,
@@ -232,7 +217,7 @@ __global__ __launch_bounds__(256) void lif_scan_buf_kernel(const float *__restri
             vv = (vv * bt + x) - sp * thp;
             int h = 0;
             if (FIN) {
-                h = spike_count<LEVELS, SIGNED>(vv, tht);
+                h = ava::lif_count<LEVELS, SIGNED>(vv, tht);
                 sp = (float)h;
             } else {
                 sp = spike_of<LEVELS, SIGNED>(vv, tht);

@@ -19,6 +19,10 @@
 //   ALIF: gth = gs ds/dth (- s_t G_{t+1}), ga = gth gain + ca, dgain += gth a_t,
 //   drho += ga (a_{t-1} - |s_{t-1}|), ca = rho ga.
 // Every operation is rounded on its own (-ffp-contract=off), in the order of the CPU statement.
+// Measured, 64 x 2048 x 2048: 960 us, 4.3 GB at 4.5 TB/s (a device copy: 5.0); 1244 us, VALU-bound, with IEEE divides
+// in the surrogates and the spikes by differences and formed again on the way back.
+#include <type_traits>
+
 #include "common.h"
 
 namespace {
@@ -35,16 +39,30 @@ __device__ __forceinline__ float spike_of(float v, float th) {
     return h;
 }
 
+// 1 / d for d in [1, 2^125) as the IEEE divide rounds it: the hardware's reciprocal (within an ulp) and one Newton
+// step with a fused residual; compared with the divide on every float of the range. 3 operations instead of about 10.
+__device__ __forceinline__ float recip(float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+
+template <int LEVELS, bool SIGNED, bool FIN>
+__device__ __forceinline__ float spike(float v, float th) {
+    return FIN ? (float)ava::lif_count<LEVELS, SIGNED>(v, th) : spike_of<LEVELS, SIGNED>(v, th);
+}
+
+// NEAR: slope |x| is below 2^60 (or NaN), so a^2 is in recip's range.
+template <bool NEAR>
 __device__ __forceinline__ float surrogate(float x, float slope) {
     const float a = 1.0f + slope * fabsf(x);
-    return 1.0f / (a * a);
+    return NEAR ? recip(a * a) : 1.0f / (a * a);
 }
 
 // d s / d v and d s / d th of one step's surrogate spike.
-template <int LEVELS, bool SIGNED>
+template <int LEVELS, bool SIGNED, bool NEAR>
 __device__ __forceinline__ void dspike(float v, float th, float slope, float &dv, float &dth) {
     if (!SIGNED) {
-        const float g = surrogate(v - th, slope);
+        const float g = surrogate<NEAR>(v - th, slope);
         dv = g;
         dth = -g;
         return;
@@ -53,12 +71,20 @@ __device__ __forceinline__ void dspike(float v, float th, float slope, float &dv
 #pragma unroll
     for (int k = 1; k <= LEVELS; k++) {
         const float kth = th * (float)k;
-        const float gu = surrogate(v - kth, slope), gd = surrogate(-v - kth, slope);
+        const float gu = surrogate<NEAR>(v - kth, slope), gd = surrogate<NEAR>(-v - kth, slope);
         a += gu + gd;
         b += (float)k * (gd - gu);
     }
     dv = a;
     dth = b;
+}
+
+// Whether a chain's thresholds stay below 3e8 (rho in [0, 1] keeps the trace within its start, the carried spike and
+// 2) and the slope below 1e6: then spikes count by ava::lif_count, and membranes below NEAR_V give NEAR surrogates.
+constexpr float NEAR_V = 1e9f;
+__device__ __forceinline__ bool tame(float th0, float rho, float gain, float a0, float s0, float slope) {
+    return fabsf(th0) < 1e8f && rho >= 0.0f && rho <= 1.0f && fabsf(gain) < 1e4f && fabsf(a0) < 1e4f &&
+           fabsf(s0) < 1e4f && slope < 1e6f;
 }
 
 struct LifBwdArgs {
@@ -69,11 +95,17 @@ struct LifBwdArgs {
     int rg;
 };
 
-template <int K, int LEVELS, bool SIGNED, bool ALIF>
-__global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+// Whether the wave's chains (this lane's: channel c, state index i) are tame.
+template <bool ALIF>
+__device__ __forceinline__ bool wave_tame(const LifBwdArgs &p, int c, int i) {
+    return __all(tame(p.ps[p.D + c], ALIF ? p.ps[2 * p.D + c] : 0.0f, ALIF ? p.ps[3 * p.D + c] : 0.0f,
+                      ALIF ? p.a0[i] : 0.0f, p.s0[i], p.slope));
+}
+
+// FIN: the wave's chains are tame.
+template <int K, int LEVELS, bool SIGNED, bool ALIF, bool FIN>
+__device__ __forceinline__ void lif_bwd_chain(const LifBwdArgs &p, int gid) {
     const int D = p.D, T = p.T;
-    if (gid >= p.B * D) return;
     const int b = gid / D, c = gid - b * D;
     const float bt = p.ps[c], th0 = p.ps[D + c], rho = p.ps[2 * D + c], gain = p.ps[3 * D + c];
     const float omr = 1.0f - rho;
@@ -114,7 +146,7 @@ __global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
                         tht = th0 + a * gain;
                     }
                     v = (v * bt + buf[i]) - sp * thp;
-                    sp = spike_of<LEVELS, SIGNED>(v, tht);
+                    sp = spike<LEVELS, SIGNED, FIN>(v, tht);
                     thp = tht;
                 }
             }
@@ -136,14 +168,13 @@ __global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
     float ckv, cks, cka, nkv = 0.0f, nks = 0.0f, nka = 0.0f;
     auto load_ck = [&](int q, float &kv, float &ks, float &ka) {
         const int t0 = seg0(q);
+        kv = v0;
+        ks = s0;
+        ka = a0;
         if (t0 > 0) {
             kv = o[(size_t)t0 * D];
             ks = o[(size_t)(t0 + 1) * D];
             ka = ALIF ? o[(size_t)(t0 + 2) * D] : 0.0f;
-        } else {
-            kv = v0;
-            ks = s0;
-            ka = a0;
         }
     };
     load_cur(0, buf);
@@ -156,7 +187,7 @@ __global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
             load_ck(q + 1, nkv, nks, nka);
         }
         const int t0 = seg0(q), n = T - q * K - t0;
-        float vs[K] = {}, as[K] = {};
+        float vs[K] = {}, as[K] = {}, ss[K] = {}, top = 0.0f;
         {
             float v = ckv, sp = cks, a = cka, thp = ALIF ? th0 + cka * gain : th0;
 #pragma unroll
@@ -168,43 +199,49 @@ __global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
                         tht = th0 + a * gain;
                     }
                     v = (v * bt + buf[i]) - sp * thp;
-                    sp = spike_of<LEVELS, SIGNED>(v, tht);
+                    sp = spike<LEVELS, SIGNED, FIN>(v, tht);
                     thp = tht;
                     vs[i] = v;
                     as[i] = a;
+                    ss[i] = sp;
+                    if (FIN) top = fmaxf(top, fabsf(v));
                 }
             }
         }
+        auto back = [&](auto near) {
+            constexpr bool NEAR = decltype(near)::value;
 #pragma unroll
-        for (int i = K - 1; i >= 0; i--) {
-            if (i < n) {
-                const float vt = vs[i], at = ALIF ? as[i] : 0.0f;
-                const float tht = ALIF ? th0 + at * gain : th0;
-                float dv, dth;
-                dspike<LEVELS, SIGNED>(vt, tht, p.slope, dv, dth);
-                float gst = gbuf[i];
-                if (p.rg) {
-                    const float qq = tht * dv, cap = 2.0f * bt;
-                    gst -= (qq > cap ? cap / dv : tht) * Gn;
+            for (int i = K - 1; i >= 0; i--) {
+                if (i < n) {
+                    const float vt = vs[i], at = ALIF ? as[i] : 0.0f;
+                    const float tht = ALIF ? th0 + at * gain : th0;
+                    float dv, dth;
+                    dspike<LEVELS, SIGNED, NEAR>(vt, tht, p.slope, dv, dth);
+                    float gst = gbuf[i];
+                    if (p.rg) {
+                        const float qq = tht * dv, cap = 2.0f * bt;
+                        gst -= (qq > cap ? cap / dv : tht) * Gn;
+                    }
+                    const float G = gst * dv + cv;
+                    gb += G * (i > 0 ? vs[i - 1] : ckv);
+                    if (ALIF) {
+                        float gth = gst * dth;
+                        if (p.rg) gth -= ss[i] * Gn;
+                        const float gaa = gth * gain + ca;
+                        gg += gth * at;
+                        const float ap = i > 0 ? as[i - 1] : cka;
+                        const float sprev = i > 0 ? ss[i - 1] : cks;
+                        gr += gaa * (ap - fabsf(sprev));
+                        ca = rho * gaa;
+                    }
+                    o[(size_t)(t0 + i) * D] = G;
+                    Gn = G;
+                    cv = bt * G;
                 }
-                const float G = gst * dv + cv;
-                gb += G * (i > 0 ? vs[i - 1] : ckv);
-                if (ALIF) {
-                    // the spikes are re-formed from the kept membranes and thresholds
-                    float gth = gst * dth;
-                    if (p.rg) gth -= spike_of<LEVELS, SIGNED>(vt, tht) * Gn;
-                    const float gaa = gth * gain + ca;
-                    gg += gth * at;
-                    const float ap = i > 0 ? as[i - 1] : cka;
-                    const float sprev = i > 0 ? spike_of<LEVELS, SIGNED>(vs[i - 1], th0 + as[i - 1] * gain) : cks;
-                    gr += gaa * (ap - fabsf(sprev));
-                    ca = rho * gaa;
-                }
-                o[(size_t)(t0 + i) * D] = G;
-                Gn = G;
-                cv = bt * G;
             }
-        }
+        };
+        if (FIN && __all(top < NEAR_V)) back(std::integral_constant<bool, true>{});
+        else back(std::integral_constant<bool, false>{});
 #pragma unroll
         for (int i = 0; i < K; i++) {
             buf[i] = nxt[i];
@@ -224,6 +261,16 @@ __global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
     p.dbeta[gid] = gb;
     if (p.drho) p.drho[gid] = ALIF ? gr : 0.0f;
     if (p.dgain) p.dgain[gid] = ALIF ? gg : 0.0f;
+}
+
+template <int K, int LEVELS, bool SIGNED, bool ALIF>
+__global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
+    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool in = gid < p.B * p.D;
+    const bool fin = wave_tame<ALIF>(p, in ? gid % p.D : 0, in ? gid : 0);
+    if (!in) return;
+    if (fin) lif_bwd_chain<K, LEVELS, SIGNED, ALIF, true>(p, gid);
+    else lif_bwd_chain<K, LEVELS, SIGNED, ALIF, false>(p, gid);
 }
 
 // Steps per segment: 5 x 16 registers of currents, gradients and replayed state. 32-step segments
@@ -271,7 +318,7 @@ __device__ __forceinline__ float *park_at(const LifSegArgs &a, int sg, int f, in
 }
 
 // one forward step of the scan (lif_scan_kernel's loop body)
-template <int LEVELS, bool SIGNED, bool ALIF>
+template <int LEVELS, bool SIGNED, bool ALIF, bool FIN>
 __device__ __forceinline__ void fwd1(float x, float bt, float th0, float rho, float omr, float gain, float &v,
                                      float &sp, float &a, float &thp) {
     float tht = th0;
@@ -280,7 +327,7 @@ __device__ __forceinline__ void fwd1(float x, float bt, float th0, float rho, fl
         tht = th0 + a * gain;
     }
     v = (v * bt + x) - sp * thp;
-    sp = spike_of<LEVELS, SIGNED>(v, tht);
+    sp = spike<LEVELS, SIGNED, FIN>(v, tht);
     thp = tht;
 }
 
@@ -298,41 +345,49 @@ __global__ __launch_bounds__(256) void lif_seg_park_kernel(LifSegArgs A) {
     *park_at(A, 0, 0, gid) = v;
     *park_at(A, 0, 1, gid) = sp;
     *park_at(A, 0, 2, gid) = a;
-    constexpr int PF = 16;
-    float buf[PF];
-    for (int t0 = 0; t0 < T; t0 += PF) {
+    // two segments' currents in flight, as the scan's
+    auto scan = [&](auto fin) {
+        constexpr bool FIN = decltype(fin)::value;
+        float buf[SK];
 #pragma unroll
-        for (int i = 0; i < PF; i++) buf[i] = t0 + i < T ? __builtin_nontemporal_load(x + (size_t)(t0 + i) * D) : 0.0f;
+        for (int i = 0; i < SK; i++) buf[i] = __builtin_nontemporal_load(x + (size_t)min(i, T - 1) * D);
+        for (int t0 = 0; t0 < T; t0 += SK) {
+            float nxt[SK];
 #pragma unroll
-        for (int i = 0; i < PF; i++) {
-            const int t = t0 + i;
-            if (t < T) {
-                fwd1<LEVELS, SIGNED, ALIF>(buf[i], bt, th0, rho, omr, gain, v, sp, a, thp);
-                if ((t + 1) % SK == 0 && t + 1 < T) {
-                    const int sg = (t + 1) / SK;
-                    *park_at(A, sg, 0, gid) = v;
-                    *park_at(A, sg, 1, gid) = sp;
-                    *park_at(A, sg, 2, gid) = a;
-                }
+            for (int i = 0; i < SK; i++) nxt[i] = __builtin_nontemporal_load(x + (size_t)min(t0 + SK + i, T - 1) * D);
+            if (t0 + SK < T) {
+#pragma unroll
+                for (int i = 0; i < SK; i++) fwd1<LEVELS, SIGNED, ALIF, FIN>(buf[i], bt, th0, rho, omr, gain, v, sp, a, thp);
+                const int sg = t0 / SK + 1;
+                *park_at(A, sg, 0, gid) = v;
+                *park_at(A, sg, 1, gid) = sp;
+                *park_at(A, sg, 2, gid) = a;
             }
+#pragma unroll
+            for (int i = 0; i < SK; i++) buf[i] = nxt[i];
         }
-    }
+    };
+    if (wave_tame<ALIF>(p, c, gid)) scan(std::integral_constant<bool, true>{});
+    else scan(std::integral_constant<bool, false>{});
 }
 
 // The segment's forward from its parked state: vs, as after each of its n steps (and the state before)
-template <int LEVELS, bool SIGNED, bool ALIF>
-__device__ __forceinline__ void seg_replay(const float *x, int D, int t0, int n, float bt, float th0, float rho,
+// (FIN: as fwd1's; returns the largest |v|)
+template <int LEVELS, bool SIGNED, bool ALIF, bool FIN>
+__device__ __forceinline__ float seg_replay(const float *x, int D, int t0, int n, float bt, float th0, float rho,
                                            float omr, float gain, float v, float sp, float a, float (&vs)[SK],
                                            float (&as)[SK]) {
-    float thp = ALIF ? th0 + a * gain : th0;
+    float thp = ALIF ? th0 + a * gain : th0, top = 0.0f;
 #pragma unroll
     for (int i = 0; i < SK; i++) {
         if (i < n) {
-            fwd1<LEVELS, SIGNED, ALIF>(x[(size_t)(t0 + i) * D], bt, th0, rho, omr, gain, v, sp, a, thp);
+            fwd1<LEVELS, SIGNED, ALIF, FIN>(x[(size_t)(t0 + i) * D], bt, th0, rho, omr, gain, v, sp, a, thp);
             vs[i] = v;
             as[i] = a;
+            top = fmaxf(top, fabsf(v));
         }
     }
+    return top;
 }
 
 // an affine function of X = (Gn, cv, ca): c[0] + c[1] Gn + c[2] cv + c[3] ca
@@ -353,12 +408,10 @@ __device__ __forceinline__ Aff scal(float s, const Aff &x) {
     return r;
 }
 
-template <int LEVELS, bool SIGNED, bool ALIF>
-__global__ __launch_bounds__(256) void lif_seg_affine_kernel(LifSegArgs A) {
+template <int LEVELS, bool SIGNED, bool ALIF, bool FIN>
+__device__ __forceinline__ void seg_affine(const LifSegArgs &A, int gid) {
     const LifBwdArgs &p = A.p;
     const int chains = p.B * p.D;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;  // chain fastest
-    if (gid >= chains * A.nseg) return;
     const int sg = gid / chains, ch = gid - sg * chains;
     const int D = p.D, T = p.T, b = ch / D, c = ch - b * D;
     const float bt = p.ps[c], th0 = p.ps[D + c], rho = p.ps[2 * D + c], gain = p.ps[3 * D + c], omr = 1.0f - rho;
@@ -366,44 +419,61 @@ __global__ __launch_bounds__(256) void lif_seg_affine_kernel(LifSegArgs A) {
     const float *x = p.cur + (size_t)b * T * D + c, *g = p.gs + (size_t)b * T * D + c;
     const float pv = *park_at(A, sg, 0, ch), ps_ = *park_at(A, sg, 1, ch), pa = *park_at(A, sg, 2, ch);
     float vs[SK] = {}, as[SK] = {};
-    seg_replay<LEVELS, SIGNED, ALIF>(x, D, t0, n, bt, th0, rho, omr, gain, pv, ps_, pa, vs, as);
+    const float top = seg_replay<LEVELS, SIGNED, ALIF, FIN>(x, D, t0, n, bt, th0, rho, omr, gain, pv, ps_, pa, vs, as);
     Aff Gn{{0.0f, 1.0f, 0.0f, 0.0f}}, cv{{0.0f, 0.0f, 1.0f, 0.0f}}, ca{{0.0f, 0.0f, 0.0f, 1.0f}};
     Aff gb = aff(0.0f), gg = aff(0.0f), gr = aff(0.0f);
+    auto back = [&](auto near) {
+        constexpr bool NEAR = decltype(near)::value;
 #pragma unroll
-    for (int i = SK - 1; i >= 0; i--) {
-        if (i < n) {
-            const float vt = vs[i], at = ALIF ? as[i] : 0.0f;
-            const float tht = ALIF ? th0 + at * gain : th0;
-            float dv, dth;
-            dspike<LEVELS, SIGNED>(vt, tht, p.slope, dv, dth);
-            const float gt = g[(size_t)(t0 + i) * D];
-            float te = 0.0f;
-            if (p.rg) {
-                const float qq = tht * dv, cap = 2.0f * bt;
-                te = qq > cap ? cap / dv : tht;
+        for (int i = SK - 1; i >= 0; i--) {
+            if (i < n) {
+                const float vt = vs[i], at = ALIF ? as[i] : 0.0f;
+                const float tht = ALIF ? th0 + at * gain : th0;
+                float dv, dth;
+                dspike<LEVELS, SIGNED, NEAR>(vt, tht, p.slope, dv, dth);
+                const float gt = g[(size_t)(t0 + i) * D];
+                float te = 0.0f;
+                if (p.rg) {
+                    const float qq = tht * dv, cap = 2.0f * bt;
+                    te = qq > cap ? cap / dv : tht;
+                }
+                const Aff gst = axpy(-te, Gn, aff(gt));   // g - te Gn
+                const Aff G = axpy(dv, gst, cv);          // gst dv + cv
+                gb = axpy(i > 0 ? vs[i - 1] : pv, G, gb);
+                if (ALIF) {
+                    Aff gth = scal(dth, gst);
+                    if (p.rg) gth = axpy(-spike<LEVELS, SIGNED, FIN>(vt, tht), Gn, gth);
+                    const Aff gaa = axpy(gain, gth, ca);
+                    gg = axpy(at, gth, gg);
+                    const float ap = i > 0 ? as[i - 1] : pa;
+                    const float sprev = i > 0 ? spike<LEVELS, SIGNED, FIN>(vs[i - 1], th0 + as[i - 1] * gain) : ps_;
+                    gr = axpy(ap - fabsf(sprev), gaa, gr);
+                    ca = scal(rho, gaa);
+                }
+                Gn = G;
+                cv = scal(bt, G);
             }
-            const Aff gst = axpy(-te, Gn, aff(gt));   // g - te Gn
-            const Aff G = axpy(dv, gst, cv);          // gst dv + cv
-            gb = axpy(i > 0 ? vs[i - 1] : pv, G, gb);
-            if (ALIF) {
-                Aff gth = scal(dth, gst);
-                if (p.rg) gth = axpy(-spike_of<LEVELS, SIGNED>(vt, tht), Gn, gth);
-                const Aff gaa = axpy(gain, gth, ca);
-                gg = axpy(at, gth, gg);
-                const float ap = i > 0 ? as[i - 1] : pa;
-                const float sprev = i > 0 ? spike_of<LEVELS, SIGNED>(vs[i - 1], th0 + as[i - 1] * gain) : ps_;
-                gr = axpy(ap - fabsf(sprev), gaa, gr);
-                ca = scal(rho, gaa);
-            }
-            Gn = G;
-            cv = scal(bt, G);
         }
-    }
+    };
+    if (FIN && __all(top < NEAR_V)) back(std::integral_constant<bool, true>{});
+    else back(std::integral_constant<bool, false>{});
     const Aff *out[6] = {&Gn, &cv, &ca, &gb, &gg, &gr};
 #pragma unroll
     for (int f = 0; f < 6; f++)
 #pragma unroll
         for (int i = 0; i < 4; i++) *ws_at(A, sg, 4 * f + i, ch) = out[f]->c[i];
+}
+
+template <int LEVELS, bool SIGNED, bool ALIF>
+__global__ __launch_bounds__(256) void lif_seg_affine_kernel(LifSegArgs A) {
+    const LifBwdArgs &p = A.p;
+    const int chains = p.B * p.D, gid = blockIdx.x * blockDim.x + threadIdx.x;  // chain fastest
+    const bool in = gid < chains * A.nseg;
+    const int ch = in ? gid % chains : 0;
+    const bool fin = wave_tame<ALIF>(p, ch % p.D, ch);
+    if (!in) return;
+    if (fin) seg_affine<LEVELS, SIGNED, ALIF, true>(A, gid);
+    else seg_affine<LEVELS, SIGNED, ALIF, false>(A, gid);
 }
 
 __device__ __forceinline__ float apply_aff(const LifSegArgs &A, int sg, int f, int ch, float Gn, float cv, float ca) {
@@ -448,12 +518,10 @@ __global__ __launch_bounds__(256) void lif_seg_carry_kernel(LifSegArgs A) {
     if (p.dgain) p.dgain[gid] = ALIF ? gg : 0.0f;
 }
 
-template <int LEVELS, bool SIGNED, bool ALIF>
-__global__ __launch_bounds__(256) void lif_seg_walk_kernel(LifSegArgs A) {
+template <int LEVELS, bool SIGNED, bool ALIF, bool FIN>
+__device__ __forceinline__ void seg_walk(const LifSegArgs &A, int gid) {
     const LifBwdArgs &p = A.p;
     const int chains = p.B * p.D;
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= chains * A.nseg) return;
     const int sg = gid / chains, ch = gid - sg * chains;
     const int D = p.D, T = p.T, b = ch / D, c = ch - b * D;
     const float bt = p.ps[c], th0 = p.ps[D + c], rho = p.ps[2 * D + c], gain = p.ps[3 * D + c], omr = 1.0f - rho;
@@ -463,30 +531,47 @@ __global__ __launch_bounds__(256) void lif_seg_walk_kernel(LifSegArgs A) {
     const float pv = *park_at(A, sg, 0, ch), ps_ = *park_at(A, sg, 1, ch), pa = *park_at(A, sg, 2, ch);
     float Gn = *ws_at(A, sg, 24, ch), cv = *ws_at(A, sg, 25, ch), ca = *ws_at(A, sg, 26, ch);
     float vs[SK] = {}, as[SK] = {};
-    seg_replay<LEVELS, SIGNED, ALIF>(x, D, t0, n, bt, th0, rho, omr, gain, pv, ps_, pa, vs, as);
+    const float top = seg_replay<LEVELS, SIGNED, ALIF, FIN>(x, D, t0, n, bt, th0, rho, omr, gain, pv, ps_, pa, vs, as);
+    auto back = [&](auto near) {
+        constexpr bool NEAR = decltype(near)::value;
 #pragma unroll
-    for (int i = SK - 1; i >= 0; i--) {
-        if (i < n) {
-            const float vt = vs[i], at = ALIF ? as[i] : 0.0f;
-            const float tht = ALIF ? th0 + at * gain : th0;
-            float dv, dth;
-            dspike<LEVELS, SIGNED>(vt, tht, p.slope, dv, dth);
-            float gst = g[(size_t)(t0 + i) * D];
-            if (p.rg) {
-                const float qq = tht * dv, cap = 2.0f * bt;
-                gst -= (qq > cap ? cap / dv : tht) * Gn;
+        for (int i = SK - 1; i >= 0; i--) {
+            if (i < n) {
+                const float vt = vs[i], at = ALIF ? as[i] : 0.0f;
+                const float tht = ALIF ? th0 + at * gain : th0;
+                float dv, dth;
+                dspike<LEVELS, SIGNED, NEAR>(vt, tht, p.slope, dv, dth);
+                float gst = g[(size_t)(t0 + i) * D];
+                if (p.rg) {
+                    const float qq = tht * dv, cap = 2.0f * bt;
+                    gst -= (qq > cap ? cap / dv : tht) * Gn;
+                }
+                const float G = gst * dv + cv;
+                if (ALIF) {
+                    float gth = gst * dth;
+                    if (p.rg) gth -= spike<LEVELS, SIGNED, FIN>(vt, tht) * Gn;
+                    ca = rho * (gth * gain + ca);
+                }
+                o[(size_t)(t0 + i) * D] = G;
+                Gn = G;
+                cv = bt * G;
             }
-            const float G = gst * dv + cv;
-            if (ALIF) {
-                float gth = gst * dth;
-                if (p.rg) gth -= spike_of<LEVELS, SIGNED>(vt, tht) * Gn;
-                ca = rho * (gth * gain + ca);
-            }
-            o[(size_t)(t0 + i) * D] = G;
-            Gn = G;
-            cv = bt * G;
         }
-    }
+    };
+    if (FIN && __all(top < NEAR_V)) back(std::integral_constant<bool, true>{});
+    else back(std::integral_constant<bool, false>{});
+}
+
+template <int LEVELS, bool SIGNED, bool ALIF>
+__global__ __launch_bounds__(256) void lif_seg_walk_kernel(LifSegArgs A) {
+    const LifBwdArgs &p = A.p;
+    const int chains = p.B * p.D, gid = blockIdx.x * blockDim.x + threadIdx.x;  // chain fastest
+    const bool in = gid < chains * A.nseg;
+    const int ch = in ? gid % chains : 0;
+    const bool fin = wave_tame<ALIF>(p, ch % p.D, ch);
+    if (!in) return;
+    if (fin) seg_walk<LEVELS, SIGNED, ALIF, true>(A, gid);
+    else seg_walk<LEVELS, SIGNED, ALIF, false>(A, gid);
 }
 
 template <int LEVELS, bool SIGNED, bool ALIF>

@@ -71,6 +71,33 @@ def test_lif_bwd(T, levels, signed, alif, rg, D):
         assert np.array_equal(gpu[k], o[k]), (k, rel(gpu[k], o[k]))
 
 
+@pytest.mark.parametrize("rg", [False, True])
+def test_lif_bwd_large_values(rg):
+    """Membranes past the range of the short reciprocal (1e9) in single segments and lanes, thresholds and traces past
+    the counted spikes' (third wave; its theta 1e9, rho above 1), slopes on both sides of 1e6: the oracle's bits from
+    the one-lane walk, and the segments' form within its usual rounding."""
+    B, T, D = 2, 70, 192
+    for slope in (2.0, 3e6):
+        x = list(lif_inputs(31 + rg, B, T, D, 2, True))
+        x[0][0, 20, 3] = 4e9
+        x[0][1, 40, 70:80] = -7e11
+        x[1][D + 130] = 1e9  # theta
+        x[1][2 * D + 140] = 1.25  # rho
+        o = O.lif_bwd(x[0], x[1], x[5], x[2], x[3], x[4], x[6], x[7], levels=2, signed=True, alif=True, slope=slope,
+                      reset_grad=rg)
+        gpu = run_lif(*x, 2, True, True, slope, rg)
+        from ava_amd import ops
+        st = ops.LifState(dev(x[2]), dev(x[3]), dev(x[4]))
+        seg = ops.lif_gen_bwd(dev(x[0]), dev(x[1]), dev(x[5]), init=st, g_vT=dev(x[6]), g_aT=dev(x[7]), slope=slope,
+                              reset_grad=rg, segments=True)
+        for k in ("dI", "dv0", "dbeta", "da0", "drho", "dgain"):
+            assert np.array_equal(gpu[k], o[k], equal_nan=True), (slope, k, rel(gpu[k], o[k]))
+            # per value: the walk's own rounding over 70 steps (a few ulp each), relative to the largest of its chain
+            d = np.abs(host(seg[k]) - o[k])
+            top = np.max(np.abs(o[k]), axis=1, keepdims=True) if k == "dI" else np.abs(o[k]) + 1e-3 * np.max(np.abs(o[k]))
+            assert np.all(d <= 1e-4 * top + 1e-30), (slope, k, float(np.max(d / (top + 1e-30))))
+
+
 def test_lif_bwd_long():
     """config[1]'s sequence length and width (T 2048, D 2048) on 8 streams, int2 with ALIF and the
     reset gradient."""
