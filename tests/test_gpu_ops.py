@@ -198,6 +198,24 @@ def test_quant_rows_matches_oracle(planes, dev):
     assert not xq[:, :, 200:].any()
 
 
+# a row of one and of four waves, whole and ragged, of no multiple of 4 (4-byte loads), longer than a workgroup holds
+@pytest.mark.parametrize("k", [3, 64, 512, 513, 1024, 1028, 4093, 4096, 4100, 8192])
+@pytest.mark.parametrize("planes", [1, 3])
+def test_quant_rows_widths_match_oracle(k, planes, dev):
+    rng = np.random.default_rng(k)
+    m = 13
+    x = (rng.standard_normal((m, k)) * np.exp(rng.standard_normal((m, 1)) * 3)).astype(np.float32)
+    x[5] = 0.0
+    x[6, k - 1] = 300.0  # the largest value in the row's tail
+    xq_o, xe_o = O.quant_planes(x, planes)
+    from ava_amd import ops
+    xq, xe = ops.quant_rows(cuda(x), planes)
+    xq, xe = host(xq), host(xe)
+    assert np.array_equal(xe, xe_o)
+    assert np.array_equal(xq[:, :, :k], xq_o)
+    assert not xq[:, :, k:].any()
+
+
 @pytest.mark.parametrize("din,dout,m", SHAPES)
 def test_q8_accumulators_bit_exact(din, dout, m, dev):
     rng = np.random.default_rng(din * 7 + m)
