@@ -419,7 +419,9 @@ __device__ inline BufRes8 buf_res8(const int8_t *base, unsigned) { return base; 
 // issued before the MFMAs of the current group, so four MFMAs cover their LDS latency (the order is
 // fixed with sched_group_barrier). A tile's first step multiplies into zero accumulators (no
 // register clearing).
-constexpr int GEMM_BM = 128, GEMM_BN = 256, GEMM_WM = 2, GEMM_WN = 4, GEMM_ILV = 2;
+// Products too small to give every CU such a tile (a prefill of a few thousand rows) take 128 x 128 (8 waves of 64 x
+// 32) or 64 x 128 tiles (32 x 32 a wave, 80 KB: two workgroups share a CU), see launch_gemm. The bits are the same.
+constexpr int GEMM_WM = 2, GEMM_WN = 4, GEMM_ILV = 2;
 
 __device__ __forceinline__ void dma16_buf(BufRes8 r, unsigned voff, unsigned soff, void *l) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -445,12 +447,12 @@ __device__ __forceinline__ void frag_schedule() {
     }
 }
 
-template <int P, int EPI, int BK, int CMB>
-__global__ __launch_bounds__(64 * GEMM_WM * GEMM_WN, 1) void q8_gemm_kernel(const int8_t *__restrict__ xq,
+template <int P, int EPI, int BK, int CMB, int BM, int BN>
+__global__ __launch_bounds__(64 * GEMM_WM * GEMM_WN, BM * BN < 16384 ? 4 : 1) void q8_gemm_kernel(const int8_t *__restrict__ xq,
                                                                         const int32_t *__restrict__ xexp, int m,
                                                                         int n, int ldk, const int8_t *__restrict__ qt,
                                                                         const float *__restrict__ scale, EpiArgs ep) {
-    constexpr int BM = GEMM_BM, BN = GEMM_BN, WM = GEMM_WM, WN = GEMM_WN, NWAVE = WM * WN, NT = 64 * NWAVE;
+    constexpr int WM = GEMM_WM, WN = GEMM_WN, NWAVE = WM * WN, NT = 64 * NWAVE;
     constexpr int CPR = BK / 16, RPI = 1024 / BK, KS = BK / 32;
     static_assert(BK == 64 || BK == 128, "K step");
     constexpr int MW = BM / WM, NW = BN / WN, FM = MW / 32, FN = NW / 32;
@@ -502,7 +504,7 @@ __global__ __launch_bounds__(64 * GEMM_WM * GEMM_WN, 1) void q8_gemm_kernel(cons
     // order and holds at most 63, so an instruction issued with 63 older ones outstanding waits for
     // the oldest: the first-step loads had then landed before the last of those was issued, and the
     // first step needs no wait (which would also wait for the epilogue's stores to reach L2).
-    static_assert(FM * FN * 16 >= 63, "an interior epilogue issues at least 63 stores per wave");
+    constexpr bool STORES_COVER = FM * FN * 16 >= 63;  // (smaller tiles wait)
     bool loaded = false;
     // the row exponents through a resource of 0 bytes when there are none: its loads read 0, so the
     // load needs no branch (a branch would make the compiler wait for the value at its join)
@@ -530,7 +532,7 @@ __global__ __launch_bounds__(64 * GEMM_WM * GEMM_WN, 1) void q8_gemm_kernel(cons
         auto step = [&](auto first, int kt) {
             constexpr bool FIRST = decltype(first)::value;
             st = (sbase + kt) & 1;
-            if (FIRST && loaded) wait_vm<63>();  // holds by itself: see `loaded`
+            if (STORES_COVER && FIRST && loaded) wait_vm<63>();  // holds by itself: see `loaded`
             else wait_vm<0>();  // this wave's loads of step kt (and the previous tile's stores) are done
             __builtin_amdgcn_s_barrier();  // every wave's are; every wave is done with the other stage
             int knext = kt + 1;
@@ -920,13 +922,14 @@ int gemm_grid(int tiles, int *grid) {
     return AVA_OK;
 }
 
-template <int P, int EPI, int BK>
+template <int P, int EPI, int BK, int BM, int BN>
 int launch_tiled(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk, const int8_t *qt, const float *scale,
                  EpiArgs ep, hipStream_t st) {
-    const int tiles = ((m + GEMM_BM - 1) / GEMM_BM) * ((n + GEMM_BN - 1) / GEMM_BN);
+    const int tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
     int grid = 0;
-    if (int r = gemm_grid(tiles, &grid)) return r;
-    const size_t lds = (size_t)2 * (P * GEMM_BM + GEMM_BN) * BK;
+    if (int r = gemm_grid(BM * BN < 16384 ? (tiles + 1) / 2 : tiles, &grid)) return r;
+    if (BM * BN < 16384) grid = std::min(2 * grid, tiles);  // two workgroups a CU
+    const size_t lds = (size_t)2 * (P * BM + BN) * BK;
     auto go = [&](auto kern) -> int {
         if (int r = ava::lds_opt_in((const void *)kern, lds)) return r;
         kern<<<dim3(grid), dim3(64 * GEMM_WM * GEMM_WN), lds, st>>>(xq, xexp, m, n, ldk, qt, scale, ep);
@@ -935,11 +938,11 @@ int launch_tiled(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk, c
     };
     // the int32 plane combine holds for K <= 1024; spike products have no row exponents (see epilogue)
     if constexpr (P == 1) {
-        if (EPI != EPI_ACC && !xexp) return go(q8_gemm_kernel<P, EPI, BK, CMB_NOEXP>);
+        if (EPI != EPI_ACC && !xexp) return go(q8_gemm_kernel<P, EPI, BK, CMB_NOEXP, BM, BN>);
     } else {
-        if (EPI != EPI_ACC && ldk <= 1024) return go(q8_gemm_kernel<P, EPI, BK, CMB_I32>);
+        if (EPI != EPI_ACC && ldk <= 1024) return go(q8_gemm_kernel<P, EPI, BK, CMB_I32, BM, BN>);
     }
-    return go(q8_gemm_kernel<P, EPI, BK, CMB_F64>);
+    return go(q8_gemm_kernel<P, EPI, BK, CMB_F64, BM, BN>);
 }
 
 template <int P, int EPI>
@@ -949,7 +952,19 @@ int launch_gemm(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk, co
     if (m <= SMALL_ROWS) return launch_small<P, EPI>(xq, xexp, m, n, ldk, qt, scale, ep, st);
     // 128-byte K steps (whole cache lines per load request) for every plane count: for the single
     // spike plane at 131,072 x 1024 x 1024 they measured 279 us against 340 us for 64-byte steps
-    return launch_tiled<P, EPI, 128>(xq, xexp, m, n, ldk, qt, scale, ep, st);
+    if constexpr (P != 2 && EPI != EPI_ACC) {
+        // The tile with the least rounds over the CUs, each weighed by its time on a full chip (128 x 256: 1).
+        int cus = 0;
+        if (int r = ava::device_cus(&cus)) return r;
+        auto rounds = [&](int bm, int bn) {
+            return (double)((((long)(m + bm - 1) / bm) * ((n + bn - 1) / bn) + cus - 1) / cus);
+        };
+        const double big = rounds(128, 256), mid = rounds(128, 128) * 0.56, small = rounds(64, 128) * 0.32;
+        if (small < big && small <= mid)
+            return launch_tiled<P, EPI, 128, 64, 128>(xq, xexp, m, n, ldk, qt, scale, ep, st);
+        if (mid < big) return launch_tiled<P, EPI, 128, 128, 128>(xq, xexp, m, n, ldk, qt, scale, ep, st);
+    }
+    return launch_tiled<P, EPI, 128, 128, 256>(xq, xexp, m, n, ldk, qt, scale, ep, st);
 }
 
 template <int EPI>
