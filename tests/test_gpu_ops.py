@@ -296,6 +296,42 @@ def test_q8_epilogues_scale_and_accumulate_bit_exact(din, dout, m, kind, dev):
     assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32))
 
 
+# (m, dout) that take each tile of a product of more than 512 rows: 128 x 256, 128 x 128 and 64 x 128, with ragged last
+# tiles both ways; K up to 1024 and beyond combine the planes differently
+@pytest.mark.parametrize("din,dout,m", [(200, 1000, 8100), (200, 1020, 4090), (1100, 1020, 3970), (200, 130, 513),
+                                        (1100, 390, 1000)])
+@pytest.mark.parametrize("kind", [1, 2, 3])
+def test_q8_tiles_bit_exact(din, dout, m, kind, dev):
+    import ctypes as C
+    import torch
+    from ava_amd import ops, _lib
+    f = getattr(_lib.lib(), "_ZN3ava7q8_gemmEPKaPKiiiPK6ava_qwiPfiPKfP12ihipStream_t")
+    f.restype = C.c_int
+    f.argtypes = [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p,
+                  C.c_void_p]
+    rng = np.random.default_rng(din + dout + m + kind)
+    w = (rng.standard_normal((din, dout)) * 0.02).astype(np.float32)
+    x = (rng.standard_normal((m, din)) * np.exp2(rng.integers(-8, 8, (m, 1)))).astype(np.float32)
+    spk = rng.integers(-2, 3, (m, din)).astype(np.int8)
+    y0 = rng.standard_normal((m, dout)).astype(np.float32)
+    cv = rng.uniform(0.5, 2.0, dout).astype(np.float32)
+    q_o, s_o = O.quantize_int8(w)
+    qw = ops.QW.from_tensor(cuda(w))
+    xq, xe = ops.quant_rows(cuda(x), 3)
+    sp = np.zeros((m, qw.ldk), np.int8)
+    sp[:, :din] = spk
+    sp = cuda(sp)
+    for planes, a, e in ((3, xq, xe.data_ptr()), (1, sp, None)):
+        v = (O.q8_matmul_planes(x, 3, q_o, s_o) if planes == 3 else
+             (spk.astype(np.float32) @ q_o.astype(np.float32)) * s_o)  # whole numbers below 2^24: exact in any order
+        want = {1: v, 2: v * cv, 3: y0 + v}[kind].astype(np.float32)
+        y, colv = cuda(y0), cuda(cv)
+        rc = f(a.data_ptr(), e, planes, m, C.addressof(qw.c), kind, y.data_ptr(), dout, colv.data_ptr(),
+               torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32)), planes
+
+
 @pytest.mark.parametrize("din,dout,m", SHAPES)
 def test_q8_spike_product_is_the_reference_bits(din, dout, m, dev):
     """Integer inputs: the i8 MFMA product equals the reference's f32 fma chain bit for bit."""
