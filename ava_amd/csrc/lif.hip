@@ -171,8 +171,10 @@ __device__ __forceinline__ bool finite_thresholds(float th0, float rho, float ga
 // end of its block (PF = LIF_SEG_STEPS). The same arithmetic as lif_scan_kernel, so the same bits. With up to one
 // wave per SIMD (65,536 chains) a step's time is its VALU operations at 8 cycles each, so waves whose thresholds
 // stay finite count spikes by lif_count: 20 operations a step instead of 27, 64 x 2048 x 1024 158 us instead of 202,
-// 4 x 2048 x 1024 146 instead of 176; 64 x 2048 x 2048 247 instead of 258, bound by HBM (5.4 TB/s).
-template <int PF, int LEVELS, bool SIGNED, bool ALIF>
+// 4 x 2048 x 1024 146 instead of 176. Past 114,688 chains and 2e8 elements HBM bounds the scan, and the counted form,
+// whose waves drift further apart, streams worse (into alternating outputs, T = 2048: 48 x 2048 channels 214 us counted,
+// 240 by differences; 56 253 / 256; 60 269 / 266; 64 295 / 281, 4.8 TB/s): COUNT is off there.
+template <int PF, int LEVELS, bool SIGNED, bool ALIF, bool COUNT>
 __global__ __launch_bounds__(256) void lif_scan_buf_kernel(const float *__restrict__ cur, int B, int T, int D,
                                                            const float *__restrict__ ps, float *__restrict__ v,
                                                            float *__restrict__ s, float *__restrict__ a,
@@ -247,7 +249,7 @@ __global__ __launch_bounds__(256) void lif_scan_buf_kernel(const float *__restri
         }
         for (int t = full * PF; t < T; t++) step(buf[t - full * PF], (unsigned)t);
     };
-    if (__all(finite_thresholds(th0, ALIF ? rho : 0.0f, ALIF ? gain : 0.0f, ALIF ? aa : 0.0f, sp)))
+    if (COUNT && __all(finite_thresholds(th0, ALIF ? rho : 0.0f, ALIF ? gain : 0.0f, ALIF ? aa : 0.0f, sp)))
         scan(std::integral_constant<bool, true>{});
     else
         scan(std::integral_constant<bool, false>{});
@@ -267,11 +269,15 @@ int launch_vp(const float *cur, int B, int T, int D, const float *ps, float *v, 
     dim3 grid(ava::ceil_div(threads, 256)), block(256);
     // the buffer form: whole waves per stream, and every offset of a stream's slab in 32 bits
     const bool bufd = VEC == 1 && PF == ava::LIF_SEG_STEPS && D % 64 == 0 && (long)T * D * 4 < (1L << 31);
+    const bool count = (long)B * D <= 114688 || (long)B * T * D <= 200000000L;  // see lif_scan_buf_kernel
 #define AVA_LIF_GO(L, S, A)                                                                                         \
     do {                                                                                                            \
-        if (bufd)                                                                                                   \
-            lif_scan_buf_kernel<PF, L, S, A><<<grid, block, 0, st>>>(cur, B, T, D, ps, v, s, a, spikes, th_out,    \
-                                                                     park);                                         \
+        if (bufd && count)                                                                                          \
+            lif_scan_buf_kernel<PF, L, S, A, true><<<grid, block, 0, st>>>(cur, B, T, D, ps, v, s, a, spikes,      \
+                                                                           th_out, park);                           \
+        else if (bufd)                                                                                              \
+            lif_scan_buf_kernel<PF, L, S, A, false><<<grid, block, 0, st>>>(cur, B, T, D, ps, v, s, a, spikes,     \
+                                                                            th_out, park);                          \
         else                                                                                                        \
             lif_scan_kernel<VEC, PF, L, S, A><<<grid, block, 0, st>>>(cur, B, T, D, ps, v, s, a, spikes, th_out,   \
                                                                       park);                                        \
