@@ -7,6 +7,8 @@ from __future__ import annotations
 import ctypes as C
 import os
 
+import torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libava_amd.so")
 
@@ -151,6 +153,12 @@ def lib():
         L.ava_model_timing.restype = i32
     _lib = L
     return L
+
+
+def current_stream():
+    """The current device's current torch stream as a hipStream_t (an int). torch.cuda.current_stream() builds a
+    Stream object, 2.9 us of a 9 us call; the raw handle takes 0.1."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 class AvaError(RuntimeError):

@@ -19,7 +19,7 @@ import ctypes as C
 import numpy as np
 import torch
 
-from ._lib import BLOCK_FIELDS, BlockParams, Params, State as _CState, check, config_struct, lib
+from ._lib import BLOCK_FIELDS, BlockParams, Params, State as _CState, check, config_struct, current_stream, lib
 
 # The end-of-text id of the reference's byte-pair vocabulary (ava_data::bpe::EOS, data/src/bpe.rs:57),
 # at which its generate ends a row (gpu/state.rs:1402, 1436).
@@ -93,7 +93,7 @@ class State:
             raise ValueError("evict: the store must be on the GPU (ava_engram_evict runs there)")
         p = lambda t: C.c_void_p(t.data_ptr()) if t is not None else None
         rule = 1 if self.eng_rule == "least-read" else 0
-        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = current_stream()
         check(lib().ava_engram_evict(p(self.eng_k), p(self.eng_v), p(self.eng_reads), p(self.eng_age), self.B,
                                      self.eng_cap, n, p(self.eng_len_dev), self.eng_k.shape[2],
                                      int(self.eng_k.dtype == torch.float16), mx, rule, stream), "ava_engram_evict")
@@ -208,7 +208,7 @@ class Model:
         if want_logits and logits is None:
             logits = torch.empty((B * T, self.cfg["vocab"]), dtype=torch.float32, device=ids.device)
         cst = st.c()
-        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = current_stream()
         check(lib().ava_model_forward(self.h, C.byref(cst), C.c_void_p(ids.data_ptr()), B, T,
                                       C.c_void_p(logits.data_ptr()) if want_logits else None, stream),
               "ava_model_forward")
@@ -251,7 +251,7 @@ class Model:
             pz = C.c_void_p(prev_nats.data_ptr()) if prev_nats is not None else None
             ld = prev_logits.stride(0)
         cst = st.c()
-        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = current_stream()
         check(lib().ava_model_decode_step(self.h, C.byref(cst), C.c_void_p(ids.data_ptr()), B, T,
                                           C.c_void_p(logits.data_ptr()), pl, ld, pn, pz, stream),
               "ava_model_decode_step")
@@ -292,7 +292,7 @@ class Model:
         elif not (nats.is_cuda and nats.dtype == torch.float64 and nats.numel() >= B and nats.is_contiguous()):
             raise ValueError("nats: a contiguous f64 GPU tensor of >= B entries is required")
         cst = st.c()
-        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = current_stream()
         check(lib().ava_model_cb_learn(self.h, C.byref(cst), C.c_void_p(logits.data_ptr()), logits.stride(0),
                                        C.c_void_p(nxt.data_ptr()), B, C.c_void_p(nats.data_ptr()), stream),
               "ava_model_cb_learn")
@@ -391,7 +391,7 @@ class Model:
         fast weights were left as they were; gpu/model/fstep/arch.rs:780-783's guard). Waits for the
         current stream."""
         n = C.c_int(0)
-        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = current_stream()
         B = getattr(self, "_last_B", 0)
         rows = (C.c_int32 * max(B, 1))()
         check(lib().ava_model_nonfinite(self.h, rows, max(B, 1), C.byref(n), stream), "ava_model_nonfinite")

@@ -27,11 +27,7 @@ from dataclasses import dataclass
 
 import torch
 
-from ._lib import QW as _QWC, check, lib
-
-
-def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+from ._lib import QW as _QWC, check, current_stream, lib
 
 
 def _p(t):
@@ -65,7 +61,7 @@ class QW:
         din, dout = w.shape
         qt = torch.empty((dout, ldk(din)), dtype=torch.int8, device=w.device)
         scale = torch.empty(dout, dtype=torch.float32, device=w.device)
-        check(lib().ava_q8_pack(_p(w), din, dout, _p(qt), _p(scale), _stream()), "ava_q8_pack")
+        check(lib().ava_q8_pack(_p(w), din, dout, _p(qt), _p(scale), current_stream()), "ava_q8_pack")
         return QW(din, dout, qt, scale)
 
 
@@ -74,7 +70,7 @@ def quant_rows(x: torch.Tensor, planes: int = 3):
     m, k = x.shape
     xq = torch.empty((planes, m, ldk(k)), dtype=torch.int8, device=x.device)
     xe = torch.empty(m, dtype=torch.int32, device=x.device)
-    check(lib().ava_q8_quant_rows(_p(x), m, k, planes, _p(xq), _p(xe), _stream()), "ava_q8_quant_rows")
+    check(lib().ava_q8_quant_rows(_p(x), m, k, planes, _p(xq), _p(xe), current_stream()), "ava_q8_quant_rows")
     return xq, xe
 
 
@@ -82,7 +78,7 @@ def gemm_acc(xq: torch.Tensor, w: QW):
     _need(xq, torch.int8, "gemm_acc")
     planes, m, _ = xq.shape
     acc = torch.empty((planes, m, w.dout), dtype=torch.int32, device=xq.device)
-    check(lib().ava_q8_gemm_acc(_p(xq), planes, m, C.byref(w.c), _p(acc), _stream()), "ava_q8_gemm_acc")
+    check(lib().ava_q8_gemm_acc(_p(xq), planes, m, C.byref(w.c), _p(acc), current_stream()), "ava_q8_gemm_acc")
     return acc
 
 
@@ -94,7 +90,7 @@ def mm(x: torch.Tensor, w: QW, planes: int = 3) -> torch.Tensor:
     y = torch.empty((m, w.dout), dtype=torch.float32, device=x.device)
     nbytes = lib().ava_q8_workspace(m, k, planes)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-    check(lib().ava_q8_matmul(_p(x), m, C.byref(w.c), planes, _p(y), _p(ws), nbytes, _stream()), "ava_q8_matmul")
+    check(lib().ava_q8_matmul(_p(x), m, C.byref(w.c), planes, _p(y), _p(ws), nbytes, current_stream()), "ava_q8_matmul")
     return y
 
 
@@ -105,7 +101,7 @@ def mm_spikes(s: torch.Tensor, w: QW) -> torch.Tensor:
     if k != w.ldk:
         raise ValueError(f"mm_spikes: input width {k}, expected ldk {w.ldk}")
     y = torch.empty((m, w.dout), dtype=torch.float32, device=s.device)
-    check(lib().ava_q8_matmul_i8(_p(s), m, C.byref(w.c), _p(y), _stream()), "ava_q8_matmul_i8")
+    check(lib().ava_q8_matmul_i8(_p(s), m, C.byref(w.c), _p(y), current_stream()), "ava_q8_matmul_i8")
     return y
 
 
@@ -138,7 +134,7 @@ def lif_gen(cur, beta, theta=None, alif=None, levels=2, signed=True, init=None, 
     spikes = torch.empty((B, T, D), dtype=torch.int8, device=dev)
     tho = torch.empty((B, D), dtype=torch.float32, device=dev) if th_out else None
     rc = lib().ava_lif_scan(_p(cur), B, T, D, _p(ps), _p(v), _p(s), _p(a), levels, int(signed),
-                            int(alif is not None), _p(spikes), _p(tho), _stream())
+                            int(alif is not None), _p(spikes), _p(tho), current_stream())
     check(rc, "ava_lif_scan")
     st = LifState(v, s, a)
     return (spikes, st, tho) if th_out else (spikes, st)
@@ -150,7 +146,7 @@ def kwta_relu(u: torch.Tensor, k: int, relu2: bool = True):
     n, h = u.shape
     a = torch.empty_like(u)
     kth = torch.empty(n, dtype=torch.float32, device=u.device)
-    check(lib().ava_kwta(_p(u), n, h, k, int(relu2), _p(a), _p(kth), _stream()), "ava_kwta")
+    check(lib().ava_kwta(_p(u), n, h, k, int(relu2), _p(a), _p(kth), current_stream()), "ava_kwta")
     return a, kth
 
 
@@ -165,7 +161,7 @@ def mem_gen(q, k, e, v, la, b, m=0.0, cap=1e5, F=None, S=None):
     S = torch.zeros((BH, hs, hs), dtype=torch.float32, device=q.device) if S is None else S.clone()
     y = torch.empty_like(q)
     check(lib().ava_mem_scan(_p(q), _p(k), _p(e), _p(v), _p(la), _p(b), BH, T, hs, g, float(m), float(cap),
-                             _p(F), _p(S), _p(y), _stream()), "ava_mem_scan")
+                             _p(F), _p(S), _p(y), current_stream()), "ava_mem_scan")
     return y, F, S
 
 
@@ -180,7 +176,7 @@ def mem_chunk(q, k, e, v, la, b, m=0.0, cap=1e5, F=None, S=None):
     S = torch.zeros((BH, hs, hs), dtype=torch.float32, device=q.device) if S is None else S.clone()
     y = torch.empty_like(q)
     check(lib().ava_mem_chunk(_p(q), _p(k), _p(e), _p(v), _p(la), _p(b), BH, T, hs, g, float(m), float(cap),
-                              _p(F), _p(S), _p(y), _stream()), "ava_mem_chunk")
+                              _p(F), _p(S), _p(y), current_stream()), "ava_mem_chunk")
     return y, F, S
 
 
@@ -196,7 +192,7 @@ def delta_rule_from(q, k, v, beta, la=None, f0=None, workspace=True):
     nb = lib().ava_delta_chunk_workspace(BH, T) if (la is None and workspace) else 0
     work = torch.empty(nb, dtype=torch.uint8, device=q.device) if nb else None
     check(lib().ava_delta_chunk(_p(q), _p(k), _p(v), _p(la), _p(beta), BH, T, hs, _p(F), _p(y), _p(work), nb,
-                                _stream()), "ava_delta_chunk")
+                                current_stream()), "ava_delta_chunk")
     return y, F
 
 
@@ -225,12 +221,12 @@ def lif_gen_bwd(cur, ps, g_spk, init=None, g_vT=None, g_aT=None, levels=2, signe
                                               int(alif), float(slope), int(reset_grad), _p(g_spk), _p(g_vT),
                                               _p(g_aT), _p(out["dI"]), _p(out["dv0"]), _p(out["da0"]),
                                               _p(out["dbeta"]), _p(out["drho"]), _p(out["dgain"]), _p(ws), nb,
-                                              _stream()), "ava_lif_scan_bwd_segments")
+                                              current_stream()), "ava_lif_scan_bwd_segments")
         return out
     check(lib().ava_lif_scan_bwd(_p(cur), B, T, D, _p(ps), _p(v0), _p(s0), _p(a0), levels, int(signed), int(alif),
                                  float(slope), int(reset_grad), _p(g_spk), _p(g_vT), _p(g_aT), _p(out["dI"]),
                                  _p(out["dv0"]), _p(out["da0"]), _p(out["dbeta"]), _p(out["drho"]),
-                                 _p(out["dgain"]), _stream()), "ava_lif_scan_bwd")
+                                 _p(out["dgain"]), current_stream()), "ava_lif_scan_bwd")
     return out
 
 
@@ -241,7 +237,7 @@ def kwta_relu2_bwd(u, kth, ga):
     _need(kth, torch.float32, "kwta_relu2_bwd kth")
     n, h = u.shape
     gu = torch.empty_like(u)
-    check(lib().ava_kwta_relu2_bwd(_p(u), _p(kth), n, h, _p(ga), _p(gu), _stream()), "ava_kwta_relu2_bwd")
+    check(lib().ava_kwta_relu2_bwd(_p(u), _p(kth), n, h, _p(ga), _p(gu), current_stream()), "ava_kwta_relu2_bwd")
     return gu
 
 
@@ -263,7 +259,7 @@ def mem_gen_bwd(q, k, e, v, la, b, dy, m=0.0, cap=1e5, F0=None, S0=None, dF_T=No
     check(lib().ava_mem_scan_bwd(_p(q), _p(k), _p(e), _p(v), _p(la), _p(b), BH, T, hs, g, float(m), float(cap),
                                  _p(F0), _p(S0), _p(dy), _p(dF_T), _p(dS_T), _p(o["dq"]), _p(o["dk"]), _p(o["de"]),
                                  _p(o["dv"]), _p(o["dla"]), _p(o["db"]), _p(o["dF0"]), _p(o["dS0"]), _p(work),
-                                 nbytes, _stream()), "ava_mem_scan_bwd")
+                                 nbytes, current_stream()), "ava_mem_scan_bwd")
     return o
 
 
@@ -278,7 +274,7 @@ def dense_back(S, G, wf, base, col, i0, L, nd):
     nf = lib().ava_dense_back_part_floats(M, nd)
     part = torch.empty(max(nf, 1), dtype=torch.float32, device=base.device)
     check(lib().ava_dense_back(_p(S), _p(G), _p(wf), _p(base), _p(out), _p(dw), col, i0, L, nd, M, _p(part), nf,
-                               _stream()), "ava_dense_back")
+                               current_stream()), "ava_dense_back")
     return out, dw[:nd]
 
 
@@ -303,11 +299,11 @@ def attend(q: torch.Tensor, ks: torch.Tensor, vs: torch.Tensor, n0: int, heads: 
             raise ValueError("attend: one head of 64 dims (heads > 1 for wider rows)")
         n = lib().ava_attend_part_floats(B, T, n0)
         part = torch.empty(max(n, 1), dtype=torch.float32, device=q.device)
-        check(lib().ava_attend(_p(q), 64, _p(ks), _p(vs), half, cap, n0, B, T, _p(out), _p(part), n, _stream()),
+        check(lib().ava_attend(_p(q), 64, _p(ks), _p(vs), half, cap, n0, B, T, _p(out), _p(part), n, current_stream()),
               "ava_attend")
         return out
     n = lib().ava_attend_heads_part_floats(B, T, n0, de, heads)
     part = torch.empty(max(n, 1), dtype=torch.float32, device=q.device)
     check(lib().ava_attend_heads(_p(q), de, _p(ks), _p(vs), half, cap, n0, B, T, de, heads, _p(out), _p(part), n,
-                                 _stream()), "ava_attend_heads")
+                                 current_stream()), "ava_attend_heads")
     return out

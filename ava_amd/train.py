@@ -17,7 +17,7 @@ import ctypes as C
 import numpy as np
 import torch
 
-from ._lib import BLOCK_FIELDS, check, config_struct, lib
+from ._lib import BLOCK_FIELDS, check, config_struct, current_stream, lib
 
 GLOBAL = ("tok_emb", "final_norm")
 
@@ -86,7 +86,7 @@ class Trainer:
         if grads is None:
             grads = torch.empty_like(flat)
         B, T = ids.shape
-        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = current_stream()
         check(lib().ava_train_step(self.h, C.c_void_p(flat.data_ptr()), C.c_void_p(ids.data_ptr()),
                                    C.c_void_p(targets.data_ptr()), B, T, C.c_void_p(grads.data_ptr()),
                                    C.c_void_p(self.loss.data_ptr()), stream), "ava_train_step")
@@ -99,7 +99,7 @@ class Trainer:
         spk = torch.empty((L, N, c["d"]), dtype=torch.int8, device="cuda")
         u = torch.empty((L, N, c["hidden"]), dtype=torch.float32, device="cuda")
         kth = torch.empty((L, N), dtype=torch.float32, device="cuda")
-        stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        stream = current_stream()
         check(lib().ava_train_decisions(self.h, C.c_void_p(spk.data_ptr()), C.c_void_p(u.data_ptr()),
                                         C.c_void_p(kth.data_ptr()), stream), "ava_train_decisions")
         return {"spikes": spk, "u": u, "kth": kth}
