@@ -889,6 +889,144 @@ int launch_small_fn(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk
     return AVA_OK;
 }
 
+// ------------------------------------------------------------------ a few f32 rows: quantizer and product in a launch
+//
+// Single rows cost launches and host calls more than work, so up to ROW_FLOATS values (k a multiple of 256) are
+// quantized by every workgroup of the product itself: the 512 threads hold the rows in registers, the rows' largest
+// magnitudes meet in LDS (whole-number maxima of the bits, in any order), and the planes go to LDS where the product's
+// fragments read them, 16-byte chunks XOR-swizzled by the row. Meanwhile the wave's first weight steps load. The rest is
+// q8_small_kernel's with 32-column blocks and 8 waves, to the same bits. Bound by the chain of latencies: 1 x 512 x 2048
+// 4.0 us where the two launches take 5.6, and a call from Python 8.4 us where it took 11.5.
+//
+// What each workgroup repeats grows with the values, and the launches that it saves do not. In a stream of launches,
+// k = 1024, n = 2048: 1 row 6.4 -> 4.6 us, 4 rows 6.8 -> 5.5, but 8 rows 6.8 -> 7.4; 1 x 4096 x 1024 9.6 -> 8.2, but 2 rows
+// 9.8 -> 10.1: hence ROW_FLOATS. ROW_COLS is a block for each CU: 1 x 1024 x 8192 8.0 -> 4.8 us, x 32768 11.0 -> 11.9.
+constexpr int ROW_MAX = 16, ROW_FLOATS = 4096, ROW_COLS = 8192, ROW_D = 4, ROW_RING = 8 * ROW_D * 2048;
+
+template <int P>
+__global__ __launch_bounds__(512) void q8_rows_kernel(const float *__restrict__ x, int m, int n, int k,
+                                                      const int8_t *__restrict__ qt, const float *__restrict__ scale,
+                                                      EpiArgs ep) {
+    extern __shared__ __attribute__((aligned(16))) int8_t smem[];  // the ring of weight steps, then the planes
+    __shared__ unsigned rmax[ROW_MAX];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n0 = blockIdx.x * 32;
+    int8_t *wbuf = smem + wave * ROW_D * 2048, *planes = smem + ROW_RING;
+    const int total = m * k;
+    f32x4 held[ROW_FLOATS / 2048];
+#pragma unroll
+    for (int i = 0; i < ROW_FLOATS / 2048; i++) {
+        const int e = i * 2048 + tid * 4;
+        held[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (e < total) held[i] = *reinterpret_cast<const f32x4 *>(x + e);
+    }
+    const int8_t *src[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int r = i * 16 + lane / 4;
+        src[i] = qt + (size_t)min(n0 + r, n - 1) * k + swz<4>(r, lane % 4) * 16;
+    }
+    // step s of this wave is K step wave + 8 s, staged in buffer s % ROW_D
+    auto issue = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) dma16(src[i] + (wave + 8 * s) * 64, wbuf + (s % ROW_D) * 2048 + i * 1024);
+    };
+    const int KT = k / 64, ns = wave < KT ? (KT - wave + 7) / 8 : 0;
+#pragma unroll
+    for (int s = 0; s < ROW_D - 1; s++)
+        if (s < ns) issue(s);
+    SmallPre<EPI_STORE, 1, 8> pre;
+    small_prefetch<P, EPI_STORE, 1, 8>(pre, m, n, 0, n0, nullptr, scale, ep, lane, wave);
+
+    if (tid < ROW_MAX) rmax[tid] = 0;
+    __syncthreads();
+    // a wave's 256 consecutive values lie in one row
+#pragma unroll
+    for (int i = 0; i < ROW_FLOATS / 2048; i++) {
+        const int e = i * 2048 + wave * 256;
+        if (e < total) {
+            float a = 0.0f;
+#pragma unroll
+            for (int z = 0; z < 4; z++) a = fmaxf(a, fabsf(held[i][z]));
+            a = ava::wave_max(a);
+            if (lane == 0) atomicMax(&rmax[e / k], __float_as_uint(a));
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ROW_FLOATS / 2048; i++) {
+        const int e = i * 2048 + tid * 4;
+        if (e < total) {
+            const int row = e / k, kk = e - row * k, ex = ava::plane_exp(__uint_as_float(rmax[row]));
+            int q[4][P];
+#pragma unroll
+            for (int z = 0; z < 4; z++) ava::to_planes<P>(held[i][z], ex, q[z]);
+#pragma unroll
+            for (int p = 0; p < P; p++)
+                *reinterpret_cast<uint32_t *>(planes + (p * m + row) * k + (((kk >> 4) ^ (row & 7)) << 4) + (kk & 15)) =
+                    ava::pack4(q[0][p], q[1][p], q[2][p], q[3][p]);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int r = wave + 8 * q, row = min((r >> 2) * 8 + (lane >> 5) * 4 + (r & 3), m - 1);
+        pre.ex[q] = ava::plane_exp(__uint_as_float(rmax[row])) - 7 * (P - 1);
+    }
+    __syncthreads();
+
+    i32x16 acc[P][1];
+#pragma unroll
+    for (int p = 0; p < P; p++) acc[p][0] = i32x16{};
+    const int frow = lane & 31, fc = lane >> 5;
+    for (int s = 0; s < ns; s++) {
+        if (s + ROW_D - 1 < ns) issue(s + ROW_D - 1);
+        wait_steps<2, ROW_D>(min(ROW_D - 1, ns - 1 - s));  // step s is in LDS; the later ones may be in flight
+        const int8_t *lb = wbuf + (s % ROW_D) * 2048;
+        const int kt = wave + 8 * s;
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            const i32x4 bf = *reinterpret_cast<const i32x4 *>(lb + frow * 64 + swz<4>(frow, ks * 2 + fc) * 16);
+#pragma unroll
+            for (int p = 0; p < P; p++) {
+                i32x4 af = {0, 0, 0, 0};
+                if (frow < m)
+                    af = *reinterpret_cast<const i32x4 *>(planes + (p * m + frow) * k +
+                                                          (((kt * 4 + ks * 2 + fc) ^ (frow & 7)) << 4));
+                acc[p][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf, acc[p][0], 0, 0, 0);
+            }
+        }
+        // the buffer is refilled ROW_D - 1 steps on: its fragment reads must have completed
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#endif
+    }
+    __syncthreads();  // every wave is done with its buffers
+    small_epilogue<P, EPI_STORE, 1, 8>(acc, smem, m, n, 0, n0, pre, ep, lane, wave);
+}
+
+// y may lie on x where the quantizer is its own launch; here every workgroup reads x while others write y.
+bool rows_fit(const float *x, const float *y, int m, const ava_qw *w) {
+    const int k = w->din;
+    const bool apart = y + (size_t)m * w->dout <= x || x + (size_t)m * k <= y;
+    return k % 256 == 0 && (long)m * k <= ROW_FLOATS && w->dout <= ROW_COLS && (uintptr_t)x % 16 == 0 && apart;
+}
+
+int launch_rows(const float *x, int m, const ava_qw *w, int planes, float *y, hipStream_t st) {
+    const int k = w->din;
+    EpiArgs ep{y, w->dout, nullptr, 1};
+    const size_t lds = (size_t)ROW_RING + (size_t)planes * m * k;
+    auto go = [&](auto kern) -> int {
+        if (int r = ava::lds_opt_in((const void *)kern, (size_t)ROW_RING + 3 * ROW_FLOATS)) return r;
+        kern<<<dim3((w->dout + 31) / 32), dim3(512), lds, st>>>(x, m, w->dout, k, w->qt, w->scale, ep);
+        AVA_LAUNCHED("q8_rows");
+        return AVA_OK;
+    };
+    static_assert(ROW_RING >= 8 * 16 * 64 * 8, "the epilogue's partial sums fit the ring");
+    static_assert(ROW_MAX * 256 >= ROW_FLOATS, "no more rows than maxima");
+    if (planes == 1) return go(q8_rows_kernel<1>);
+    if (planes == 2) return go(q8_rows_kernel<2>);
+    return go(q8_rows_kernel<3>);
+}
+
 // 8 waves per workgroup when the grid gives a CU one workgroup or fewer, else 4 (two per CU); single
 // planes (spikes) stage so little per step that 4 waves do better.
 template <int P, int EPI, int FN>
@@ -1086,6 +1224,7 @@ extern "C" int ava_q8_matmul(const float *x, int m, const ava_qw *w, int planes,
                 "q8_matmul: workspace %zu < %zu bytes", ws_bytes, ava_q8_workspace(m, w->din, planes));
     if (m == 0) return AVA_OK;
     hipStream_t st = (hipStream_t)stream;
+    if (rows_fit(x, y, m, w)) return launch_rows(x, m, w, planes, y, st);
     int8_t *xq = (int8_t *)ws;
     int32_t *xe = (int32_t *)(((uintptr_t)(xq + (size_t)planes * m * w->ldk) + 255) & ~(uintptr_t)255);
     if (int r = ava::launch_quant_rows(x, m, w->din, w->din, planes, xq, xe, st)) return r;
@@ -1151,6 +1290,7 @@ extern "C" int ava_q8_matmul_noalloc(const float *x, int m, const ava_qw *w, int
     void *ws = nullptr;
     if (int r = scratch_ptr(&ws)) return r;
     hipStream_t st = (hipStream_t)stream;
+    if (rows_fit(x, y, m, w)) return launch_rows(x, m, w, planes, y, st);
     int8_t *xq = (int8_t *)ws;
     int32_t *xe = (int32_t *)(((uintptr_t)(xq + (size_t)planes * m * w->ldk) + 255) & ~(uintptr_t)255);
     if (int r = ava::launch_quant_rows(x, m, w->din, w->din, planes, xq, xe, st)) return r;
