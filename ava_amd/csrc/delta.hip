@@ -322,18 +322,32 @@ __global__ __launch_bounds__(256) void delta_inv_kernel(DeltaInvArgs p) {
 //   P3  Y = QF + X D, F += K^T D
 // and the next chunk's K, Q, V, T' arrive in registers during the chunk and are split into LDS at its end.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 constexpr int PST = 72;  // bf16 per row of a term plane
 constexpr int PLANE = C * PST;
 constexpr int NTMAX = 3;  // term planes per buffer
 
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+// The terms of two values, packed as they are stored: one conversion gives a term of both, and each is taken back by
+// a shift or a mask (5.5 operations a value; a value at a time, with its terms packed afterwards, 8.5).
 template <int N>
-__device__ __forceinline__ void splitn(float x, __bf16 (&o)[N]) {
+__device__ __forceinline__ void split2(float a, float b, unsigned (&o)[N]) {
 #pragma unroll
     for (int i = 0; i < N; i++) {
-        o[i] = (__bf16)x;
-        x = x - (float)o[i];
+        o[i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+        a = a - __uint_as_float(o[i] << 16);
+        b = b - __uint_as_float(o[i] & 0xffff0000u);
     }
+}
+template <int N>
+__device__ __forceinline__ void split4(float a, float b, float c, float d, u32x2 (&o)[N]) {
+    unsigned lo[N], hi[N];
+    split2<N>(a, b, lo);
+    split2<N>(c, d, hi);
+#pragma unroll
+    for (int i = 0; i < N; i++) o[i] = u32x2{lo[i], hi[i]};
 }
 
 // Products over the wave's quadrant, k = 0..63: A's rows ar0 .. ar0 + 31 and B's columns bc0 .. bc0 + 31
@@ -349,6 +363,17 @@ __device__ __forceinline__ Frag<P> ldf(const __bf16 *B, int row, int k) {
     Frag<P> f;
 #pragma unroll
     for (int i = 0; i < P; i++) f.t[i] = *reinterpret_cast<const bf16x8 *>(B + i * PLANE + row * PST + k);
+    return f;
+}
+// K's columns (B5), 16-byte chunk k / 8 of row r at chunk (k / 8) ^ (r / 8): stage() writes them two k at a time down
+// the rows, 4 rows apart from lane to lane, and each of a wave's 16 rows would meet in 2 banks without the swizzle.
+// (Reads are of 8 consecutive rows at one chunk, as in the other buffers.)
+__device__ __forceinline__ int kcol(int r, int k) { return r * PST + (((k >> 3) ^ (r >> 3)) << 3) + (k & 7); }
+template <int P>
+__device__ __forceinline__ Frag<P> ldf_kcol(const __bf16 *B, int row, int k) {
+    Frag<P> f;
+#pragma unroll
+    for (int i = 0; i < P; i++) f.t[i] = *reinterpret_cast<const bf16x8 *>(B + i * PLANE + kcol(row, k));
     return f;
 }
 struct Acc3 {
@@ -380,6 +405,16 @@ __device__ __forceinline__ void mq_bf(f32x16 &acc, const __bf16 *A, int ar0, con
         mfma_terms<P>(c, ldf<P>(A, ar0 + r, k0 + 16 * ks), ldf<P>(B, bc0 + r, k0 + 16 * ks));
     acc = total<P>(c);
 }
+// the same with A = K's columns
+template <int P>
+__device__ __forceinline__ void mq_bf_kcol(f32x16 &acc, const __bf16 *A, int ar0, const __bf16 *B, int bc0, int lane) {
+    const int r = lane & 31, k0 = 8 * (lane >> 5);
+    Acc3 c{acc, {}, {}};
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++)
+        mfma_terms<P>(c, ldf_kcol<P>(A, ar0 + r, k0 + 16 * ks), ldf<P>(B, bc0 + r, k0 + 16 * ks));
+    acc = total<P>(c);
+}
 // acc1 (+)= A1 B and acc2 (+)= A2 B (one B operand)
 template <int P>
 __device__ __forceinline__ void mq_bf_2a(f32x16 &acc1, const __bf16 *A1, int a1r0, f32x16 &acc2, const __bf16 *A2,
@@ -404,33 +439,21 @@ __device__ __forceinline__ void put_cols(__bf16 *B, const f32x16 &x, int row0, i
     const int c = col0 + (lane & 31);
 #pragma unroll
     for (int g = 0; g < 4; g++) {
-        bf16x4 t[P];
-#pragma unroll
-        for (int z = 0; z < 4; z++) {
-            __bf16 o[P];
-            splitn<P>(x[4 * g + z], o);
-#pragma unroll
-            for (int i = 0; i < P; i++) t[i][z] = o[i];
-        }
+        u32x2 t[P];
+        split4<P>(x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3], t);
         const int r = row0 + g * 8 + (lane >> 5) * 4;
 #pragma unroll
-        for (int i = 0; i < P; i++) *reinterpret_cast<bf16x4 *>(B + i * PLANE + c * PST + r) = t[i];
+        for (int i = 0; i < P; i++) *reinterpret_cast<u32x2 *>(B + i * PLANE + c * PST + r) = t[i];
     }
 }
 
 // 4 consecutive values of a row into a term buffer (row layout) at row r, columns c .. c + 3
 template <int P>
 __device__ __forceinline__ void put_row4(__bf16 *B, int r, int c, const f32x4 &x) {
-    bf16x4 t[P];
+    u32x2 t[P];
+    split4<P>(x[0], x[1], x[2], x[3], t);
 #pragma unroll
-    for (int z = 0; z < 4; z++) {
-        __bf16 o[P];
-        splitn<P>(x[z], o);
-#pragma unroll
-        for (int i = 0; i < P; i++) t[i][z] = o[i];
-    }
-#pragma unroll
-    for (int i = 0; i < P; i++) *reinterpret_cast<bf16x4 *>(B + i * PLANE + r * PST + c) = t[i];
+    for (int i = 0; i < P; i++) *reinterpret_cast<u32x2 *>(B + i * PLANE + r * PST + c) = t[i];
 }
 
 constexpr size_t DELTA_BF_LDS = 5 * (size_t)NTMAX * PLANE * sizeof(__bf16) + sizeof(float) * C * LD;
@@ -451,6 +474,10 @@ __device__ __forceinline__ void mq_bf_half(f32x16 &acc, const __bf16 *A, int ar0
 // Y; wave w >= 4 ("state" waves) owns quadrant w - 4 of F (f32 in its registers) and computes X^T and the
 // update K^T D; D = T' R splits its k range between the two sets (the state waves' half added through
 // the LDS that held V). Each phase thus has two waves per SIMD to overlap.
+// Bound by its phases' latencies (5 barriers a chunk; one workgroup's LDS fills a CU), so what shortens a phase counts:
+// 256 heads x 4096, both launches, 671 -> 613 us when the terms came to be split in pairs (split2: 12% fewer VALU
+// operations, no spilled registers) and K's columns written as pairs into swizzled rows (12 instead of
+// 24 LDS writes a thread and chunk, without bank conflicts).
 __global__ __launch_bounds__(512) void delta_seq_bf_kernel(DeltaArgs p, const float *__restrict__ Tp) {
     extern __shared__ __attribute__((aligned(16))) float smb[];
     __bf16 *B1 = reinterpret_cast<__bf16 *>(smb);  // F columns (P1), then R columns (P2)
@@ -476,14 +503,14 @@ __global__ __launch_bounds__(512) void delta_seq_bf_kernel(DeltaArgs p, const fl
     }
 
     // the next chunk's inputs in registers: float4 j of thread t is row (t + 512 j) / 16, columns
-    // 4 ((t + 512 j) % 16) .. + 3
+    // 4 ((t + 512 j) % 16) .. + 3; of K, row 2 (t / 16) + j, so that a thread holds two rows' values of a column
     f32x4 pk[2], pq[2], pv[2], pt[2];
     auto fetch = [&](int ch) {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int idx = tid + 512 * j;
             const size_t o = (size_t)(ch * C + (idx >> 4)) * C + (idx & 15) * 4;
-            pk[j] = *reinterpret_cast<const f32x4 *>(kh + o);
+            pk[j] = *reinterpret_cast<const f32x4 *>(kh + (size_t)(ch * C + 2 * (tid >> 4) + j) * C + (tid & 15) * 4);
             pq[j] = *reinterpret_cast<const f32x4 *>(qh + o);
             pv[j] = *reinterpret_cast<const f32x4 *>(vh + o);
             pt[j] = *reinterpret_cast<const f32x4 *>(Th + (size_t)ch * C * C + (idx >> 4) * C + (idx & 15) * 4);
@@ -491,23 +518,28 @@ __global__ __launch_bounds__(512) void delta_seq_bf_kernel(DeltaArgs p, const fl
     };
     // K rows (B4) and K columns (B5) from one split, Q rows (B2), T' rows (B3); V as f32
     auto stage = [&]() {
+        {
+            const int r = 2 * (tid >> 4), c = (tid & 15) * 4;
+            u32x2 k0[3], k1[3];
+            split4<3>(pk[0][0], pk[0][1], pk[0][2], pk[0][3], k0);
+            split4<3>(pk[1][0], pk[1][1], pk[1][2], pk[1][3], k1);
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                *reinterpret_cast<u32x2 *>(B4 + i * PLANE + r * PST + c) = k0[i];
+                *reinterpret_cast<u32x2 *>(B4 + i * PLANE + (r + 1) * PST + c) = k1[i];
+#pragma unroll
+                for (int z = 0; z < 4; z++) {
+                    const unsigned a = k0[i][z >> 1], b = k1[i][z >> 1];
+                    *reinterpret_cast<unsigned *>(B5 + i * PLANE + kcol(c + z, r)) =
+                        z & 1 ? (a >> 16) | (b & 0xffff0000u) : (a & 0xffffu) | (b << 16);
+                }
+            }
+        }
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int idx = tid + 512 * j, r = idx >> 4, c = (idx & 15) * 4;
-            bf16x4 kt[3];
 #pragma unroll
-            for (int z = 0; z < 4; z++) {
-                __bf16 o[3];
-                splitn<3>(pk[j][z], o);
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    kt[i][z] = o[i];
-                    B5[i * PLANE + (c + z) * PST + r] = o[i];
-                }
-                sV[r * LD + c + z] = pv[j][z];
-            }
-#pragma unroll
-            for (int i = 0; i < 3; i++) *reinterpret_cast<bf16x4 *>(B4 + i * PLANE + r * PST + c) = kt[i];
+            for (int z = 0; z < 4; z++) sV[r * LD + c + z] = pv[j][z];
             put_row4<3>(B2, r, c, pq[j]);
             put_row4<3>(B3, r, c, pt[j]);
         }
@@ -563,7 +595,7 @@ __global__ __launch_bounds__(512) void delta_seq_bf_kernel(DeltaArgs p, const fl
             for (int i = 0; i < 16; i++) yh[(size_t)(t0 + row0 + qrow(i, lane)) * C + col0 + lc] = qf[i];
         } else {
             f32x16 a = {};
-            mq_bf<3>(a, B5, row0, B3, col0, lane);
+            mq_bf_kcol<3>(a, B5, row0, B3, col0, lane);
 #pragma unroll
             for (int i = 0; i < 16; i++) Fr[i] = Fr[i] + a[i];
             put_cols<3>(B1, Fr, row0, col0, lane);
