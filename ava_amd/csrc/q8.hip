@@ -603,7 +603,7 @@ __global__ __launch_bounds__(64 * GEMM_WM * GEMM_WN, BM * BN < 16384 ? 4 : 1) vo
     wait_vm<0>();  // no load into LDS outlives the workgroup
 }
 
-// Products of at most this many rows take the few-rows kernel.
+// Products of more rows never take the few-rows kernel (see launch_gemm).
 constexpr int SMALL_ROWS = 512;
 // Few-rows products of at least this many columns take 64-column blocks.
 constexpr int SMALL_WIDE_COLS = 4096;
@@ -1086,8 +1086,22 @@ int launch_tiled(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk, c
 template <int P, int EPI>
 int launch_gemm(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk, const int8_t *qt, const float *scale,
                 EpiArgs ep, hipStream_t st) {
-    // few rows (decode): 32-row blocks with the K steps spread over the waves
-    if (m <= SMALL_ROWS) return launch_small<P, EPI>(xq, xexp, m, n, ldk, qt, scale, ep, st);
+    // Few rows (decode): 32-row blocks with the K steps spread over the waves, while the CUs hold them about at once. Past
+    // 1.5 of 32 x 64 a CU (2 for spikes and long rows, which hide the loads' latencies worse in tiles) the tiles below
+    // take less time, whose operands are read once per 64 to 128 rows. Three planes, us here / in tiles, weights from the
+    // caches (from HBM): k = 1024, 128 x 5120 (320 blocks) 8.4 / 7.5 (10.4 / 11.0), 192 x 4096 (384) 8.7 / 7.5 (10.2 / 10.9),
+    // 256 x 4096 (512) 9.4 / 7.6 (10.7 / 11.0), 256 x 5120 (640) 13.0 / 7.8 (14.8 / 11.1), 256 x 8192 16.2 / 8.6 (18.3 / 11.5),
+    // 512 x 8192 29.0 / 14.5; k = 4096: 192 x 4096 (384) 24.4 / 25.8, 288 x 4096 (576) 33.1 / 25.7. Spikes, k = 1024: 256 x 4096
+    // (512) 6.2 / 6.3, 256 x 5120 8.4 / 6.3. Two planes have the largest tile only, and stay here.
+    if (m <= SMALL_ROWS) {
+        bool here = m <= 64 || P == 2 || EPI == EPI_ACC;
+        if (!here) {
+            int cus = 0;
+            if (int r = ava::device_cus(&cus)) return r;
+            here = (long)((m + 31) / 32) * ((n + 63) / 64) * 2 <= (P == 1 || ldk > 2048 ? 4L : 3L) * cus;
+        }
+        if (here) return launch_small<P, EPI>(xq, xexp, m, n, ldk, qt, scale, ep, st);
+    }
     // 128-byte K steps (whole cache lines per load request) for every plane count: for the single
     // spike plane at 131,072 x 1024 x 1024 they measured 279 us against 340 us for 64-byte steps
     if constexpr (P != 2 && EPI != EPI_ACC) {

@@ -367,6 +367,15 @@ def test_q8_tiles_bit_exact(din, dout, m, kind, dev):
         assert np.array_equal(host(y).view(np.uint32), want.view(np.uint32)), planes
 
 
+# Up to 512 rows the tiles take over past 1.5 of 32 x 64 blocks a CU (two for spikes), from 65 rows: on either side of
+# both lines, with ragged tiles both ways
+@pytest.mark.parametrize("din,dout,m", [(200, 8190, 90), (200, 8200, 90), (1100, 8200, 65), (1100, 8200, 64),
+                                        (200, 2060, 512)])
+@pytest.mark.parametrize("kind", [1, 2, 3])
+def test_q8_tiles_of_few_rows_bit_exact(din, dout, m, kind, dev):
+    test_q8_tiles_bit_exact(din, dout, m, kind, dev)
+
+
 @pytest.mark.parametrize("din,dout,m", SHAPES)
 def test_q8_spike_product_is_the_reference_bits(din, dout, m, dev):
     """Integer inputs: the i8 MFMA product equals the reference's f32 fma chain bit for bit."""
