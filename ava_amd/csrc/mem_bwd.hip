@@ -18,15 +18,16 @@
 //      every step; and, in other workgroups of the same launch, the reverse walk of (dF, dS) as if no
 //      element reached the bound, parking (dF, dS) at every chunk's end and dr_j of every step, and writing dv.
 //      The forward marks the workgroups in which an element did reach it.
-//   2. mem_bwd_bound_kernel: the reverse walk again, with the bound's mask, in the marked workgroups' columns
-//      (the others return at once).
+//   2. mem_bwd_bound_kernel: the reverse walk again from the parked end, with the bound's mask, for the heads with a
+//      marked workgroup (the others return at once).
 //   3. mem_bwd_rows_kernel: per (head, chunk) the steps replayed from the parked states and walked back from
 //      the parked gradients. r_j and dr_j are known, so no column sum is left: lane = row, each wave 8
-//      columns, the row sums in the lane, the per-column values in scalar registers.
+//      columns, the row sums in the lane, the per-column values in scalar registers. The first chunk's workgroups end
+//      with dF0 and dS0. Every output but dv is written here, after the last read of the inputs it may lie on.
 // Measured, per-channel gates and momentum: 64 heads x 2048 steps 783 us (walks 478 us under the profiler, rows 445), 16 heads 343
 // us, 256 heads 2.64 ms, 1024 heads x 512 steps 2.59 ms; one kernel that parked every 4th state and walked three times
 // in series, the last walk forming the row sums too: 2.41, 1.87, 5.14 and 3.49 ms.
-// Workspace per (head, chunk): (F, S, dF, dS) of 16 KB (F and dF without momentum), and r and dr per step.
+// Workspace per (head, chunk): (F, S, dF, dS) of 16 KB (F and dF without momentum), and r, dr and room for dv per step.
 #include <algorithm>
 
 #include "common.h"
@@ -361,12 +362,6 @@ __global__ __launch_bounds__(256) void mem_bwd_walk_kernel(MemBwdArgs p) {
             }
         }
     }
-#pragma unroll
-    for (int m = 0; m < NE; m++) {
-        const size_t o = fb + (size_t)(i0 + m / CPL) * HS + j0 + m % CPL;
-        if (p.dF0) p.dF0[o] = dF[m];
-        if (MOM && p.dS0) p.dS0[o] = dS[m];
-    }
 }
 
 // 2. The reverse walk with the bound's mask, for the heads in which an element reached it: every
@@ -380,14 +375,19 @@ __global__ __launch_bounds__(256) void mem_bwd_bound_kernel(MemBwdArgs p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15;
     const int i0 = 4 * l16, j = 16 * cg + 4 * wave + (lane >> 4);
     const int T = p.T, nck = (T + CK - 1) / CK;
-    const size_t hb = (size_t)bh * T * HS, fb = (size_t)bh * HS * HS;
+    const size_t hb = (size_t)bh * T * HS;
     const float M = p.m, cap = p.cap;
+    // the gradients after the last step, as the first walk parked them
     float dF[4], dS[4];
+    {
+        const f32x4 f = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, nck - 1, 1) + j * HS + i0);
+        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (MOM) s = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, nck - 1, 3) + j * HS + i0);
 #pragma unroll
-    for (int m = 0; m < 4; m++) {
-        const size_t o = fb + (size_t)(i0 + m) * HS + j;
-        dF[m] = p.dFT ? p.dFT[o] : 0.0f;
-        dS[m] = (MOM && p.dST) ? p.dST[o] : 0.0f;
+        for (int m = 0; m < 4; m++) {
+            dF[m] = f[m];
+            dS[m] = s[m];
+        }
     }
     for (int c = nck - 1; c >= 0; c--) {
         const int n = min(CK, T - c * CK);
@@ -434,12 +434,6 @@ __global__ __launch_bounds__(256) void mem_bwd_bound_kernel(MemBwdArgs p) {
                 }
             }
     }
-#pragma unroll
-    for (int m = 0; m < 4; m++) {
-        const size_t o = fb + (size_t)(i0 + m) * HS + j;
-        if (p.dF0) p.dF0[o] = dF[m];
-        if (MOM && p.dS0) p.dS0[o] = dS[m];
-    }
 }
 
 // 3. The rows' gradients of one (head, chunk): lane = row, wave w columns 8w .. 8w + 7. The steps are replayed from
@@ -451,10 +445,10 @@ __global__ __launch_bounds__(256) void mem_bwd_bound_kernel(MemBwdArgs p) {
 // 210; keeping all 16 F (one workgroup per CU) 580, without the operands' read-ahead 487.
 constexpr int RW = 8, RG = 2, HC = CK / 2;  // waves (8 columns each), steps per combine, steps whose F are kept
 
-typedef const __attribute__((address_space(4))) float *ScalarPtr;  // uniform, not written by the kernel
+typedef const __attribute__((address_space(4))) float *ScalarPtr;  // uniform, written (by an output on an input) after the last read only
 
 struct RowsLds {
-    float q[CK][HS], e[CK][HS], a[CK][HS], bk[CK][HS], abe[CK][HS];
+    float q[CK][HS], k[CK][HS], e[CK][HS], a[CK][HS], b[CK][HS], abe[CK][HS];
     float red[2][RW][RG][5][HS];  // per buffer, wave and step: dq, sum gP F, sv, sr, sum dr F
 };
 
@@ -481,7 +475,7 @@ __device__ __forceinline__ void rows_chunk(const MemBwdArgs &p, RowsLds &L, int 
     // A step's operands are read while the step before it is computed, and not earlier (sched_barrier ends each
     // step: the scalar registers hold two steps').
     struct FwdIn {
-        float v[NC], r[NC], a, k, x;
+        float v[NC], r[NC], a, b, k, x;
     };
     struct RevIn {
         float v[NC], r[NC], y[NC], d[NC], q, e, a;
@@ -493,7 +487,8 @@ __device__ __forceinline__ void rows_chunk(const MemBwdArgs &p, RowsLds &L, int 
             in.r[z] = rr[s * HS + z];
         }
         in.a = L.a[s][lane];
-        in.k = L.bk[s][lane];
+        in.b = L.b[s][lane];
+        in.k = L.k[s][lane];
         in.x = L.abe[s][lane];
     };
     auto read_rev = [&](RevIn &in, int s) {
@@ -510,9 +505,10 @@ __device__ __forceinline__ void rows_chunk(const MemBwdArgs &p, RowsLds &L, int 
     };
     // F after a step from F before it (S in place)
     auto replay = [&](const FwdIn &in, const float (&Fa)[NC], float (&Fb)[NC]) {
+        const float bk = in.b * in.k;
 #pragma unroll
         for (int z = 0; z < NC; z++) {
-            const float u = fmaf(-in.x, in.r[z], in.k * in.v[z]);
+            const float u = fmaf(-in.x, in.r[z], bk * in.v[z]);
             if (MOM) S[z] = fmaf(M, S[z], u);
             const float f = fmaf(in.a, Fa[z], MOM ? S[z] : u);
             Fb[z] = BOUND ? __builtin_amdgcn_fmed3f(f, -cap, cap) : f;
@@ -600,7 +596,7 @@ __device__ __forceinline__ void rows_chunk(const MemBwdArgs &p, RowsLds &L, int 
                     return x;
                 };
                 const size_t o = hb + (size_t)t * HS + lane, og = G1 ? (size_t)bh * p.T + t : o;
-                const float a = L.a[s][lane], b = p.b[og], e = L.e[s][lane], sr = sum(3);
+                const float a = L.a[s][lane], b = L.b[s][lane], e = L.e[s][lane], sr = sum(3);
                 if ((wave & 1) == 0) {
                     p.dq[o] = sum(0);
                     const float da = fmaf(-(b * e), sr, sum(1)) * a;
@@ -614,7 +610,7 @@ __device__ __forceinline__ void rows_chunk(const MemBwdArgs &p, RowsLds &L, int 
                     const float sv = sum(2);
                     p.dk[o] = b * sv;
                     p.de[o] = fmaf(-(a * b), sr, sum(4));
-                    const float db = fmaf(-(a * e), sr, p.k[o] * sv);
+                    const float db = fmaf(-(a * e), sr, L.k[s][lane] * sv);
                     if (G1) {
                         const float x = ava::wave_sum(db);
                         if (lane == 0) p.db[og] = x;
@@ -624,6 +620,16 @@ __device__ __forceinline__ void rows_chunk(const MemBwdArgs &p, RowsLds &L, int 
                 }
             }
         }
+    }
+    if (c == 0) {
+        const size_t o = (size_t)bh * HS * HS + (size_t)lane * HS + NC * wave;
+        auto put = [&](float *dst, const float (&X)[NC]) {
+            if (!dst) return;
+#pragma unroll
+            for (int z = 0; z < NC; z++) dst[o + z] = X[z];
+        };
+        put(p.dF0, dF);
+        if (MOM) put(p.dS0, dS);
     }
 }
 
@@ -639,9 +645,10 @@ __global__ __launch_bounds__(64 * RW, 4) void mem_bwd_rows_kernel(MemBwdArgs p) 
             const size_t o = ((size_t)bh * p.T + c * CK + s) * HS + lane, og = G1 ? (size_t)bh * p.T + c * CK + s : o;
             const float a = expf(p.la[og]), b = p.b[og], e = p.e[o];
             L.q[s][lane] = p.q[o];
+            L.k[s][lane] = p.k[o];
             L.e[s][lane] = e;
             L.a[s][lane] = a;
-            L.bk[s][lane] = b * p.k[o];
+            L.b[s][lane] = b;
             L.abe[s][lane] = (a * b) * e;
         }
     }
@@ -665,9 +672,14 @@ __global__ __launch_bounds__(64 * RW, 4) void mem_bwd_rows_kernel(MemBwdArgs p) 
         rows_chunk<G1, MOM, false, false>(p, L, bh, c, n, lane, wave);
 }
 
+// dv, formed in the workspace (see ava_mem_scan_bwd)
+__global__ __launch_bounds__(256) void mem_bwd_copy_kernel(const float *__restrict__ x, float *__restrict__ y, size_t n) {
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) y[i] = x[i];
+}
+
 struct Layout {
-    size_t ck, r, hit;  // floats
-    size_t bytes() const { return (ck + 2 * r + hit) * sizeof(float); }
+    size_t ck, r, hit;  // floats: the parked states; r, dr, and dv where it cannot go out at once; the marks
+    size_t bytes() const { return (ck + 3 * r + hit) * sizeof(float); }
 };
 Layout layout(int BH, int T, bool mom) {
     return {(size_t)BH * ((T + CK - 1) / CK) * (mom ? 4 : 2) * HS * HS, (size_t)BH * T * HS, (size_t)BH * 8};
@@ -699,8 +711,14 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
     const Layout lo = layout(BH, T, mom);
     float *w = (float *)work;
     MemBwdArgs p{q, k, e, v, la, b, F0, mom ? S0 : nullptr, dy, dF_T, mom ? dS_T : nullptr, dq, dk, de, dv, dla, db,
-                 dF0, mom ? dS0 : nullptr, w, w + lo.ck, w + lo.ck + lo.r, (int *)(w + lo.ck + 2 * lo.r), 0, BH, T, m, cap};
+                 dF0, mom ? dS0 : nullptr, w, w + lo.ck, w + lo.ck + lo.r, (int *)(w + lo.ck + 3 * lo.r), 0, BH, T, m, cap};
     const hipStream_t st = (hipStream_t)stream;
+    // An output may be an input's buffer. The rows kernel writes the others, each element after its last read; the
+    // walks write dv while the inputs are still wanted, so on one of them it goes through the workspace.
+    const size_t nv = lo.r, ng = (size_t)BH * T * g;
+    auto on = [&](const float *x, size_t n) { return (uintptr_t)dv < (uintptr_t)(x + n) && (uintptr_t)x < (uintptr_t)(dv + nv); };
+    const bool late = on(q, nv) || on(k, nv) || on(e, nv) || on(v, nv) || on(dy, nv) || on(la, ng) || on(b, ng);
+    if (late) p.dv = w + lo.ck + 2 * lo.r;
     const int rows = BH * ava::ceil_div(T, CK);
     auto walk = [&](auto kern, int groups) {
         p.groups = groups;
@@ -713,6 +731,7 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
         else walk(w1, 1);
         bound<<<BH * 4, 256, 0, st>>>(p);
         rows_k<<<rows, 64 * RW, 0, st>>>(p);
+        if (late) mem_bwd_copy_kernel<<<(unsigned)std::min<size_t>(2048, (nv + 255) / 256), 256, 0, st>>>(p.dv, dv, nv);
     };
 #define AVA_MB(G1_, MOM_)                                                                                            \
     run(mem_bwd_walk_kernel<G1_, MOM_, 2, 1>, mem_bwd_walk_kernel<G1_, MOM_, 4, 1>,                                 \

@@ -199,7 +199,8 @@ int ava_kwta_relu2_bwd(const float *u, const float *kth, int n, int h, const flo
  * dq, dk, de, dv [BH][T][hs]; dla, db [BH][T][g]; dF0, dS0 [BH][hs][hs] (nullable) = dL/d(F0, S0).
  * The bound clamp(., +-cap) passes no gradient where it holds. work: device memory of
  * ava_mem_scan_bwd_workspace(BH, T, m != 0) bytes (the states and their gradients at every 16th step, and the
- * columns' recalls and their gradients at every step). Replaces memg_bwd_* /
+ * columns' recalls, their gradients and dv at every step). An output may be the buffer of an input of its layout (dF0
+ * on dF_T or F0, dk on k, dv on dy, db on b). Replaces memg_bwd_* /
  * memg_bwd4_* (gpu/lif.cu:3411-3888; MemGenBwd, gpu/mem_gen.rs:296-470) and the gradient of delta_rec
  * (gpu/arch.rs:1091-1136). */
 size_t ava_mem_scan_bwd_workspace(int BH, int T, int momentum);

@@ -302,6 +302,41 @@ def test_mem_bwd_walk_shapes(BH, T, g, m, cap):
         assert e < 1e-5, (n, e)
 
 
+# outputs on inputs of their layout: the carried gradients; each on its own input; turned round; on dy
+ALIASES = [{"dF0": "dF_T", "dS0": "dS_T"}, {"dF0": "F0", "dS0": "S0"},
+           {"dq": "q", "dk": "k", "de": "e", "dv": "v", "dla": "la", "db": "b"},
+           {"dq": "k", "dk": "e", "de": "v", "dv": "q", "dla": "b", "db": "la"}, {"dv": "dy"}, {"dq": "dy", "dv": "k"}]
+
+
+@pytest.mark.parametrize("alias", ALIASES)
+@pytest.mark.parametrize("BH,T,g,m", [(6, 37, 64, 0.5), (6, 37, 1, 0.0), (70, 18, 64, 0.5), (130, 33, 1, 0.5)])
+@pytest.mark.parametrize("cap", [1e5, 0.6])
+def test_mem_bwd_in_place(alias, BH, T, g, m, cap):
+    """Outputs on the inputs' buffers, through the C entry (the wrapper allocates its own): the bits of a call
+    with buffers of its own, with and without elements at the bound."""
+    import ctypes as C
+    from ava_amd import _lib
+    names = ("q", "k", "e", "v", "la", "b", "F0", "S0", "dy", "dF_T", "dS_T")
+    x = mem_inputs(BH + T + g, BH, T, g)
+    print(f"mem_bwd in place {alias} BH={BH} T={T} g={g} m={m} cap={cap}", flush=True)
+    want = run_mem(x, m, cap)
+    i = {n: dev(z) for n, z in zip(names, x)}
+    like = {"dla": "la", "db": "b", "dF0": "F0", "dS0": "S0"}
+    o = {n: i[alias[n]] if n in alias else torch.empty_like(i[like.get(n, "q")])
+         for n in ("dq", "dk", "de", "dv", "dla", "db", "dF0", "dS0")}
+    L = _lib.lib()
+    nb = L.ava_mem_scan_bwd_workspace(BH, T, int(m != 0))
+    work = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    p = lambda t: C.c_void_p(t.data_ptr())
+    s = lambda n: p(i[n]) if m else None
+    _lib.check(L.ava_mem_scan_bwd(p(i["q"]), p(i["k"]), p(i["e"]), p(i["v"]), p(i["la"]), p(i["b"]), BH, T, 64, g, m,
+                                  cap, p(i["F0"]), s("S0"), p(i["dy"]), p(i["dF_T"]), s("dS_T"), p(o["dq"]), p(o["dk"]),
+                                  p(o["de"]), p(o["dv"]), p(o["dla"]), p(o["db"]), p(o["dF0"]),
+                                  p(o["dS0"]) if m else None, p(work), nb, _lib.current_stream()), "ava_mem_scan_bwd")
+    for n in MEM_OUT + (("dS0",) if m else ()):
+        assert np.array_equal(host(o[n]), want[n]), n
+
+
 def test_wrappers_ignore_the_default_dtype():
     """The wrappers allocate float32 whatever torch's default dtype is (a float64 default once gave
     float64 output buffers that the kernels, writing float32, left mostly unwritten)."""
