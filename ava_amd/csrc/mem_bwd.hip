@@ -37,6 +37,9 @@ namespace {
 constexpr int HS = 64, CK = 16;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// the caller's tensors, which need not lie on 16 bytes (the hardware takes any multiple of 4)
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 
 template <int CTRL>
 __device__ __forceinline__ float dppf(float v) {
@@ -102,7 +105,7 @@ struct Loader {
         q = k = e = c = la = b = z;
         if (t0 < 0 || t >= p.T) return;
         const size_t o = ((size_t)bh * p.T + t) * HS + si;
-        auto at = [&](const float *x) { return *reinterpret_cast<const f32x4 *>(x + o); };
+        auto at = [&](const float *x) -> f32x4 { return *reinterpret_cast<const f32x4u *>(x + o); };
         k = at(p.k);
         e = at(p.e);
         c = at(FWD ? p.v : p.dy);
@@ -657,8 +660,8 @@ __global__ __launch_bounds__(64 * RW, 4) void mem_bwd_rows_kernel(MemBwdArgs p) 
     {
         const size_t o = ((size_t)bh * p.T + c * CK) * HS + min(2 * tid, n * HS - 2);
         for (const float *x : {p.v, p.dy, (const float *)p.r, (const float *)p.dr}) {
-            const float2 w = *reinterpret_cast<const float2 *>(x + o);
-            warm += w.x + w.y;
+            const f32x2u w = *reinterpret_cast<const f32x2u *>(x + o);
+            warm += w[0] + w[1];
         }
     }
     const bool bound = head_hit(p, bh);

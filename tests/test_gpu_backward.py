@@ -337,6 +337,36 @@ def test_mem_bwd_in_place(alias, BH, T, g, m, cap):
         assert np.array_equal(host(o[n]), want[n]), n
 
 
+@pytest.mark.parametrize("BH,T,g,m", [(6, 37, 64, 0.5), (130, 18, 1, 0.0)])
+@pytest.mark.parametrize("cap", [1e5, 0.6])
+def test_mem_bwd_off_16_bytes(BH, T, g, m, cap):
+    """Inputs and outputs one float past a 16-byte boundary: the bits of aligned ones."""
+    x = mem_inputs(BH + T + g, BH, T, g)
+    print(f"mem_bwd off 16 bytes BH={BH} T={T} g={g} m={m} cap={cap}", flush=True)
+    want = run_mem(x, m, cap)
+    import ctypes as C
+    from ava_amd import _lib
+    L = _lib.lib()
+
+    def off(n):
+        t = torch.empty(n + 1, dtype=torch.float32, device="cuda")[1:]
+        assert t.data_ptr() % 16 == 4
+        return t
+
+    i = [off(z.size).copy_(dev(z).view(-1)) for z in x]
+    o = {n: off(want[n].size) for n in MEM_OUT + (("dS0",) if m else ())}
+    nb = L.ava_mem_scan_bwd_workspace(BH, T, int(m != 0))
+    work = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    p = lambda t: C.c_void_p(t.data_ptr())
+    q, k, e, v, la, b, F0, S0, dy, dF, dS = (p(t) for t in i)
+    _lib.check(L.ava_mem_scan_bwd(q, k, e, v, la, b, BH, T, 64, g, m, cap, F0, S0 if m else None, dy, dF,
+                                  dS if m else None, p(o["dq"]), p(o["dk"]), p(o["de"]), p(o["dv"]), p(o["dla"]),
+                                  p(o["db"]), p(o["dF0"]), p(o["dS0"]) if m else None, p(work), nb,
+                                  _lib.current_stream()), "ava_mem_scan_bwd")
+    for n in o:
+        assert np.array_equal(host(o[n]), want[n].reshape(-1)), n
+
+
 def test_wrappers_ignore_the_default_dtype():
     """The wrappers allocate float32 whatever torch's default dtype is (a float64 default once gave
     float64 output buffers that the kernels, writing float32, left mostly unwritten)."""
