@@ -1,14 +1,17 @@
 // The training step's f32 products on the f16 matrix cores of gfx950.
 //
 // C [m][n] = A . B (+ C) for f32 operands, with each operand split into two f16 terms under a power of
-// two per row of A and per column of B: x = 2^e (hi + lo + r), hi the f16 nearest x 2^-e and lo the f16
-// nearest the rest, so |r| <= 2^-23 |x 2^-e| (or 2^-25 for values far below the row's largest, which is
-// scaled to [2^14, 2^15)). Three of the four term products are kept, hi hi in one accumulator, hi lo and
-// lo hi in another (lo lo is below 2^-22 of the product), f32 accumulation, and the powers of two go back
-// exactly in the epilogue. The error against float64 is below that of an f32 matrix product: each matrix
-// instruction adds 16 products to a sum, so a sum is rounded K/16 times instead of K/4 (relative 2-norm on
-// normal inputs, this form against rocBLAS f32: K = 1024 2.1e-7 / 5.7e-7, 4096 4.1e-7 / 1.2e-6, 8192 in 8 parts
-// 2.2e-7 / 1.6e-6, 64 7.9e-8 / 1.4e-7; rows spread over 40 binades the same; log-normal inputs 2.8e-7 / 2.7e-7).
+// two per row of A and per column of B: x = 2^e (hi + 2^-12 lo + r), hi the f16 nearest x 2^-e and lo the f16
+// nearest 2^12 times the rest. The row's largest value is scaled to [2^14, 2^15), lo's factor gives the rest hi's
+// range: |r| <= 2^-23 |x 2^-e|, and at most 2^-51 of the row's largest for values some 2^28 below it. Three of the four term
+// products are kept, hi hi in one accumulator, hi lo and lo hi in another (lo lo is at most 2^-22 of the product), f32
+// accumulation, and the powers of two go back exactly in the epilogue. The sum is rounded once per matrix instruction
+// of 16 products, K/16 times instead of K/4. Relative 2-norm against float64, this form / a library f32 product: normal
+// operands K = 64 9.8e-8 / 1.4e-7, 1024 1.4e-7 / 5.7e-7, 4096 2.2e-7 / 1.2e-6; rows spread over 40 binades the same;
+// log-normal (sigma 1, 2) at K = 1024 1.4e-7 / 5.7e-7, 1.5e-7 / 5.3e-7; a training step's operands (spikes, normed rows, relu^2
+// rows, the logits' gradient, token gradients of log-normal size) 0.7-2.9e-7 / 1.3-9.0e-7; one element of a row 1e8 times the others, meeting
+// zeros 1.4e-7 / 5.7e-7 (1e9 2.8e-7, 1e10 2.6e-6). Where one product is nearly all of a sum, an f32 product rounds it
+// once and this one's operands count: one-hot rows 4.4e-8 / 0, log-normal of sigma 3 8.1e-8 / 1.3e-8.
 // Measured: 8192 x 1024 x 1024 49 us (352 TFLOP/s of f32 products, 1.05 PFLOP/s of f16) against 148 us in
 // rocBLAS, 8192 x 8192 x 1024 361 / 1000, 1024 x 4096 x 8192 171 / 460; a large bf16 library product runs at
 // 1.2 PFLOP/s on the same card, so the matrix cores bound it. The splits move 12 bytes an element.
@@ -39,10 +42,11 @@ __device__ __forceinline__ int split_exp(float amax) {
     return ex - 15;
 }
 
+constexpr float LO_SCALE = 4096.0f;  // |x 2^-e - hi| <= 2^-11 of a value below 2^15: lo stays below 2^15 too
 __device__ __forceinline__ void split1(float x, int e, _Float16 &hi, _Float16 &lo) {
     const float t = ldexpf(x, -e);
     hi = (_Float16)t;
-    lo = (_Float16)(t - (float)hi);
+    lo = (_Float16)((t - (float)hi) * LO_SCALE);
 }
 
 // W waves per row of x [rows][cols] (cols <= 256 W NV): its exponent, then its blocks of 32. A lane holds
@@ -383,7 +387,7 @@ __global__ __launch_bounds__(512, 1) void hgemm_kernel(HgemmArgs p) {
             }
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                float v = ldexpf(acc[i][j][r] + crs[i][j][r], row_exp(er, r) + eb[j]);
+                float v = ldexpf(fmaf(crs[i][j][r], 1.0f / LO_SCALE, acc[i][j][r]), row_exp(er, r) + eb[j]);
                 if (add) v = old[r] + v;
                 store_f32(rc, voc[j] + soff(r), 0, v);
             }
