@@ -159,3 +159,30 @@ def test_zero_rows_subnormals_and_extremes():
         c, parts = product(a, b, cols, cols)
         check(a, b, c, parts)
         assert torch.all(c[5] == 0.0) and torch.all(c[:, 9] == 0.0)
+
+
+@pytest.mark.parametrize("cols", [False, True])
+@pytest.mark.parametrize("k", [96, 2048])
+def test_infinities_and_nan_as_in_an_f32_product(cols, k):
+    """An infinity or NaN reaches its own row or column only, as the infinity (of its sign) or NaN that a product of the
+    values gives, also with values beside it that f16 would not hold (1e6; a value more than 2^39 below its row's largest
+    counts as zero to an infinity it meets); opposite infinities and infinity times zero give NaN."""
+    a, b = rnd(31, 140, k), rnd(32, 270, k)
+    b[:, 5] = torch.where(b[:, 5] > 0, 1.0, -2.0)  # no second term
+    a[3, 5] = float("inf")
+    a[4, 5], a[4, 6] = float("-inf"), 1e6
+    a[5, 7] = float("nan")
+    a[6, 5], a[6, 8] = float("inf"), float("-inf")
+    b[10, 5] = 0.0
+    b[20, 9] = float("inf")
+    b[21, 9] = float("nan")
+    a[7, 9] = 0.0
+    c, parts = product(a, b, cols, cols)
+    got, want = f64(c), f64(a) @ f64(b).t()
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    inf = torch.isinf(want)
+    assert inf.any() and torch.equal(torch.isinf(got), inf) and torch.equal(got[inf], want[inf])
+    keep_a = torch.isfinite(a).all(1)
+    keep_b = torch.isfinite(b).all(1)
+    assert torch.isfinite(got[keep_a.cpu()][:, keep_b.cpu()]).all()
+    check(a[keep_a], b[keep_b], c[keep_a][:, keep_b], parts)
