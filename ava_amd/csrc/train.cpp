@@ -89,6 +89,7 @@ struct ava_trainer {
     // the products' split operands (a stack: see Arena) and scratch
     char *hplanes = nullptr;
     size_t hplanes_bytes = 0, hplanes_used = 0;
+    int unsplit = 0;  // products of the step that found no room there
     float *hpart = nullptr;
     size_t hpart_floats = 0;
 
@@ -146,13 +147,24 @@ struct Arena {
     ~Arena() { tr->hplanes_used = used; }
 };
 
+// The bytes of an operand of `rows` rows over k in the stack: its planes, its exponents and, over the rows of x (tr), the
+// columns' partial maxima.
+size_t al256(size_t n) { return (n + 255) & ~(size_t)255; }
+size_t split_bytes(size_t rows, size_t k, bool tr) {
+    return al256(ava::hgemm_plane_bytes(rows, (int)k)) + al256(rows * 4) +
+           (tr ? al256(ava::hgemm_part_floats((int)k, (int)rows) * 4) : 0);
+}
+size_t split_bytes(const Op &x, bool tr) {
+    if ((tr ? x.t : x.n).planes) return 0;
+    return tr ? split_bytes(x.cols, x.rows, true) : split_bytes(x.rows, x.cols, false);
+}
+
 // Splits x over k = rows (tr) or cols, if it is not yet and the stack has room.
 int split(ava_trainer *t, Op &x, bool tr, hipStream_t st) {
     ava::HgemmOp &o = tr ? x.t : x.n;
     if (o.planes) return AVA_OK;
     const int rows = tr ? x.cols : x.rows, k = tr ? x.rows : x.cols;
-    const size_t pb = (ava::hgemm_plane_bytes(rows, k) + 255) & ~(size_t)255, eb = ((size_t)rows * 4 + 255) & ~(size_t)255;
-    const size_t need = pb + eb + (tr ? ((ava::hgemm_part_floats(x.rows, x.cols) * 4 + 255) & ~(size_t)255) : 0);
+    const size_t pb = al256(ava::hgemm_plane_bytes(rows, k)), eb = al256((size_t)rows * 4), need = split_bytes(x, tr);
     if (t->hplanes_used + need > t->hplanes_bytes) return AVA_OK;
     char *p = t->hplanes + t->hplanes_used;
     t->hplanes_used += need;
@@ -184,7 +196,12 @@ int gemm(ava_trainer *t, bool tA, bool tB, Op &A, Op &B, bool keepA, bool keepB,
     const ava::HgemmOp &pa = tA ? A.t : A.n, &pb = tB ? B.n : B.t;
     const bool thin = std::min(M, N) <= 64 && macs >= HGEMM_THIN && (M >= N ? pa : pb).planes;
     const int parts = ava::hgemm_splits(M, N, K);
-    if (!f32 && (macs >= HGEMM_MACS || thin) && (parts == 1 || (size_t)parts * M * N <= t->hpart_floats)) {
+    bool cores = !f32 && (macs >= HGEMM_MACS || thin) && (parts == 1 || (size_t)parts * M * N <= t->hpart_floats);
+    if (cores && t->hplanes_used + split_bytes(A, tA) + split_bytes(B, !tB) > t->hplanes_bytes) {
+        cores = false;
+        t->unsplit++;
+    }
+    if (cores) {
         if (keepA)
             if (int r = split(t, A, tA, st)) return r;
         if (keepB)
@@ -192,7 +209,7 @@ int gemm(ava_trainer *t, bool tA, bool tB, Op &A, Op &B, bool keepA, bool keepB,
         Arena call(t);
         if (int r = split(t, A, tA, st)) return r;
         if (int r = split(t, B, !tB, st)) return r;
-        if (pa.planes && pb.planes) return ava::hgemm(pa, pb, M, N, K, C, ldc, add, t->hpart, t->hpart_floats, st);
+        return ava::hgemm(pa, pb, M, N, K, C, ldc, add, t->hpart, t->hpart_floats, st);
     }
     const float one = 1.0f, beta = add ? 1.0f : 0.0f;
     const rocblas_status s =
@@ -276,17 +293,14 @@ int ensure(ava_trainer *t, int B, int T) {
         AF(t->lws, t->lws_floats);
         for (size_t i = 0; i < L; i++) AF(t->acts[i].lpark, ava::lif_park_floats(B, T, (int)d));
     }
-    // the split operands: the largest set alive at once (the head's products, the MLP's, the memory's with the
-    // normed rows kept); none when no product of this batch is large enough. A product that finds no room
-    // runs in rocBLAS.
+    // the split operands: both of the largest product and, beside them, one kept for several products (the normed
+    // rows); none when no product of this batch is large enough
     t->hplanes_bytes = t->hpart_floats = 0;
-    if ((double)N * d * std::max<size_t>(H, V) >= HGEMM_MACS) {
-        auto pl = [](size_t rows, size_t k) {
-            return ava::hgemm_plane_bytes(rows, (int)k) + 4 * (rows + ava::hgemm_part_floats((int)k, (int)rows)) + 4096;
-        };
-        t->hplanes_bytes = std::max({pl(N, d) + pl(V, d), pl(V, N) + pl(d, N), pl(N, V) + pl(d, V),
-                                     pl(H, N) + pl(d, N), pl(N, d) + pl(H, d), pl(N, H) + pl(d, H),
-                                     pl(d, N) * 2 + pl(N, d) + pl(d, d)}) + pl(d, N);
+    if ((double)N * d * std::max({H, V, d, de}) >= HGEMM_MACS) {
+        auto two = [](size_t m, size_t n, size_t k) { return split_bytes(m, k, true) + split_bytes(n, k, true); };
+        for (size_t x : {V, H, d, de, nh, r})
+            t->hplanes_bytes = std::max({t->hplanes_bytes, two(N, x, d), two(N, d, x), two(x, d, N)});
+        t->hplanes_bytes += std::max(split_bytes(N, d, true), split_bytes(d, N, true));
         TR(alloc(t, (void **)&t->hplanes, t->hplanes_bytes));
         t->hpart_floats = ava::hgemm_part_max();
         AF(t->hpart, t->hpart_floats);
@@ -322,6 +336,7 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
     const float *wdense = pb + t->dense_off;
     AVA_HIP(hipMemsetAsync(grads, 0, t->nparams * sizeof(float), st));
     t->hplanes_used = 0;
+    t->unsplit = 0;
     // a named operand keeps its planes to the end of its Arena
     auto mm = [&](bool tA, bool tB, auto &&A, auto &&B, bool add, float *C, int ldc) {
         return gemm(t, tA, tB, A, B, std::is_lvalue_reference<decltype(A)>::value,
@@ -338,7 +353,6 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
         const float *xin = i == 0 ? x0 : (c.dense ? t->xmix + (size_t)(i - 1) * Nd : t->streams + (size_t)i * Nd);
         // spiking layer: z = rms(x) Win, cur = z (1 - beta), the scan, x1 = x + s Wout
         TR(ava::train::rms_fwd(xin, N, d, w("lif_norm"), a.h1, a.inv1, st));
-        Arena fwd(t);  // this block's split operands
         // (the currents stay in rocBLAS: their last bits decide spikes, and a step's spikes are those of a step
         // before the split products; 148 us against 69 with the splits at 8192 rows)
         Op h1{a.h1, N, d, d}, win{w("win"), d, d, d};
@@ -358,16 +372,19 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
         TR(mm(false, false, Op{a.S, N, d, d}, Op{w("wout"), d, d, d}, true, a.x1, d));
         // memory
         TR(ava::train::rms_fwd(a.x1, N, d, w("mem_norm"), a.h2, a.inv2, st));
-        Op h2{a.h2, N, d, d};
-        TR(mm(false, false, h2, Op{w("wq"), d, d, d}, false, a.q, d));
-        TR(mm(false, false, h2, Op{w("wk"), d, d, d}, false, a.k, d));
-        TR(mm(false, false, h2, Op{w("wv"), d, d, d}, false, a.v, d));
-        TR(mm(false, false, h2, Op{w("we"), d, d, d}, false, a.we, d));
-        TR(mm(false, false, h2, Op{w("wg"), d, d, d}, false, a.g, d));
-        TR(mm(false, false, h2, Op{w("wa"), d, nh, nh}, false, a.zab, 2 * nh));
-        TR(mm(false, false, h2, Op{w("wb"), d, nh, nh}, false, a.zab + nh, 2 * nh));
-        TR(mm(false, false, h2, Op{w("wa1"), d, r, r}, false, a.z1, 2 * r));
-        TR(mm(false, false, h2, Op{w("wb1"), d, r, r}, false, a.z1 + r, 2 * r));
+        {
+            Arena mem(t);
+            Op h2{a.h2, N, d, d};
+            TR(mm(false, false, h2, Op{w("wq"), d, d, d}, false, a.q, d));
+            TR(mm(false, false, h2, Op{w("wk"), d, d, d}, false, a.k, d));
+            TR(mm(false, false, h2, Op{w("wv"), d, d, d}, false, a.v, d));
+            TR(mm(false, false, h2, Op{w("we"), d, d, d}, false, a.we, d));
+            TR(mm(false, false, h2, Op{w("wg"), d, d, d}, false, a.g, d));
+            TR(mm(false, false, h2, Op{w("wa"), d, nh, nh}, false, a.zab, 2 * nh));
+            TR(mm(false, false, h2, Op{w("wb"), d, nh, nh}, false, a.zab + nh, 2 * nh));
+            TR(mm(false, false, h2, Op{w("wa1"), d, r, r}, false, a.z1, 2 * r));
+            TR(mm(false, false, h2, Op{w("wb1"), d, r, r}, false, a.z1 + r, 2 * r));
+        }
         TR(mm(false, false, Op{a.z1, N, r, 2 * r}, Op{w("wa2"), r, d, d}, false, a.lra, d));
         TR(mm(false, false, Op{a.z1 + r, N, r, 2 * r}, Op{w("wb2"), r, d, d}, false, a.lrb, d));
         if (i == 0) vfirst = a.v;
@@ -385,11 +402,14 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
         const float *x3 = a.x2;
         if (i == c.eng_block) {
             TR(ava::train::rms_fwd(a.x2, N, d, w("eng_norm"), a.h3, a.inv3, st));
-            Op h3{a.h3, N, d, d};
-            TR(split(t, h3, false, st));  // one split for three thin products
-            TR(mm(false, false, h3, Op{w("ewq"), d, de, de}, false, a.eq, de));
-            TR(mm(false, false, h3, Op{w("ewk"), d, de, de}, false, a.ek, de));
-            TR(mm(false, false, h3, Op{w("ewv"), d, de, de}, false, a.ev, de));
+            {
+                Arena eng(t);
+                Op h3{a.h3, N, d, d};
+                TR(split(t, h3, false, st));  // one split for three thin products
+                TR(mm(false, false, h3, Op{w("ewq"), d, de, de}, false, a.eq, de));
+                TR(mm(false, false, h3, Op{w("ewk"), d, de, de}, false, a.ek, de));
+                TR(mm(false, false, h3, Op{w("ewv"), d, de, de}, false, a.ev, de));
+            }
             TR(ava_attend_heads(a.eq, de, a.ek, a.ev, 0, T, 0, B, T, de, enh, a.att, t->att_part, t->att_part_floats,
                                 st));
             AVA_HIP(hipMemcpyAsync(a.x3, a.x2, Nd * 4, hipMemcpyDeviceToDevice, st));
@@ -449,8 +469,8 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
             TrainAttn at{a.eq, a.ek, a.ev, a.att, t->datt, t->deq, t->dek, t->dev, t->alse, t->adsum,
                          B, T, de, enh, de / enh, (float)(1.0 / sqrt((double)(de / enh)))};
             TR(ava::train::attn_bwd(at, st));
-            Op h3{a.h3, N, d, d};
             Arena eng(t);
+            Op h3{a.h3, N, d, d};
             TR(split(t, h3, true, st));  // one split for three thin products
             TR(mm(true, false, h3, Op{t->deq, N, de, de}, false, gw("ewq"), de));
             TR(mm(true, false, h3, Op{t->dek, N, de, de}, false, gw("ewk"), de));
@@ -625,6 +645,8 @@ extern "C" int ava_train_step(ava_trainer *t, const float *params, const int32_t
     if (int e = ensure(t, B, T)) return e;
     return step(t, params, ids, targets, B, T, grads, loss, (hipStream_t)stream);
 }
+
+extern "C" int ava_train_unsplit(const ava_trainer *t) { return t ? t->unsplit : 0; }
 
 extern "C" int ava_train_decisions(const ava_trainer *t, int8_t *spikes, float *u, float *kth, ava_stream stream) {
     AVA_REQUIRE(t && t->N > 0, AVA_ERR_ARG, "train_decisions: no step has run");

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from ava_amd import synth
+from ava_amd._lib import lib
 
 import train_ref as R
 
@@ -27,12 +28,15 @@ def test_train_step_matches_autograd(name, B, T):
 
 # Batches whose head, wide-layer and square products go to the f16 matrix cores: rows that fill neither a
 # 128-row tile nor a 64-value K block (1029, 501), K cut into parts and not, a vocabulary that is no
-# multiple of 4 (the 4-byte split passes, a ragged last tile), thin products on shared operands.
+# multiple of 4 (the 4-byte split passes, a ragged last tile), thin products on shared operands; vocabularies
+# below and above the wide layer (the largest operands are then W2's or the head's), an engram read as wide as the block.
 @pytest.mark.parametrize("name,B,T,over", [("ava04_d512", 1, 501, {}), ("ava04_d512", 1, 1029, {"vocab": 5003}),
-                                           ("ava04_d1024", 3, 704, {"vocab": 300})])
+                                           ("ava04_d1024", 3, 704, {"vocab": 300}),
+                                           ("ava04_d512", 1, 1029, {"vocab": 300}),
+                                           ("ava04_d1024", 1, 2000, {"vocab": 300, "eng_dim": 1024, "eng_heads": 32})])
 def test_train_step_on_the_matrix_cores_matches_autograd(name, B, T, over):
     cfg = synth.config(name)
-    cfg.update(layers=1, eng_block=0, **over)
+    cfg.update({"layers": 1, "eng_block": 0, **over})
     check_step(name, cfg, B, T)
 
 
@@ -48,6 +52,7 @@ def check_step(name, cfg, B, T):
     flat = tr.pack(prm)
     loss, grads = tr.step(flat, torch.from_numpy(ids).cuda(), torch.from_numpy(tgt).cuda())
     torch.cuda.synchronize()
+    assert lib().ava_train_unsplit(tr.h) == 0  # no product fell back to the library for want of room
     dec = tr.decisions(B, T)
     spikes = dec["spikes"].cpu().numpy()
     keep = (dec["u"] - dec["kth"][:, :, None] >= 0.0).to(torch.uint8).cpu().numpy()
