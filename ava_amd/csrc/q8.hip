@@ -1088,11 +1088,13 @@ int launch_gemm(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk, co
                 EpiArgs ep, hipStream_t st) {
     // Few rows (decode): 32-row blocks with the K steps spread over the waves, while the CUs hold them about at once. Past
     // 1.5 of 32 x 64 a CU (2 for spikes and long rows, which hide the loads' latencies worse in tiles) the tiles below
-    // take less time, whose operands are read once per 64 to 128 rows. Three planes, us here / in tiles, weights from the
+    // take less time, whose operands are read once per 64 to 128 rows: less with the weights in the caches, the same within 3%
+    // up to 2 a CU with the weights from HBM. Three planes, us here / in tiles, weights from the
     // caches (from HBM): k = 1024, 128 x 5120 (320 blocks) 8.4 / 7.5 (10.4 / 11.0), 192 x 4096 (384) 8.7 / 7.5 (10.2 / 10.9),
-    // 256 x 4096 (512) 9.4 / 7.6 (10.7 / 11.0), 256 x 5120 (640) 13.0 / 7.8 (14.8 / 11.1), 256 x 8192 16.2 / 8.6 (18.3 / 11.5),
-    // 512 x 8192 29.0 / 14.5; k = 4096: 192 x 4096 (384) 24.4 / 25.8, 288 x 4096 (576) 33.1 / 25.7. Spikes, k = 1024: 256 x 4096
-    // (512) 6.2 / 6.3, 256 x 5120 8.4 / 6.3. Two planes have the largest tile only, and stay here.
+    // 448 x 2048 (448) 11.0 / 8.0 (12.4 / 10.7), 256 x 4096 (512) 9.6 / 8.1 (10.7 / 11.0), 128 x 8192 (512) 9.3 / 7.9 (10.6 / 10.6),
+    // 256 x 5120 (640) 13.0 / 7.8 (14.8 / 11.1), 256 x 8192 16.2 / 8.6 (18.3 / 11.5), 512 x 8192 29.0 / 14.5; k = 4096: 192 x 4096
+    // (384) 24.4 / 25.8, 288 x 4096 (576) 33.1 / 25.7. Spikes, k = 1024: 256 x 4096 (512) 6.6 / 6.5 (8.0 / 9.8), 320 x 4096
+    // (640) 8.8 / 6.6 (10.8 / 9.8). Two planes have the largest tile only, and stay here.
     if (m <= SMALL_ROWS) {
         bool here = m <= 64 || P == 2 || EPI == EPI_ACC;
         if (!here) {
@@ -1105,13 +1107,22 @@ int launch_gemm(const int8_t *xq, const int32_t *xexp, int m, int n, int ldk, co
     // 128-byte K steps (whole cache lines per load request) for every plane count: for the single
     // spike plane at 131,072 x 1024 x 1024 they measured 279 us against 340 us for 64-byte steps
     if constexpr (P != 2 && EPI != EPI_ACC) {
-        // The tile with the least rounds over the CUs, each weighed by its time on a full chip (128 x 256: 1).
+        // The tile with the least rounds over the CUs, each weighed by its time on a full chip: at k = 1024 a round of
+        // 128 x 256 tiles takes 20.7 us, of 128 x 128 12.2, of 64 x 128 6.2 (three planes; spikes 11.3 / 7.3 / 3.6). A last
+        // round of large tiles that leaves half the CUs idle takes 0.7 of one (k = 4096, 64 to 128 of 256: 51-60 us against 75;
+        // 192: 63), and a smaller tile has to gain 5% on that: it reads each operand more often, which weights from HBM
+        // feel. us, large / chosen by whole rounds: k = 4096, 192 large tiles 63 / 71 (spikes 34 / 44), 632 203 / 223 (100 / 118);
+        // k = 1024, 160 of 640 x 8192, weights from HBM, 19.0 / 22.6 (15.3 / 19.4). Smaller ones pay off up to half a round (128
+        // tiles: 18.8 / 14.3) and just past a whole one (10,000 x 1024, 314 tiles: 37.6 / 31.1, spikes 21.6 / 16.5). Up to
+        // k = 512 starts and epilogues are most of a tile, and whole rounds tell (3072 x 2048 x 512, 192 tiles: 12.5 / 12.0).
         int cus = 0;
         if (int r = ava::device_cus(&cus)) return r;
-        auto rounds = [&](int bm, int bn) {
-            return (double)((((long)(m + bm - 1) / bm) * ((n + bn - 1) / bn) + cus - 1) / cus);
-        };
-        const double big = rounds(128, 256), mid = rounds(128, 128) * 0.56, small = rounds(64, 128) * 0.32;
+        auto tiles = [&](int bm, int bn) { return ((long)(m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+        auto rounds = [&](int bm, int bn) { return (double)((tiles(bm, bn) + cus - 1) / cus); };
+        const long t = tiles(128, 256), last = t % cus;
+        const bool whole = ldk <= 512;
+        const double big = whole ? rounds(128, 256) : 0.95 * (t / cus + (last ? std::max(0.7, 0.4 + 0.6 * last / cus) : 0.0));
+        const double mid = rounds(128, 128) * 0.56, small = rounds(64, 128) * 0.32;
         if (small < big && small <= mid)
             return launch_tiled<P, EPI, 128, 64, 128>(xq, xexp, m, n, ldk, qt, scale, ep, st);
         if (mid < big) return launch_tiled<P, EPI, 128, 128, 128>(xq, xexp, m, n, ldk, qt, scale, ep, st);
