@@ -231,14 +231,14 @@ __device__ __forceinline__ void park(float *dst, const float (&X)[R * CPL], int 
     }
 }
 
-// 1. The walks. 4 / CPL workgroups per head and direction, each 16 CPL columns: lane l of wave w holds rows 4 (l &
-// 15).. + 3 of the CPL columns from j0, so a column sum is 4 FMAs and 4 DPP adds. A step's time is the dependent
-// chain through that sum and back (about 15 operations) against its issue and its LDS reads (5 16-byte vectors a
-// wave, 8 cycles of the CU's LDS each): step t + 1's operands are read during step t, and one barrier per chunk
+// 1. The walks. Lane l of the 64 / R lanes of a column holds its rows R l .. R l + R - 1, a wave R CPL columns, so a head and
+// direction has 16 / (R CPL) workgroups: 8 (R = 2), or 4, 2 and 1 (R = 4; CPL = 1, 2, 4). A column sum is R FMAs and 4 DPP adds
+// over the 16 lanes of a DPP row (R = 2: and a lane swap between two rows). A step's time is the dependent
+// chain through that sum and back (about 15 operations) against its issue and its LDS reads (5 vectors of R floats a
+// lane): step t + 1's operands are read during step t, and one barrier per chunk
 // covers the staging of the next. A wave alone on its SIMD issues one VALU operation per 8 cycles, two waves share
-// them: so few heads are split into more, smaller workgroups (2 rows a lane up to 32 heads; 4 rows of 1, 2 and 4
-// columns up to 64, 128 and beyond, where the operations per element fall: 9, 8 and 7 forward). 64 heads: 478 us with 1
-// column a lane (two waves per SIMD), 468 with 2 (one wave). The columns' r (dr, dv) of step s stay in lane s of the 16, so a chunk's go out in
+// them: so few heads are split into more, smaller workgroups, and the operations per element fall with more columns a lane (9, 8
+// and 7 forward). The columns' r (dr, dv) of step s stay in lane s, so a chunk's go out in
 // one store. Workgroups: the forward walks first, then the reverse.
 template <bool G1, bool MOM, int R, int CPL>
 __global__ __launch_bounds__(256) void mem_bwd_walk_kernel(MemBwdArgs p) {
@@ -716,6 +716,8 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
     MemBwdArgs p{q, k, e, v, la, b, F0, mom ? S0 : nullptr, dy, dF_T, mom ? dS_T : nullptr, dq, dk, de, dv, dla, db,
                  dF0, mom ? dS0 : nullptr, w, w + lo.ck, w + lo.ck + lo.r, (int *)(w + lo.ck + 3 * lo.r), 0, BH, T, m, cap};
     const hipStream_t st = (hipStream_t)stream;
+    int cus = 0;
+    if (int r = ava::device_cus(&cus)) return r;
     // An output may be an input's buffer. The rows kernel writes the others, each element after its last read; the
     // walks write dv while the inputs are still wanted, so on one of them it goes through the workspace.
     const size_t nv = lo.r, ng = (size_t)BH * T * g;
@@ -728,9 +730,13 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
         kern<<<BH * groups * 2, 256, 0, st>>>(p);
     };
     auto run = [&](auto w8, auto w4, auto w2, auto w1, auto bound, auto rows_k) {
-        if (BH <= 32) walk(w8, 8);
-        else if (BH <= 64) walk(w4, 4);
-        else if (BH <= 128) walk(w2, 2);
+        // A head's columns over 4 or 2 workgroups a direction while the CUs hold them all at once (three each, by LDS), over 8
+        // only while each has a CU to itself. All three launches, T = 1024, momentum, 8 / 4 / 2 / 1 workgroups: 16 heads
+        // 198 / 200 / 271 / 424 us, 32 277 / 241 / 311 / 462, 64 559 / 400 / 421 / 583, 96 747 / 569 / 589 / 671, 128 980 / 797 / 702
+        // / 769, 192 1427 / 1101 / 1004 / 1123, 256 - / 1446 / 1301 / 1296.
+        if (16L * BH <= cus) walk(w8, 8);
+        else if (8L * BH <= 3L * cus) walk(w4, 4);
+        else if (4L * BH <= 3L * cus) walk(w2, 2);
         else walk(w1, 1);
         bound<<<BH * 4, 256, 0, st>>>(p);
         rows_k<<<rows, 64 * RW, 0, st>>>(p);
