@@ -108,7 +108,7 @@ def lib():
         "ava_train_param_slot": [vp, C.c_char_p, i32, C.POINTER(sz), C.POINTER(sz)],
         "ava_train_step": [vp, vp, vp, vp, i32, i32, vp, vp, vp],
         "ava_train_decisions": [vp, vp, vp, vp, vp],
-        "ava_train_unsplit": [vp],
+        "ava_train_products": [vp, C.POINTER(C.c_int), C.POINTER(C.c_int)],
     }
     for name, args in sig.items():
         fn = getattr(L, name, None)

@@ -89,7 +89,7 @@ struct ava_trainer {
     // the products' split operands (a stack: see Arena) and scratch
     char *hplanes = nullptr;
     size_t hplanes_bytes = 0, hplanes_used = 0;
-    int unsplit = 0;  // products of the step that found no room there
+    int split = 0, unsplit = 0;  // products of the step in split form, and those that found no room there
     float *hpart = nullptr;
     size_t hpart_floats = 0;
 
@@ -179,10 +179,14 @@ int split(ava_trainer *t, Op &x, bool tr, hipStream_t st) {
 
 // Products of at least this many multiply-adds go to the f16 matrix cores: 8192 x 1024 x 1024 (8.6e9) takes
 // 49 us there and 12 + 8 us to split both operands, 148 us in rocBLAS; 2048 x 1024 x 1024 (2.1e9) 29 + 4 + 8
-// against 36; below, rocBLAS. Thin ones (at most 64 rows or columns: the gates, the rank-r read-outs, the
+// against 36, and a step of 2048 rows takes 4.47 ms with the line at 3e9, 4.55 at 2e9. Sums over K >= 4096 go from 2e9, where rocBLAS has few
+// tiles of long chains: a step of 256 rows 1.30 ms against 1.68, its 256 x 1024 x 8192 in rocBLAS. Below, rocBLAS.
+// Thin ones (at most 64 rows or columns: the gates, the rank-r read-outs, the
 // single-head engram) go there from HGEMM_THIN when the large operand is already split for another product:
 // 8192 x 64 x 1024 18 us against 29, 1024 x 64 x 8192 24 against 58.
-constexpr double HGEMM_MACS = 2e9, HGEMM_THIN = 1e8;
+constexpr double HGEMM_MACS = 3e9, HGEMM_LONG_MACS = 2e9, HGEMM_THIN = 1e8;
+constexpr int HGEMM_LONG = 4096;
+double hgemm_line(int K) { return K >= HGEMM_LONG ? HGEMM_LONG_MACS : HGEMM_MACS; }
 
 // row-major C [M][N] (ldc) = op(A) op(B) (+ C with add), op(A) [M][K] (A stored [M][K], or [K][M] when tA)
 // keepA, keepB: the operand is used again, its planes stay when the call ends (they are split first, below the
@@ -196,7 +200,7 @@ int gemm(ava_trainer *t, bool tA, bool tB, Op &A, Op &B, bool keepA, bool keepB,
     const ava::HgemmOp &pa = tA ? A.t : A.n, &pb = tB ? B.n : B.t;
     const bool thin = std::min(M, N) <= 64 && macs >= HGEMM_THIN && (M >= N ? pa : pb).planes;
     const int parts = ava::hgemm_splits(M, N, K);
-    bool cores = !f32 && (macs >= HGEMM_MACS || thin) && (parts == 1 || (size_t)parts * M * N <= t->hpart_floats);
+    bool cores = !f32 && (macs >= hgemm_line(K) || thin) && (parts == 1 || (size_t)parts * M * N <= t->hpart_floats);
     if (cores && t->hplanes_used + split_bytes(A, tA) + split_bytes(B, !tB) > t->hplanes_bytes) {
         cores = false;
         t->unsplit++;
@@ -209,6 +213,7 @@ int gemm(ava_trainer *t, bool tA, bool tB, Op &A, Op &B, bool keepA, bool keepB,
         Arena call(t);
         if (int r = split(t, A, tA, st)) return r;
         if (int r = split(t, B, !tB, st)) return r;
+        t->split++;
         return ava::hgemm(pa, pb, M, N, K, C, ldc, add, t->hpart, t->hpart_floats, st);
     }
     const float one = 1.0f, beta = add ? 1.0f : 0.0f;
@@ -296,7 +301,7 @@ int ensure(ava_trainer *t, int B, int T) {
     // the split operands: both of the largest product and, beside them, one kept for several products (the normed
     // rows); none when no product of this batch is large enough
     t->hplanes_bytes = t->hpart_floats = 0;
-    if ((double)N * d * std::max({H, V, d, de}) >= HGEMM_MACS) {
+    if ((double)N * d * std::max({H, V, d, de}) >= HGEMM_LONG_MACS) {
         auto two = [](size_t m, size_t n, size_t k) { return split_bytes(m, k, true) + split_bytes(n, k, true); };
         for (size_t x : {V, H, d, de, nh, r})
             t->hplanes_bytes = std::max({t->hplanes_bytes, two(N, x, d), two(N, d, x), two(x, d, N)});
@@ -336,7 +341,7 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
     const float *wdense = pb + t->dense_off;
     AVA_HIP(hipMemsetAsync(grads, 0, t->nparams * sizeof(float), st));
     t->hplanes_used = 0;
-    t->unsplit = 0;
+    t->split = t->unsplit = 0;
     // a named operand keeps its planes to the end of its Arena
     auto mm = [&](bool tA, bool tB, auto &&A, auto &&B, bool add, float *C, int ldc) {
         return gemm(t, tA, tB, A, B, std::is_lvalue_reference<decltype(A)>::value,
@@ -646,7 +651,12 @@ extern "C" int ava_train_step(ava_trainer *t, const float *params, const int32_t
     return step(t, params, ids, targets, B, T, grads, loss, (hipStream_t)stream);
 }
 
-extern "C" int ava_train_unsplit(const ava_trainer *t) { return t ? t->unsplit : 0; }
+extern "C" int ava_train_products(const ava_trainer *t, int *split, int *unsplit) {
+    AVA_REQUIRE(t && split && unsplit, AVA_ERR_ARG, "train_products: NULL argument");
+    *split = t->split;
+    *unsplit = t->unsplit;
+    return AVA_OK;
+}
 
 extern "C" int ava_train_decisions(const ava_trainer *t, int8_t *spikes, float *u, float *kth, ava_stream stream) {
     AVA_REQUIRE(t && t->N > 0, AVA_ERR_ARG, "train_decisions: no step has run");

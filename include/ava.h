@@ -431,9 +431,10 @@ int ava_train_step(ava_trainer *t, const float *params, const int32_t *ids, cons
  * [layers][B*T][d] int8, the wide layer's u [layers][B*T][hidden] and its k-th values kth [layers][B*T]
  * (device, nullable each). */
 int ava_train_decisions(const ava_trainer *t, int8_t *spikes, float *u, float *kth, ava_stream stream);
-/* Of the last step's products meant for the matrix cores, how many found no room for their operands' split form and
- * ran in the library (no counterpart in the reference; 0: the trainer's scratch holds them all). */
-int ava_train_unsplit(const ava_trainer *t);
+/* Of the last step's products, how many ran on the f16 matrix cores in split form, and how many meant for them found no
+ * room for their operands' split form and ran in the library (no counterpart in the reference; 0: the trainer's scratch
+ * holds them all). */
+int ava_train_products(const ava_trainer *t, int *split, int *unsplit);
 
 #ifdef __cplusplus
 }

@@ -2,6 +2,8 @@
 same forward (tests/train_ref.py, pinned against oracle/forward64.py in tests/test_train_ref.py),
 with the GPU step's own spikes and kWTA index sets forced in the statement. Bars: the loss within 1e-5
 relative, every parameter's gradient within 1e-4 of that tensor's largest reference magnitude."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -26,21 +28,21 @@ def test_train_step_matches_autograd(name, B, T):
     check_step(name, synth.config(name), B, T)
 
 
-# Batches whose head, wide-layer and square products go to the f16 matrix cores: rows that fill neither a
-# 128-row tile nor a 64-value K block (1029, 501), K cut into parts and not, a vocabulary that is no
+# Batches whose head, wide-layer, square and engram products go to the f16 matrix cores, at least so many of them: rows that
+# fill neither a 128-row tile nor a 64-value K block (501, 1229, 2871), K cut into parts and not, a vocabulary that is no
 # multiple of 4 (the 4-byte split passes, a ragged last tile), thin products on shared operands; vocabularies
 # below and above the wide layer (the largest operands are then W2's or the head's), an engram read as wide as the block.
-@pytest.mark.parametrize("name,B,T,over", [("ava04_d512", 1, 501, {}), ("ava04_d512", 1, 1029, {"vocab": 5003}),
-                                           ("ava04_d1024", 3, 704, {"vocab": 300}),
-                                           ("ava04_d512", 1, 1029, {"vocab": 300}),
-                                           ("ava04_d1024", 1, 2000, {"vocab": 300, "eng_dim": 1024, "eng_heads": 32})])
-def test_train_step_on_the_matrix_cores_matches_autograd(name, B, T, over):
+@pytest.mark.parametrize("name,B,T,over,cores", [
+    ("ava04_d512", 1, 501, {}, 1), ("ava04_d512", 1, 1229, {"vocab": 5003}, 3),
+    ("ava04_d1024", 3, 957, {"vocab": 300}, 28),
+    ("ava04_d1024", 2, 1440, {"vocab": 300, "eng_dim": 1024, "eng_heads": 32}, 40)])
+def test_train_step_on_the_matrix_cores_matches_autograd(name, B, T, over, cores):
     cfg = synth.config(name)
-    cfg.update({"layers": 1, "eng_block": 0, **over})
-    check_step(name, cfg, B, T)
+    cfg.update(layers=1, eng_block=0, **over)
+    check_step(name, cfg, B, T, cores)
 
 
-def check_step(name, cfg, B, T):
+def check_step(name, cfg, B, T, cores=0):
     from ava_amd.train import Trainer
     prm = synth.params(cfg, seed=81)
     rng = np.random.default_rng(82)
@@ -52,7 +54,10 @@ def check_step(name, cfg, B, T):
     flat = tr.pack(prm)
     loss, grads = tr.step(flat, torch.from_numpy(ids).cuda(), torch.from_numpy(tgt).cuda())
     torch.cuda.synchronize()
-    assert lib().ava_train_unsplit(tr.h) == 0  # no product fell back to the library for want of room
+    split, unsplit = C.c_int(), C.c_int()
+    assert lib().ava_train_products(tr.h, C.byref(split), C.byref(unsplit)) == 0
+    print(f"{split.value} products on the matrix cores", flush=True)
+    assert split.value >= cores and unsplit.value == 0  # none fell back to the library for want of room
     dec = tr.decisions(B, T)
     spikes = dec["spikes"].cpu().numpy()
     keep = (dec["u"] - dec["kth"][:, :, None] >= 0.0).to(torch.uint8).cpu().numpy()
