@@ -186,6 +186,10 @@ int split(ava_trainer *t, Op &x, bool tr, hipStream_t st) {
 // 8192 x 64 x 1024 18 us against 29, 1024 x 64 x 8192 24 against 58.
 constexpr double HGEMM_MACS = 3e9, HGEMM_LONG_MACS = 2e9, HGEMM_THIN = 1e8;
 constexpr int HGEMM_LONG = 4096;
+// A large operand of three thin products alone (the single-head engram's) is split for them from so many multiply-adds
+// each: a step of one d = 1024 block with / without, 3072 rows (2.0e8) 6.35 / 6.34 ms, 4096 (2.7e8) 6.32 / 6.38, 8192 9.32 / 9.41;
+// d = 512, 4096 rows (1.3e8) 4.30 / 4.23, 16,384 (5.4e8) 9.82 / 9.88.
+constexpr double HGEMM_THIN_SPLIT = 2.5e8;
 double hgemm_line(int K) { return K >= HGEMM_LONG ? HGEMM_LONG_MACS : HGEMM_MACS; }
 
 // row-major C [M][N] (ldc) = op(A) op(B) (+ C with add), op(A) [M][K] (A stored [M][K], or [K][M] when tA)
@@ -342,6 +346,7 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
     AVA_HIP(hipMemsetAsync(grads, 0, t->nparams * sizeof(float), st));
     t->hplanes_used = 0;
     t->split = t->unsplit = 0;
+    const bool eng_split = de <= 64 && (double)N * de * d >= HGEMM_THIN_SPLIT;
     // a named operand keeps its planes to the end of its Arena
     auto mm = [&](bool tA, bool tB, auto &&A, auto &&B, bool add, float *C, int ldc) {
         return gemm(t, tA, tB, A, B, std::is_lvalue_reference<decltype(A)>::value,
@@ -410,7 +415,7 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
             {
                 Arena eng(t);
                 Op h3{a.h3, N, d, d};
-                TR(split(t, h3, false, st));  // one split for three thin products
+                if (eng_split) TR(split(t, h3, false, st));  // one split for three thin products
                 TR(mm(false, false, h3, Op{w("ewq"), d, de, de}, false, a.eq, de));
                 TR(mm(false, false, h3, Op{w("ewk"), d, de, de}, false, a.ek, de));
                 TR(mm(false, false, h3, Op{w("ewv"), d, de, de}, false, a.ev, de));
@@ -476,7 +481,7 @@ int step(ava_trainer *t, const float *prm, const int32_t *ids, const int32_t *tg
             TR(ava::train::attn_bwd(at, st));
             Arena eng(t);
             Op h3{a.h3, N, d, d};
-            TR(split(t, h3, true, st));  // one split for three thin products
+            if (eng_split) TR(split(t, h3, true, st));  // one split for three thin products
             TR(mm(true, false, h3, Op{t->deq, N, de, de}, false, gw("ewq"), de));
             TR(mm(true, false, h3, Op{t->dek, N, de, de}, false, gw("ewk"), de));
             TR(mm(true, false, h3, Op{t->dev, N, de, de}, false, gw("ewv"), de));
