@@ -80,11 +80,12 @@ __device__ __forceinline__ void dspike(float v, float th, float slope, float &dv
 }
 
 // Whether a chain's thresholds stay below 3e8 (rho in [0, 1] keeps the trace within its start, the carried spike and
-// 2) and the slope below 1e6: then spikes count by ava::lif_count, and membranes below NEAR_V give NEAR surrogates.
+// 2) and the slope is in [0, 1e6): then spikes count by ava::lif_count, and membranes below NEAR_V give NEAR surrogates. (A
+// trainer's slope may be negative, and 1 + slope |x| then anything down to 0.)
 constexpr float NEAR_V = 1e9f;
 __device__ __forceinline__ bool tame(float th0, float rho, float gain, float a0, float s0, float slope) {
     return fabsf(th0) < 1e8f && rho >= 0.0f && rho <= 1.0f && fabsf(gain) < 1e4f && fabsf(a0) < 1e4f &&
-           fabsf(s0) < 1e4f && slope < 1e6f;
+           fabsf(s0) < 1e4f && slope >= 0.0f && slope < 1e6f;
 }
 
 struct LifBwdArgs {

@@ -157,6 +157,38 @@ def test_lif_bwd_segments_long():
         assert e < 1e-5, (k, e)
 
 
+@pytest.mark.parametrize("slope", [-0.5, -0.25, 0.0])
+def test_lif_bwd_segments_any_slope(slope):
+    """The training step's form takes any slope (ava_train_new does not bound it): with a negative one 1 + slope |x| may be 0,
+    whose surrogate is an infinity and not NaN. One 32-step segment: the oracle's bits."""
+    import ctypes as C
+    from ava_amd import _lib
+    B, T, D = 2, 32, 64
+    f = getattr(_lib.lib(), "_ZN3ava16lif_scan_bwd_segEPKfiiiS1_S1_S1_S1_iiifiS1_S1_S1_PfS2_S2_S2_S2_S2_S2_mS1_P12ihipStream_t")
+    cur, ps, v0, s0, a0, g, _, _ = lif_inputs(8, B, T, D, 1, False)
+    ps[:D], ps[D:2 * D] = 0.5, 1.0
+    v0[:], s0[:] = 0.0, 0.0
+    cur[:, :, :8] = 0.0
+    cur[:, T - 1, :4] = 3.0  # x = v - theta = 2: 1 + slope |x| = 0 at slope -0.5
+    cur[:, T - 1, 4:8] = 5.0  # 4: at slope -0.25
+    o = O.lif_bwd(cur, ps, g, v0, s0, a0, levels=1, signed=False, alif=False, slope=slope)
+    d = [dev(x) for x in (cur, ps, v0, s0, a0, g)]
+    out = [torch.empty((B, T, D), device="cuda")] + [torch.empty((B, D), device="cuda") for _ in range(5)]
+    nb = _lib.lib().ava_lif_scan_bwd_segments_workspace(B, T, D)
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    p = lambda t: C.c_void_p(t.data_ptr())
+    f.restype = C.c_int
+    f.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int] + [C.c_void_p] * 4 + [C.c_int] * 3 + [C.c_float, C.c_int] + \
+        [C.c_void_p] * 10 + [C.c_size_t, C.c_void_p, C.c_void_p]
+    rc = f(p(d[0]), B, T, D, p(d[1]), p(d[2]), p(d[3]), p(d[4]), 1, 0, 0, slope, 0, p(d[5]), None, None,
+           *(p(x) for x in out), p(ws), nb // 4, None, _lib.current_stream())
+    assert rc == 0
+    want = o["dI"]
+    if slope < 0:
+        assert np.isinf(want[:, T - 1]).any()
+    assert np.array_equal(host(out[0]), want, equal_nan=True)
+
+
 def test_kwta_relu2_bwd():
     from ava_amd import ops
     rng = np.random.default_rng(3)
