@@ -18,17 +18,21 @@
 //      every step; and, in other workgroups of the same launch, the reverse walk of (dF, dS) as if no
 //      element reached the bound, parking (dF, dS) at every chunk's end and dr_j of every step, and writing dv.
 //      The forward marks the workgroups in which an element did reach it.
-//   2. mem_bwd_bound_kernel: the reverse walk again from the parked end, with the bound's mask, for the heads with a
-//      marked workgroup (the others return at once).
+//   2. mem_bwd_bound_kernel: the reverse walk again from the parked end, with the bound's mask, in the marked
+//      workgroups' columns (the others return at once).
 //   3. mem_bwd_rows_kernel: per (head, chunk) the steps replayed from the parked states and walked back from
 //      the parked gradients. r_j and dr_j are known, so no column sum is left: lane = row, each wave 8
 //      columns, the row sums in the lane, the per-column values in scalar registers. The first chunk's workgroups end
 //      with dF0 and dS0. Every output but dv is written here, after the last read of the inputs it may lie on.
 // Measured, per-channel gates and momentum: 64 heads x 2048 steps 783 us (walks 478 us under the profiler, rows 445), 16 heads 343
 // us, 256 heads 2.64 ms, 1024 heads x 512 steps 2.59 ms; one kernel that parked every 4th state and walked three times
-// in series, the last walk forming the row sums too: 2.41, 1.87, 5.14 and 3.49 ms.
+// in series, the last walk forming the row sums too: 2.41, 1.87, 5.14 and 3.49 ms. With elements at the bound in every head
+// 64 heads x 2048 1.33 ms, 16 heads 0.84, 256 4.2, 512 x 1024 3.6, 1024 x 1024 7.2 (that kernel, bound or not: 2.40, 1.91, 5.1, 3.6,
+// 7.0); with the bound's walk waiting for each chunk's loads in turn, and every head's unmasked reverse walk before it, 2.41, 1.61,
+// 5.0, 4.9 and 9.8.
 // Workspace per (head, chunk): (F, S, dF, dS) of 16 KB (F and dF without momentum), and r, dr and room for dv per step.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -72,7 +76,7 @@ struct MemBwdArgs {
     float *ck;       // [BH][chunk][state][64 columns][64 rows]: F, dF (and S, dS with momentum)
     float *r, *dr;   // [BH][T][64]
     int *hit;        // [BH][groups]: an element of the forward workgroup's columns reached the bound
-    int groups, BH, T;
+    int groups, part, BH, T;  // part: which walks a launch holds (0 both, 1 the forward, 2 the reverse)
     float m, cap;
 };
 
@@ -80,6 +84,14 @@ struct MemBwdArgs {
 __device__ __forceinline__ bool head_hit(const MemBwdArgs &p, int bh) {
     int any = 0;
     for (int g = 0; g < p.groups; g++) any |= p.hit[bh * p.groups + g];
+    return any != 0;
+}
+
+// Whether one did in the 16 columns from 16 cg, by the forward workgroups that hold some of them. (Columns mix in
+// neither walk: the first one's results stand where none did.)
+__device__ __forceinline__ bool cols_hit(const MemBwdArgs &p, int bh, int cg) {
+    int any = 0;
+    for (int g = cg * p.groups / 4; 4 * g < (cg + 1) * p.groups; g++) any |= p.hit[bh * p.groups + g];
     return any != 0;
 }
 
@@ -239,13 +251,13 @@ __device__ __forceinline__ void park(float *dst, const float (&X)[R * CPL], int 
 // covers the staging of the next. A wave alone on its SIMD issues one VALU operation per 8 cycles, two waves share
 // them: so few heads are split into more, smaller workgroups, and the operations per element fall with more columns a lane (9, 8
 // and 7 forward). The columns' r (dr, dv) of step s stay in lane s, so a chunk's go out in
-// one store. Workgroups: the forward walks first, then the reverse.
+// one store. Workgroups: the forward walks first, then the reverse (see ava_mem_scan_bwd for many heads).
 template <bool G1, bool MOM, int R, int CPL>
 __global__ __launch_bounds__(256) void mem_bwd_walk_kernel(MemBwdArgs p) {
     constexpr int LPC = HS / R, WC = CPL * R, NG = HS / (4 * WC), NE = R * CPL;  // lanes a column, columns a wave
     __shared__ __attribute__((aligned(16))) Stage sg[2];
-    const bool rev = (int)blockIdx.x >= p.BH * NG;
-    const int wg = blockIdx.x - (rev ? p.BH * NG : 0), bh = wg / NG, cg = wg - bh * NG;
+    const bool rev = p.part ? p.part == 2 : (int)blockIdx.x >= p.BH * NG;
+    const int wg = blockIdx.x - (rev && !p.part ? p.BH * NG : 0), bh = wg / NG, cg = wg - bh * NG;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lc = lane & (LPC - 1);
     const int i0 = R * lc, j0 = 4 * WC * cg + WC * wave + CPL * (lane / LPC);
     const int T = p.T, nck = (T + CK - 1) / CK;
@@ -316,6 +328,11 @@ __global__ __launch_bounds__(256) void mem_bwd_walk_kernel(MemBwdArgs p) {
         dF[m] = p.dFT ? p.dFT[o] : 0.0f;
         dS[m] = (MOM && p.dST) ? p.dST[o] : 0.0f;
     }
+    if (p.part && p.hit[bh * NG + cg]) {  // these columns are walked with the bound's mask
+        park<R, CPL>(parked<MOM>(p, bh, nck - 1, 1), dF, i0, j0);
+        if (MOM) park<R, CPL>(parked<MOM>(p, bh, nck - 1, 3), dS, i0, j0);
+        return;
+    }
     Loader<G1, false> in;
     in.load(p, bh, (nck - 1) * CK, tid);
     in.stage(sg[(nck - 1) & 1], tid);
@@ -367,75 +384,120 @@ __global__ __launch_bounds__(256) void mem_bwd_walk_kernel(MemBwdArgs p) {
     }
 }
 
-// 2. The reverse walk with the bound's mask, for the heads in which an element reached it: every
-// chunk's states are replayed from its parked ones (r is known) and kept, then the chunk is walked back.
+// 2. The reverse walk with the bound's mask, in the marked columns: every chunk's states are replayed from its parked
+// ones (r is known) and kept, then the chunk is walked back. As in the walks above, a chunk's inputs are loaded two chunks
+// ahead into registers and staged one ahead (double-buffered, one barrier a chunk), and the parked states come one ahead.
 template <bool G1, bool MOM>
 __global__ __launch_bounds__(256) void mem_bwd_bound_kernel(MemBwdArgs p) {
     const int bh = blockIdx.x >> 2, cg = blockIdx.x & 3;
-    if (!head_hit(p, bh)) return;
-    __shared__ __attribute__((aligned(16))) Stage sg;
-    __shared__ float sv[CK][HS];
+    if (!cols_hit(p, bh, cg)) return;
+    __shared__ __attribute__((aligned(16))) Stage sg[2];
+    __shared__ float sv[2][CK][16], sr[2][CK][16];  // v and r of the workgroup's 16 columns
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15;
-    const int i0 = 4 * l16, j = 16 * cg + 4 * wave + (lane >> 4);
+    const int i0 = 4 * l16, jl = 4 * wave + (lane >> 4), j = 16 * cg + jl;
     const int T = p.T, nck = (T + CK - 1) / CK;
     const size_t hb = (size_t)bh * T * HS;
     const float M = p.m, cap = p.cap;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto state = [&](int c, int which) {
+        return *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, c, which) + j * HS + i0);
+    };
     // the gradients after the last step, as the first walk parked them
     float dF[4], dS[4];
     {
-        const f32x4 f = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, nck - 1, 1) + j * HS + i0);
-        f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (MOM) s = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, nck - 1, 3) + j * HS + i0);
+        const f32x4 f = state(nck - 1, 1), s = MOM ? state(nck - 1, 3) : zero;
 #pragma unroll
         for (int m = 0; m < 4; m++) {
             dF[m] = f[m];
             dS[m] = s[m];
         }
     }
-    for (int c = nck - 1; c >= 0; c--) {
-        const int n = min(CK, T - c * CK);
-        __syncthreads();
-        Loader<G1, false> in;
+    Loader<G1, false> in;
+    float lv, lr;  // v and r of step tid / 16, column tid % 16
+    auto load = [&](int c) {
         in.load(p, bh, c * CK, tid);
-        in.stage(sg, tid);
-        for (int z = tid; z < n * HS; z += 256) sv[z / HS][z % HS] = p.v[hb + (size_t)c * CK * HS + z];
-        __syncthreads();
-        park<4, 1>(parked<MOM>(p, bh, c, 1), dF, i0, j);
-        if (MOM) park<4, 1>(parked<MOM>(p, bh, c, 3), dS, i0, j);
+        const int t = c * CK + (tid >> 4);
+        lv = lr = 0.0f;
+        if (c < 0 || t >= T) return;
+        const size_t o = hb + (size_t)t * HS + 16 * cg + (tid & 15);
+        lv = p.v[o];
+        lr = p.r[o];
+    };
+    auto stage = [&](int b) {
+        in.stage(sg[b], tid);
+        sv[b][tid >> 4][tid & 15] = lv;
+        sr[b][tid >> 4][tid & 15] = lr;
+    };
+    load(nck - 1);
+    stage((nck - 1) & 1);
+    load(nck - 2);
+    f32x4 f0 = state(nck - 1, 0), s0 = MOM ? state(nck - 1, 2) : zero;
+    for (int c = nck - 1; c >= 0; c--) {
+        __syncthreads();  // chunk c is staged; everyone is done with the other buffer
+        if (c > 0) stage((c - 1) & 1);
+        load(c - 2);
         float Ft[CK + 1][4], S[4];
-        const f32x4 f0 = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, c, 0) + j * HS + i0);
-        f32x4 s0 = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (MOM) s0 = *reinterpret_cast<const f32x4 *>(parked<MOM>(p, bh, c, 2) + j * HS + i0);
 #pragma unroll
         for (int m = 0; m < 4; m++) {
             Ft[0][m] = f0[m];
             S[m] = s0[m];
         }
+        if (c > 0) {
+            f0 = state(c - 1, 0);
+            if (MOM) s0 = state(c - 1, 2);
+        }
+        park<4, 1>(parked<MOM>(p, bh, c, 1), dF, i0, j);
+        if (MOM) park<4, 1>(parked<MOM>(p, bh, c, 3), dS, i0, j);
+        const int n = min(CK, T - c * CK), b = c & 1;
+        const Stage &st = sg[b];
+        float keptr = 0.0f, keptv = 0.0f;
+        auto chunk = [&](auto full) {
+            constexpr bool FULL = decltype(full)::value;
+            // a step's operands are read during the step before it, and not earlier (registers: see sched_barrier)
+            struct {
+                f32x4 x, k, a;
+                float r, v;
+            } in[2];
+            auto read = [&](int s) {
+                auto at = [&](const float (&d)[CK][HS]) { return *reinterpret_cast<const f32x4 *>(&d[s][i0]); };
+                in[s & 1] = {at(st.abe), at(st.bk), at(st.a), sr[b][s][jl], sv[b][s][jl]};
+            };
+            read(0);
 #pragma unroll
-        for (int s = 0; s < CK; s++)
-            if (s < n) {
-                const float r = p.r[hb + (size_t)(c * CK + s) * HS + j], vj = sv[s][j];
+            for (int s = 0; s < CK; s++)
+                if (FULL || s < n) {
+                    if (s + 1 < CK) read(s + 1);
+                    const auto &z = in[s & 1];
 #pragma unroll
-                for (int m = 0; m < 4; m++) {
-                    const float u = fmaf(-sg.abe[s][i0 + m], r, sg.bk[s][i0 + m] * vj);
-                    if (MOM) S[m] = fmaf(M, S[m], u);
-                    const float f = fmaf(sg.a[s][i0 + m], Ft[s][m], MOM ? S[m] : u);
-                    Ft[s + 1][m] = __builtin_amdgcn_fmed3f(f, -cap, cap);
+                    for (int m = 0; m < 4; m++) {
+                        const float u = fmaf(-z.x[m], z.r, z.k[m] * z.v);
+                        if (MOM) S[m] = fmaf(M, S[m], u);
+                        const float f = fmaf(z.a[m], Ft[s][m], MOM ? S[m] : u);
+                        Ft[s + 1][m] = __builtin_amdgcn_fmed3f(f, -cap, cap);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            }
+            StepIn<4, 1, false> x[2];
+            x[1].read(st, n - 1, i0, j);
+            if (!FULL) x[0] = x[1];
 #pragma unroll
-        for (int s = CK - 1; s >= 0; s--)
-            if (s < n) {
-                StepIn<4, 1, false> x;
-                x.read(sg, s, i0, j);
-                float dr[1], dv[1];
-                rev_step<MOM, 4, 1>(dF, dS, x, M, Ft[s + 1], cap, dr, dv);
-                if (l16 == 0) {
-                    const size_t o = hb + (size_t)(c * CK + s) * HS + j;
-                    p.dr[o] = dr[0];
-                    p.dv[o] = dv[0];
+            for (int s = CK - 1; s >= 0; s--)
+                if (FULL || s < n) {
+                    if (s > 0) x[(s - 1) & 1].read(st, s - 1, i0, j);
+                    float dr[1], dv[1];
+                    rev_step<MOM, 4, 1>(dF, dS, x[s & 1], M, Ft[s + 1], cap, dr, dv);
+                    keptr = l16 == s ? dr[0] : keptr;
+                    keptv = l16 == s ? dv[0] : keptv;
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            }
+        };
+        if (n == CK) chunk(std::integral_constant<bool, true>{});
+        else chunk(std::integral_constant<bool, false>{});
+        if (l16 < n) {
+            const size_t o = hb + (size_t)(c * CK + l16) * HS + j;
+            p.dr[o] = keptr;
+            p.dv[o] = keptv;
+        }
     }
 }
 
@@ -714,7 +776,7 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
     const Layout lo = layout(BH, T, mom);
     float *w = (float *)work;
     MemBwdArgs p{q, k, e, v, la, b, F0, mom ? S0 : nullptr, dy, dF_T, mom ? dS_T : nullptr, dq, dk, de, dv, dla, db,
-                 dF0, mom ? dS0 : nullptr, w, w + lo.ck, w + lo.ck + lo.r, (int *)(w + lo.ck + 3 * lo.r), 0, BH, T, m, cap};
+                 dF0, mom ? dS0 : nullptr, w, w + lo.ck, w + lo.ck + lo.r, (int *)(w + lo.ck + 3 * lo.r), 0, 0, BH, T, m, cap};
     const hipStream_t st = (hipStream_t)stream;
     int cus = 0;
     if (int r = ava::device_cus(&cus)) return r;
@@ -727,7 +789,16 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
     const int rows = BH * ava::ceil_div(T, CK);
     auto walk = [&](auto kern, int groups) {
         p.groups = groups;
-        kern<<<BH * groups * 2, 256, 0, st>>>(p);
+        // From two heads a CU the forward walks alone fill the chip: they go first, and the reverse walks of columns that
+        // reached the bound are left to the bound kernel.
+        if (BH >= 2 * cus) {
+            p.part = 1;
+            kern<<<BH * groups, 256, 0, st>>>(p);
+            p.part = 2;
+            kern<<<BH * groups, 256, 0, st>>>(p);
+        } else {
+            kern<<<BH * groups * 2, 256, 0, st>>>(p);
+        }
     };
     auto run = [&](auto w8, auto w4, auto w2, auto w1, auto bound, auto rows_k) {
         // A head's columns over 4 or 2 workgroups a direction while the CUs hold them all at once (three each, by LDS), over 8
