@@ -103,8 +103,8 @@ __device__ __forceinline__ bool wave_tame(const LifBwdArgs &p, int c, int i) {
                       ALIF ? p.a0[i] : 0.0f, p.s0[i], p.slope));
 }
 
-// FIN: the wave's chains are tame.
-template <int K, int LEVELS, bool SIGNED, bool ALIF, bool FIN>
+// FIN: the wave's chains are tame. KEEP: the spikes are kept for the way back, not formed again (see ava_lif_scan_bwd).
+template <int K, int LEVELS, bool SIGNED, bool ALIF, bool FIN, bool KEEP>
 __device__ __forceinline__ void lif_bwd_chain(const LifBwdArgs &p, int gid) {
     const int D = p.D, T = p.T;
     const int b = gid / D, c = gid - b * D;
@@ -188,7 +188,11 @@ __device__ __forceinline__ void lif_bwd_chain(const LifBwdArgs &p, int gid) {
             load_ck(q + 1, nkv, nks, nka);
         }
         const int t0 = seg0(q), n = T - q * K - t0;
-        float vs[K] = {}, as[K] = {}, ss[K] = {}, top = 0.0f;
+        float vs[K] = {}, as[K] = {}, ss[KEEP ? K : 1] = {}, top = 0.0f;
+        auto spk = [&](int i) {
+            if constexpr (KEEP) return ss[i];
+            else return spike<LEVELS, SIGNED, FIN>(vs[i], ALIF ? th0 + as[i] * gain : th0);
+        };
         {
             float v = ckv, sp = cks, a = cka, thp = ALIF ? th0 + cka * gain : th0;
 #pragma unroll
@@ -204,7 +208,7 @@ __device__ __forceinline__ void lif_bwd_chain(const LifBwdArgs &p, int gid) {
                     thp = tht;
                     vs[i] = v;
                     as[i] = a;
-                    ss[i] = sp;
+                    if constexpr (KEEP) ss[i] = sp;
                     if (FIN) top = fmaxf(top, fabsf(v));
                 }
             }
@@ -227,11 +231,11 @@ __device__ __forceinline__ void lif_bwd_chain(const LifBwdArgs &p, int gid) {
                     gb += G * (i > 0 ? vs[i - 1] : ckv);
                     if (ALIF) {
                         float gth = gst * dth;
-                        if (p.rg) gth -= ss[i] * Gn;
+                        if (p.rg) gth -= spk(i) * Gn;
                         const float gaa = gth * gain + ca;
                         gg += gth * at;
                         const float ap = i > 0 ? as[i - 1] : cka;
-                        const float sprev = i > 0 ? ss[i - 1] : cks;
+                        const float sprev = i > 0 ? spk(i - 1) : cks;
                         gr += gaa * (ap - fabsf(sprev));
                         ca = rho * gaa;
                     }
@@ -264,14 +268,14 @@ __device__ __forceinline__ void lif_bwd_chain(const LifBwdArgs &p, int gid) {
     if (p.dgain) p.dgain[gid] = ALIF ? gg : 0.0f;
 }
 
-template <int K, int LEVELS, bool SIGNED, bool ALIF>
+template <int K, int LEVELS, bool SIGNED, bool ALIF, bool KEEP>
 __global__ __launch_bounds__(256, 2) void lif_bwd_kernel(LifBwdArgs p) {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     const bool in = gid < p.B * p.D;
     const bool fin = wave_tame<ALIF>(p, in ? gid % p.D : 0, in ? gid : 0);
     if (!in) return;
-    if (fin) lif_bwd_chain<K, LEVELS, SIGNED, ALIF, true>(p, gid);
-    else lif_bwd_chain<K, LEVELS, SIGNED, ALIF, false>(p, gid);
+    if (fin) lif_bwd_chain<K, LEVELS, SIGNED, ALIF, true, KEEP>(p, gid);
+    else lif_bwd_chain<K, LEVELS, SIGNED, ALIF, false, KEEP>(p, gid);
 }
 
 // Steps per segment: 5 x 16 registers of currents, gradients and replayed state. 32-step segments
@@ -604,16 +608,24 @@ extern "C" int ava_lif_scan_bwd(const float *cur, int B, int T, int D, const flo
                  B, T, D, slope, reset_grad ? 1 : 0};
     const hipStream_t st = (hipStream_t)stream;
     dim3 grid(ava::ceil_div((long)B * D, 256)), block(256);
-#define AVA_LB(L, S, A) lif_bwd_kernel<SEG, L, S, A><<<grid, block, 0, st>>>(p)
+    // One level's spikes cost little to form again, and keeping them takes 140 registers where 123 let a fourth wave share
+    // a SIMD: kept while three waves a SIMD hold all chains (unsigned, us kept / not: 32 x 1024 x 2048 308 / 325, 64 x 512 x 2048
+    // 216 / 219, 256 x 128 x 1024 114 / 101, 256 x 256 x 1024 225 / 211). Two levels' are always kept.
+    int cus = 0;
+    if (int r = ava::device_cus(&cus)) return r;
+    const bool keep = (long)B * D <= 3L * 256 * cus;
+#define AVA_LB(L, S, A, K) lif_bwd_kernel<SEG, L, S, A, K><<<grid, block, 0, st>>>(p)
     if (!is_signed) {
-        if (alif) AVA_LB(1, false, true);
-        else AVA_LB(1, false, false);
+        if (!alif) AVA_LB(1, false, false, false);
+        else if (keep) AVA_LB(1, false, true, true);
+        else AVA_LB(1, false, true, false);
     } else if (levels == 1) {
-        if (alif) AVA_LB(1, true, true);
-        else AVA_LB(1, true, false);
+        if (!alif) AVA_LB(1, true, false, false);
+        else if (keep) AVA_LB(1, true, true, true);
+        else AVA_LB(1, true, true, false);
     } else {
-        if (alif) AVA_LB(2, true, true);
-        else AVA_LB(2, true, false);
+        if (alif) AVA_LB(2, true, true, true);
+        else AVA_LB(2, true, false, true);
     }
 #undef AVA_LB
     AVA_LAUNCHED("lif_scan_bwd");

@@ -98,6 +98,20 @@ def test_lif_bwd_large_values(rg):
             assert np.all(d <= 1e-4 * top + 1e-30), (slope, k, float(np.max(d / (top + 1e-30))))
 
 
+@pytest.mark.parametrize("levels,signed", [(1, True), (1, False), (2, True)])
+def test_lif_bwd_many_chains(levels, signed):
+    """More chains than three waves a SIMD hold (256 x 1024 on 256 CUs): one level's spikes are formed again on the way
+    back instead of kept. The oracle's bits, with the reset gradient (which reads them)."""
+    B, T, D = 256, 19, 1024
+    x = lif_inputs(61 + levels, B, T, D, levels, signed)
+    print(f"lif_bwd many chains levels={levels} signed={signed}", flush=True)
+    o = O.lif_bwd(x[0], x[1], x[5], x[2], x[3], x[4], x[6], x[7], levels=levels, signed=signed, alif=True, slope=2.0,
+                  reset_grad=True)
+    gpu = run_lif(*x, levels, signed, True, 2.0, True)
+    for k in ("dI", "dv0", "da0", "dbeta", "drho", "dgain"):
+        assert np.array_equal(gpu[k], o[k]), (k, rel(gpu[k], o[k]))
+
+
 def test_lif_bwd_long():
     """config[1]'s sequence length and width (T 2048, D 2048) on 8 streams, int2 with ALIF and the
     reset gradient."""
