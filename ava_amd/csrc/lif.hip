@@ -173,7 +173,9 @@ __device__ __forceinline__ bool finite_thresholds(float th0, float rho, float ga
 // stay finite count spikes by lif_count: 20 operations a step instead of 27, 64 x 2048 x 1024 158 us instead of 202,
 // 4 x 2048 x 1024 146 instead of 176. Past 114,688 chains and 2e8 elements HBM bounds the scan, and the counted form,
 // whose waves drift further apart, streams worse (into alternating outputs, T = 2048: 48 x 2048 channels 214 us counted,
-// 240 by differences; 56 253 / 256; 60 269 / 266; 64 295 / 281, 4.8 TB/s): COUNT is off there.
+// 240 by differences; 56 253 / 256; 60 269 / 266; 64 295 / 281, 4.8 TB/s): COUNT is off there. One level saves fewer operations,
+// and HBM bounds it past one wave per SIMD (signed, T = 512: 32 x 2048 channels 49 us counted, 54 by differences; 48 70.7 / 69.9; 64
+// 83.6 / 77.6): COUNT is off from there.
 template <int PF, int LEVELS, bool SIGNED, bool ALIF, bool COUNT>
 __global__ __launch_bounds__(256) void lif_scan_buf_kernel(const float *__restrict__ cur, int B, int T, int D,
                                                            const float *__restrict__ ps, float *__restrict__ v,
@@ -269,7 +271,8 @@ int launch_vp(const float *cur, int B, int T, int D, const float *ps, float *v, 
     dim3 grid(ava::ceil_div(threads, 256)), block(256);
     // the buffer form: whole waves per stream, and every offset of a stream's slab in 32 bits
     const bool bufd = VEC == 1 && PF == ava::LIF_SEG_STEPS && D % 64 == 0 && (long)T * D * 4 < (1L << 31);
-    const bool count = (long)B * D <= 114688 || (long)B * T * D <= 200000000L;  // see lif_scan_buf_kernel
+    const bool count = is_signed && levels == 2 ? (long)B * D <= 114688 || (long)B * T * D <= 200000000L
+                                                 : (long)B * D <= 65536;  // see lif_scan_buf_kernel
 #define AVA_LIF_GO(L, S, A)                                                                                         \
     do {                                                                                                            \
         if (bufd && count)                                                                                          \

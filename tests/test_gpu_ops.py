@@ -95,6 +95,25 @@ def test_lif_config1_shape_bit_exact(B, T, D, dev):
     assert np.mean(np.abs(spk_o) == 2) > 0  # both levels occur
 
 
+@pytest.mark.parametrize("signed", [True, False])
+@pytest.mark.parametrize("B", [64, 65])
+def test_lif_one_level_many_chains_bit_exact(B, signed, dev):
+    """One level at and past 65,536 chains (64 x 1024): the counted form, then the differences."""
+    T, D = 40, 1024
+    rng = np.random.default_rng(12)
+    cur = (rng.standard_normal((B, T, D)) * 1.3).astype(np.float32)
+    beta = sig(rng.uniform(0.5, 3.0, D).astype(np.float32))
+    ps = np.concatenate([beta, np.full(D, 0.9, np.float32), np.full(D, 0.95, np.float32),
+                         np.full(D, 0.05, np.float32)]).astype(np.float32)
+    spk_o, v_o, _, a_o = O.lif_scan(cur, ps, levels=1, signed=signed, alif=True)
+    from ava_amd import ops
+    spk, st = ops.lif_gen(cuda(cur), cuda(beta), cuda(ps[D:2 * D]), (cuda(ps[2 * D:3 * D]), cuda(ps[3 * D:])),
+                          levels=1, signed=signed)
+    assert np.array_equal(host(spk), spk_o)
+    assert np.array_equal(host(st.v).view(np.uint32), v_o.view(np.uint32))
+    assert np.array_equal(host(st.a).view(np.uint32), a_o.view(np.uint32))
+
+
 def test_lif_thresholds_outside_the_counted_form(dev):
     """Waves (64 channels) whose thresholds may leave the finite range take the difference form: infinite and
     huge thetas, a trace that grows (rho > 1), a carried spike of infinity, against currents that reach infinity; the
