@@ -790,8 +790,8 @@ extern "C" int ava_mem_scan_bwd(const float *q, const float *k, const float *e, 
     auto walk = [&](auto kern, int groups) {
         p.groups = groups;
         // From two heads a CU the forward walks alone fill the chip: they go first, and the reverse walks of columns that
-        // reached the bound are left to the bound kernel.
-        if (BH >= 2 * cus) {
+        // reached the bound are left to the bound kernel. (Up to two chunks the launch more costs what they take.)
+        if (BH >= 2 * cus && T > 2 * CK) {
             p.part = 1;
             kern<<<BH * groups, 256, 0, st>>>(p);
             p.part = 2;

@@ -331,12 +331,12 @@ def clear_heads(x, m, cap):
 
 
 @pytest.mark.parametrize("BH,T", [(16, 33), (32, 16), (33, 33), (65, 17), (96, 18), (97, 17), (129, 47), (193, 16),
-                                  (512, 17), (530, 33)])
+                                  (512, 32), (530, 33)])
 @pytest.mark.parametrize("g,m", [(64, 0.5), (1, 0.0)])
 @pytest.mark.parametrize("cap", [1e5, 0.6])
 def test_mem_bwd_walk_shapes(BH, T, g, m, cap):
     """Each split of a head's columns over workgroups (on 256 CUs up to 16, 96, 192 heads, more; from
-    512 the two walks one after the other), chunks of 16 steps whole and
+    512 and past 32 steps the two walks one after the other), chunks of 16 steps whole and
     short, with the bound never and often reached (the reverse walk's second form and the masked rows)."""
     x = mem_inputs(BH + T + g, BH, T, g)
     print(f"mem_bwd BH={BH} T={T} g={g} m={m} cap={cap}", flush=True)

@@ -61,8 +61,8 @@ def test_mem_scan_matches_recurrence(g, m, T, BH):
 
 # each split of a head's columns over workgroups (up to 64, 128, 384, 512 heads, more), head counts that are and are
 # not multiples of the XCDs, whole chunks of 16 steps with a short one behind them
-@pytest.mark.parametrize("BH", [64, 65, 129, 136, 385, 392, 513])
-@pytest.mark.parametrize("g,m,T", [(64, 0.5, 33), (1, 0.0, 16)])
+@pytest.mark.parametrize("BH", [64, 65, 129, 136, 385, 392, 512, 513])
+@pytest.mark.parametrize("g,m,T", [(64, 0.5, 33), (1, 0.0, 16), (64, 0.5, 65)])
 def test_mem_scan_splits_match_recurrence(BH, g, m, T):
     print(f"mem_scan BH={BH} g={g} m={m} T={T}", flush=True)
     q, k, e, v, la, b = inputs(BH, T, g, BH + T)
