@@ -475,7 +475,7 @@ __device__ __forceinline__ void mq_bf_half(f32x16 &acc, const __bf16 *A, int ar0
 // update K^T D; D = T' R splits its k range between the two sets (the state waves' half added through
 // the LDS that held V). Each phase thus has two waves per SIMD to overlap.
 // Bound by its phases' latencies (5 barriers a chunk; one workgroup's LDS fills a CU), so what shortens a phase counts:
-// 256 heads x 4096, both launches, 671 -> 613 us when the terms came to be split in pairs (split2: 12% fewer VALU
+// 256 heads x 4096, both launches, 645 -> 609 us (another box 678 -> 615) when the terms came to be split in pairs (split2: 12% fewer VALU
 // operations, no spilled registers) and K's columns written as pairs into swizzled rows (12 instead of
 // 24 LDS writes a thread and chunk, without bank conflicts).
 __global__ __launch_bounds__(512) void delta_seq_bf_kernel(DeltaArgs p, const float *__restrict__ Tp) {

@@ -24,7 +24,7 @@
 //      the parked gradients. r_j and dr_j are known, so no column sum is left: lane = row, each wave 8
 //      columns, the row sums in the lane, the per-column values in scalar registers. The first chunk's workgroups end
 //      with dF0 and dS0. Every output but dv is written here, after the last read of the inputs it may lie on.
-// Measured, per-channel gates and momentum: 64 heads x 2048 steps 783 us (walks 478 us under the profiler, rows 445), 16 heads 343
+// Measured, per-channel gates and momentum: 64 heads x 2048 steps 783 us (under the profiler walks 426, rows 438), 16 heads 343
 // us, 256 heads 2.64 ms, 1024 heads x 512 steps 2.59 ms; one kernel that parked every 4th state and walked three times
 // in series, the last walk forming the row sums too: 2.41, 1.87, 5.14 and 3.49 ms. With elements at the bound in every head
 // 64 heads x 2048 1.33 ms, 16 heads 0.84, 256 4.2, 512 x 1024 3.6, 1024 x 1024 7.2 (that kernel, bound or not: 2.40, 1.91, 5.1, 3.6,

@@ -70,7 +70,7 @@ __global__ void q8_pack_kernel(const float *__restrict__ w, int din, int dout, i
 
 // W waves per row (1 or 4): the row's absmax, its exponent, then its planes (padding zeroed). A lane holds NV groups of 4
 // values of the row (ldq <= 256 W NV; 16-byte loads when V4), so the row is read once, and the loads are all in
-// flight; longer rows (NV = 0) are read again. Bound by HBM: 131,072 x 1024 in 3 planes (0.92 GB) 185 us; reading the row
+// flight; longer rows (NV = 0) are read again. Bound by HBM: 131,072 x 1024 in 3 planes (0.92 GB) 152 us; reading the row
 // twice in 4-byte loads took 335.
 template <int P, int W, int NV, bool V4>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const float *__restrict__ x, int m, int k, int ldx,
